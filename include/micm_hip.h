@@ -309,9 +309,11 @@ int micm_hip_state_set_handoff(micm_hip_state* state, int64_t steps);
  * substitution tables, bit 1 the LU tables; -1: the library's choice; tables that
  * do not fit next to the cell's data stay in global memory), or 4: the compact
  * per-cell layout (no tables staged, fewer arrays in LDS so that more cells fit a CU;
- * needs more than 64 threads and at least one thread per species, else ignored), its
- * register budget chosen from occupancy; 5 / 6 / 7: the compact layout with 256 threads built
- * for three waves per SIMD (168 registers) / two (256) / no register bound.  A tuning
+ * needs more than 64 threads and at least one thread per species, else ignored).  With 256
+ * threads and 16 to 256 species the compact layout is the kernel that takes the factor's last
+ * rows as a dense block, which the library's choice of staging (-1) also picks; 5 / 6 / 7: that
+ * kernel built for three waves per SIMD (168 registers) / two (256) / two, 4 leaving the choice
+ * to the occupancy.  A tuning
  * knob in the role of the vector length L of the reference's GPU policies
  * (cuda_solver_builder.hpp:24-38); results do not depend on it. */
 int micm_hip_state_set_cooperative_shape(micm_hip_state* state, int32_t threads, int32_t stage);

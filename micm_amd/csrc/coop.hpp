@@ -182,10 +182,9 @@ namespace micm_hip
     return v;
   }
 
-  // out[s] = f(yv)[s]
+  // The reactions' rates at yv into L.scratch
   template<int NT>
-  __device__ inline void coop_forcing(const DevMech& m, const DevCoop& c, const CoopLds& L, const double* yv,
-                                      double* out)
+  __device__ inline void coop_rates(const DevMech& m, const DevCoop& c, const CoopLds& L, const double* yv)
   {
     const int tid = threadIdx.x;
     const int R = m.n_reactions;
@@ -227,10 +226,31 @@ namespace micm_hip
         }
       }
     }
+  }
+
+  // out[s] = f(yv)[s]
+  template<int NT>
+  __device__ inline void coop_forcing(const DevMech& m, const DevCoop& c, const CoopLds& L, const double* yv,
+                                      double* out)
+  {
+    coop_rates<NT>(m, c, L, yv);
     coop_sync<NT>();
-    for (int s = tid; s < m.n_species; s += NT)
+    for (int s = threadIdx.x; s < m.n_species; s += NT)
       out[s] = gather_sum(0.0, c.spec_rxn, c.spec_coef, c.spec_offsets[s], c.spec_offsets[s + 1], L.scratch);
     coop_sync<NT>();
+  }
+
+  // f(yv) of this thread's species (0 beyond the last); L.scratch is read until the next
+  // barrier
+  template<int NT>
+  __device__ inline double coop_forcing_own(const DevMech& m, const DevCoop& c, const CoopLds& L, const double* yv)
+  {
+    const int s = threadIdx.x;
+    coop_rates<NT>(m, c, L, yv);
+    coop_sync<NT>();
+    return s < m.n_species
+               ? gather_sum(0.0, c.spec_rxn, c.spec_coef, c.spec_offsets[s], c.spec_offsets[s + 1], L.scratch)
+               : 0.0;
   }
 
   // L.jac = -J(y); with TO_ALU the elements go straight to their factor positions

@@ -87,6 +87,27 @@ namespace micm_hip
     int32_t n_tasks;
   };
 
+  // Rows of a substitution, sixteen tasks a level (RowLevels).
+  struct DevRows
+  {
+    const uint32_t* heads;
+    const uint4* terms;  // sixteen per task: lane k's terms k, 16 + k, 32 + k, 48 + k
+    const int32_t* groups;
+    int32_t n_levels;
+  };
+
+  // The factor's last rows and columns as a dense block (TailTables).
+  struct DevTail
+  {
+    int32_t size;  // 0: none
+    int32_t first, head, nnz;
+    const int32_t* jac_pos;
+    const int32_t* diag_pos;
+    const uint64_t* row_mask;
+    DevLevels lu;
+    DevRows fwd, bwd;
+  };
+
   // Tables of the cooperative (one workgroup per cell) form; see MechanismTables.
   struct DevCoop
   {

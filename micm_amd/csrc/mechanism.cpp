@@ -755,6 +755,314 @@ namespace micm_hip
       t.jel_pack.insert(t.jel_pack.end(), 8, 0);
     }
 
+    // A row of a substitution: its output, divisor and terms in order.
+    struct SubstitutionRow
+    {
+      uint32_t out = 0, diag = kNoDivisor;
+      std::vector<uint32_t> terms;  // ALU position | x position << 16
+    };
+
+    // Rows (each after the rows it reads) as levels of kRowSlots tasks: a list schedule that
+    // fills each level with the ready tasks on the longest remaining paths.  `zero`: ALU
+    // position of the zero, `zero_x`: x position of a zero.
+    RowLevels row_levels(const std::vector<SubstitutionRow>& rows, int32_t n, uint32_t zero, uint32_t zero_x)
+    {
+      // tasks: a row, or the parts of at most kRowTerms terms of a longer one
+      struct Task
+      {
+        uint32_t row, first, count;
+        bool last;
+      };
+      std::vector<Task> tasks;
+      std::vector<int32_t> final_task(n, -1);  // the task that finishes an x position
+      for (size_t r = 0; r < rows.size(); ++r)
+      {
+        const uint32_t count = static_cast<uint32_t>(rows[r].terms.size());
+        uint32_t q = 0;
+        do
+        {
+          const uint32_t c = std::min<uint32_t>(count - q, kRowTerms);
+          tasks.push_back(Task{ static_cast<uint32_t>(r), q, c, q + c == count });
+          q += c;
+        } while (q < count);
+        final_task[rows[r].out] = static_cast<int32_t>(tasks.size()) - 1;
+      }
+      const size_t nt = tasks.size();
+      std::vector<std::vector<uint32_t>> succ(nt);
+      std::vector<uint32_t> deps(nt, 0);
+      for (size_t t = 0; t < nt; ++t)
+      {
+        std::vector<uint32_t> before;
+        if (t > 0 && tasks[t - 1].row == tasks[t].row)
+          before.push_back(static_cast<uint32_t>(t) - 1);
+        for (uint32_t q = 0; q < tasks[t].count; ++q)
+        {
+          const int32_t f = final_task[rows[tasks[t].row].terms[tasks[t].first + q] >> 16];
+          if (f >= 0)
+            before.push_back(static_cast<uint32_t>(f));
+        }
+        std::sort(before.begin(), before.end());
+        before.erase(std::unique(before.begin(), before.end()), before.end());
+        for (uint32_t b : before)
+          succ[b].push_back(static_cast<uint32_t>(t));
+        deps[t] = static_cast<uint32_t>(before.size());
+      }
+      // longest path to the end, in tasks (the dependency graph is acyclic: a row reads only
+      // rows that were final before it in the substitution's own order)
+      std::vector<uint32_t> order;
+      std::vector<uint32_t> left(deps);
+      for (size_t t = 0; t < nt; ++t)
+        if (left[t] == 0)
+          order.push_back(static_cast<uint32_t>(t));
+      for (size_t q = 0; q < order.size(); ++q)
+        for (uint32_t s : succ[order[q]])
+          if (--left[s] == 0)
+            order.push_back(s);
+      std::vector<int32_t> height(nt, 0);
+      for (size_t q = order.size(); q-- > 0;)
+        for (uint32_t s : succ[order[q]])
+          height[order[q]] = std::max(height[order[q]], height[s] + 1);
+      RowLevels out;
+      std::vector<uint32_t> ready, next;
+      left = deps;
+      for (size_t t = 0; t < nt; ++t)
+        if (left[t] == 0)
+          ready.push_back(static_cast<uint32_t>(t));
+      while (!ready.empty())
+      {
+        // the longest remaining paths first; among equals the longest sums, so that the
+        // sums of one level are of like length
+        std::stable_sort(ready.begin(), ready.end(), [&](uint32_t a, uint32_t b) {
+          if (height[a] != height[b])
+            return height[a] > height[b];
+          return tasks[a].count > tasks[b].count;
+        });
+        const size_t take = std::min<size_t>(ready.size(), kRowSlots);
+        int32_t groups = 0;
+        next.assign(ready.begin() + static_cast<std::ptrdiff_t>(take), ready.end());
+        for (size_t s = 0; s < static_cast<size_t>(kRowSlots); ++s)
+        {
+          // an empty slot subtracts zeros from the zero of x
+          uint32_t head = zero_x | (kNoDivisor << 16);
+          std::array<uint32_t, 4 * kRowSlots> words;
+          words.fill(zero | (zero_x << 16));
+          if (s < take)
+          {
+            const Task& t = tasks[ready[s]];
+            const SubstitutionRow& r = rows[t.row];
+            head = r.out | ((t.last ? r.diag : kNoDivisor) << 16);
+            for (uint32_t q = 0; q < t.count; ++q)
+              words[4 * (q % kRowSlots) + q / kRowSlots] = r.terms[t.first + q];
+            groups = std::max(groups, static_cast<int32_t>((t.count + kRowSlots - 1) / kRowSlots));
+            for (uint32_t x : succ[ready[s]])
+              if (--left[x] == 0)
+                next.push_back(x);
+          }
+          out.heads.push_back(head);
+          out.terms.insert(out.terms.end(), words.begin(), words.end());
+        }
+        out.groups.push_back(groups);
+        ready.swap(next);
+      }
+      return out;
+    }
+
+    // Number of levels of a substitution's or the factorisation's head for a block that
+    // starts at row `first` (tail_size's cost estimate).
+    struct TailEstimate
+    {
+      int64_t lu_rounds = 0, fwd_levels = 0, bwd_levels = 0;
+    };
+
+    TailEstimate tail_estimate(const MechanismTables& t, int32_t first)
+    {
+      const int32_t n = static_cast<int32_t>(t.n_species);
+      TailEstimate e;
+      auto rounds = [](std::vector<int64_t>& width, int64_t cap) {
+        int64_t r = 0;
+        for (int64_t w : width)
+          r += (w + cap - 1) / cap;
+        return r;
+      };
+      auto count = [](std::vector<int64_t>& width, int32_t l) {
+        if (static_cast<size_t>(l) >= width.size())
+          width.resize(static_cast<size_t>(l) + 1, 0);
+        ++width[static_cast<size_t>(l)];
+      };
+      std::vector<int32_t> lvl_l(t.lower_col.size(), 0), lvl_u(t.upper_col.size(), 0);
+      std::vector<int64_t> width;
+      for (size_t q = 0; q < t.lu_out.size(); ++q)
+      {
+        int32_t l = 0, terms = 0;
+        for (int32_t k = t.lu_term_offsets[q]; k < t.lu_term_offsets[q + 1]; ++k)
+        {
+          if (t.lower_col[t.lu_term_l[k]] >= first)
+            break;
+          l = std::max({ l, lvl_l[t.lu_term_l[k]], lvl_u[t.lu_term_u[k]] });
+          ++terms;
+        }
+        const bool lower = t.lu_div[q] >= 0;
+        const bool divides = lower && t.lower_col[t.lu_out[q]] < first;
+        if (divides)
+          l = std::max(l, lvl_u[t.lu_div[q]]);
+        if (terms > 0 || divides)
+        {
+          count(width, l);
+          ++l;
+        }
+        (lower ? lvl_l : lvl_u)[t.lu_out[q]] = l;
+      }
+      e.lu_rounds = rounds(width, 256);
+      std::vector<int32_t> lvl(n, 0);
+      width.clear();
+      for (int32_t i = 0; i < n; ++i)
+      {
+        int32_t l = -1;
+        for (int32_t q = t.fwd_offsets[i]; q < t.fwd_offsets[i + 1] && t.fwd_col[q] < first; ++q)
+          l = std::max(l, lvl[t.fwd_col[q]]);
+        if (l >= 0)
+          count(width, l);
+        lvl[i] = l + 1;
+      }
+      e.fwd_levels = rounds(width, kRowSlots);
+      std::fill(lvl.begin(), lvl.end(), 0);
+      width.clear();
+      for (int32_t i = first - 1; i >= 0; --i)
+      {
+        int32_t l = 0;
+        for (int32_t q = t.bwd_offsets[i]; q < t.bwd_offsets[i + 1] && t.bwd_col[q] < first; ++q)
+          l = std::max(l, lvl[t.bwd_col[q]]);
+        count(width, l);
+        lvl[i] = l + 1;
+      }
+      e.bwd_levels = rounds(width, kRowSlots);
+      return e;
+    }
+
+    // The block's size: the one with the least estimated clocks of one factorisation and
+    // four substitutions, from the measured cost of a level of the head's schedules and of
+    // a pivot, column and row of the block.
+    int32_t tail_size(const MechanismTables& t)
+    {
+      const int32_t n = static_cast<int32_t>(t.n_species);
+      constexpr int64_t kLuRound = 1000, kRowLevel = 480, kPivot = 260, kPivotElement = 10, kColumn = 42, kRow = 100,
+                        kRowGroup = 87;
+      int32_t best = 0;
+      int64_t best_cost = 0;
+      for (int32_t d = kTailBlock; d <= kTailMax && d <= n; d += kTailBlock)
+      {
+        const TailEstimate e = tail_estimate(t, n - d);
+        int64_t cost = kLuRound * e.lu_rounds + 4 * kRowLevel * (e.fwd_levels + e.bwd_levels) + 4 * kColumn * d;
+        for (int64_t q = 1; q <= d / kTailBlock; ++q)
+          cost += kTailBlock * (kPivot + kPivotElement * q * q + 4 * (kRow + kRowGroup * q));
+        if (best == 0 || cost < best_cost)
+        {
+          best = d;
+          best_cost = cost;
+        }
+      }
+      return best;
+    }
+
+    void build_tail_tables(MechanismTables& t)
+    {
+      TailTables& tail = t.tail;
+      tail = TailTables{};
+      const int32_t n = static_cast<int32_t>(t.n_species);
+      if (!t.coop_levels_ok)
+        return;
+      const int32_t d = tail_size(t);
+      if (d == 0)
+        return;
+      const int32_t first = n - d, stride = d + 1;
+      // ALU position -> position with the block
+      std::vector<int32_t> pos(t.alu_col.size());
+      int32_t head = 0;
+      for (int32_t i = 0; i < n; ++i)
+        for (int32_t p = t.alu_row_ptr[i]; p < t.alu_row_ptr[i + 1]; ++p)
+          if (i < first || t.alu_col[p] < first)
+            pos[p] = head++;
+      tail.row_mask.assign(static_cast<size_t>(d), 0);
+      for (int32_t i = first; i < n; ++i)
+        for (int32_t p = t.alu_row_ptr[i]; p < t.alu_row_ptr[i + 1]; ++p)
+          if (t.alu_col[p] >= first)
+          {
+            pos[p] = head + (i - first) * stride + (t.alu_col[p] - first);
+            tail.row_mask[static_cast<size_t>(i - first)] |= uint64_t(1) << (t.alu_col[p] - first);
+          }
+      if (head + d * stride >= static_cast<int32_t>(kUnitDivisor))
+        return;
+      tail.size = d;
+      tail.first = first;
+      tail.head = head;
+      tail.nnz = head + d * stride;
+      for (int32_t p : t.jac_to_alu)
+        tail.jac_pos.push_back(pos[p]);
+      for (int32_t p : t.alu_diag)
+        tail.diag_pos.push_back(pos[p]);
+      const uint32_t zero = static_cast<uint32_t>(tail.nnz), zero_x = static_cast<uint32_t>(n);
+      // LU: the products with pivots before the block; elements outside the block complete,
+      // with their division, the block's without one
+      {
+        std::vector<int32_t> level(t.alu_col.size(), 0), ready;
+        std::vector<uint32_t> terms;
+        std::vector<LevelTask> tasks;
+        for (size_t e = 0; e < t.lu_out.size(); ++e)
+        {
+          const bool lower = t.lu_div[e] >= 0;
+          const int32_t out = lower ? t.alu_lower[t.lu_out[e]] : t.alu_upper[t.lu_out[e]];
+          const bool divides = lower && t.lower_col[t.lu_out[e]] < first;
+          const int32_t diag = divides ? t.alu_upper[t.lu_div[e]] : -1;
+          terms.clear();
+          ready.clear();
+          for (int32_t q = t.lu_term_offsets[e]; q < t.lu_term_offsets[e + 1]; ++q)
+          {
+            if (t.lower_col[t.lu_term_l[q]] >= first)
+              break;  // pivots ascend
+            const int32_t l = t.alu_lower[t.lu_term_l[q]], u = t.alu_upper[t.lu_term_u[q]];
+            terms.push_back(static_cast<uint32_t>(pos[l]) | (static_cast<uint32_t>(pos[u]) << 16));
+            ready.push_back(std::max(level[l], level[u]));
+          }
+          if (terms.empty() && !divides)
+            continue;
+          level[out] = add_segments(tasks, static_cast<uint32_t>(pos[out]),
+                                    divides ? static_cast<uint32_t>(pos[diag]) : kNoDivisor, terms, ready,
+                                    divides ? level[diag] : 0, kLuBlockingDefault) + 1;
+        }
+        const TaskOrder order = task_order(tasks);
+        const std::vector<int32_t> capped = cap_levels(tasks, order, 256);
+        tail.lu = pack_levels(tasks, &capped, zero * 0x10001u);
+      }
+      // substitutions: rows and row parts that read x before the block (forward) and the
+      // rows before the block (back)
+      {
+        std::vector<SubstitutionRow> rows;
+        for (int32_t i = 0; i < n; ++i)
+        {
+          SubstitutionRow r;
+          r.out = static_cast<uint32_t>(i);
+          for (int32_t q = t.fwd_offsets[i]; q < t.fwd_offsets[i + 1] && t.fwd_col[q] < first; ++q)
+            r.terms.push_back(static_cast<uint32_t>(pos[t.alu_lower[t.fwd_mat[q]]]) |
+                              (static_cast<uint32_t>(t.fwd_col[q]) << 16));
+          if (!r.terms.empty())
+            rows.push_back(std::move(r));
+        }
+        tail.fwd = row_levels(rows, n, zero, zero_x);
+        rows.clear();
+        for (int32_t i = first - 1; i >= 0; --i)
+        {
+          SubstitutionRow r;
+          r.out = static_cast<uint32_t>(i);
+          r.diag = static_cast<uint32_t>(pos[t.alu_diag[i]]);
+          for (int32_t q = t.bwd_offsets[i]; q < t.bwd_offsets[i + 1]; ++q)
+            r.terms.push_back(static_cast<uint32_t>(pos[t.alu_upper[t.bwd_mat[q]]]) |
+                              (static_cast<uint32_t>(t.bwd_col[q]) << 16));
+          rows.push_back(std::move(r));
+        }
+        tail.bwd = row_levels(rows, n, zero, zero_x);
+      }
+    }
+
     // Tables of the discrete adjoint.  The transposed substitutions have no counterpart in
     // the reference; their sums run in ascending column order.
     void build_adjoint_tables(MechanismTables& t)
@@ -1159,6 +1467,7 @@ namespace micm_hip
       t.bwd_offsets.push_back(static_cast<int32_t>(t.bwd_mat.size()));
     }
     build_cooperative_schedule(t);
+    build_tail_tables(t);
     build_adjoint_tables(t);
     for (size_t i = 0; i < t.lu_term_l.size(); ++i)
     {

@@ -91,6 +91,39 @@ namespace micm_hip
   constexpr int kChainLanes = 64;
   constexpr int kChainTasks = 128;  // the headers sit in two registers of each lane
 
+  // Rows of a substitution outside the dense tail (TailTables), sixteen tasks a level: the
+  // sixteen lanes of one DPP row of a wavefront form a task's products and subtract them in
+  // order (tail.hpp, ordered_sub16).  Slot s of level l is task 16 l + s.
+  struct RowLevels
+  {
+    std::vector<uint32_t> heads;   // per slot: out | diag << 16 (kNoDivisor: no division)
+    std::vector<uint32_t> terms;   // per slot 16 lanes x 4 words: term 16 g + lane (ALU position | x position << 16)
+    std::vector<int32_t> groups;   // per level: groups of sixteen terms of its longest task
+    int32_t n_levels() const { return static_cast<int32_t>(groups.size()); }
+  };
+  constexpr int kRowSlots = 16;
+  constexpr int kRowTerms = 64;  // a longer row continues in a task of a later level
+
+  // The last `size` rows and columns of the factor as a dense block (see tail.hpp): the
+  // pivots before it run as level schedules over the remaining (head) positions, the block
+  // itself is factorised in registers and its triangles are solved by one wavefront.
+  // Position of an element: the head elements in row order, then the block row by row with
+  // size + 1 doubles a row (an odd stride, so that a column's rows fall in different LDS
+  // banks), then one zero.
+  struct TailTables
+  {
+    int32_t size = 0;  // a multiple of 16 up to 64; 0: none
+    int32_t first = 0;  // first row of the block
+    int32_t head = 0;  // elements outside the block
+    int32_t nnz = 0;   // positions without the zero
+    std::vector<int32_t> jac_pos, diag_pos;  // of a Jacobian element, of a species' diagonal
+    std::vector<uint64_t> row_mask;          // per block row: its columns in the fill pattern
+    LevelSchedule lu;                        // products with pivots before the block
+    RowLevels fwd, bwd;
+  };
+  constexpr int kTailBlock = 16;
+  constexpr int kTailMax = 64;
+
   // Rate parameters as consumed by the device (per sorted reaction, stride
   // MICM_HIP_RATE_PARAM_STRIDE).  Derived values live in spare slots:
   //   BRANCHED  slot 5 = k0, slot 6 = z   (reaction_rate_store.hpp:286-293)
@@ -165,6 +198,7 @@ namespace micm_hip
     ColumnSweep fwd_sweep;  // lv_fwd's last levels as a column sweep
     TaskChain bwd_chain;    // lv_bwd's first levels as a task chain
     LevelSchedule lv_bwd;  // out = row, diag = U[i][i] position, terms (ALU position | column << 16)
+    TailTables tail;
     // packed operands: reaction -> reactant ids, Jacobian term -> (process, dependent ids);
     // three / two 16-bit ids and the count in bits 48-63 (0xffff: more, use the lists)
     std::vector<uint64_t> rxn_pack, term_pack;
