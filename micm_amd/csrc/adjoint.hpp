@@ -49,18 +49,6 @@ namespace micm_hip
     const int32_t* hes_slot;
   };
 
-  // Checkpoints of recorded Solves: per cell max_records records of n_species + 1 doubles,
-  // (H, y at the start of an accepted step) or (kClampTag, y before the post-solve clamp);
-  // counts[cell] records written so far (above max_records: the tape overflowed and later
-  // records were dropped).
-  struct Tape
-  {
-    double* records;
-    int64_t* counts;
-    int64_t max_records;
-  };
-  constexpr double kClampTag = -1.0;
-
   __host__ __device__ inline size_t adjoint_lds_doubles(int nnz_alu, int n, int stages, int n_reactions, int n_terms)
   {
     const int tmp = n_reactions > n_terms ? n_reactions : n_terms;

@@ -92,7 +92,6 @@ namespace micm_hip
   {
     const uint32_t* heads;
     const uint4* terms;  // sixteen per task: lane k's terms k, 16 + k, 32 + k, 48 + k
-    const int32_t* groups;
     int32_t n_levels;
   };
 
@@ -105,7 +104,10 @@ namespace micm_hip
     const int32_t* diag_pos;
     const uint64_t* row_mask;
     DevLevels lu;
-    DevRows fwd, bwd;
+    // the forward substitution's levels (fwd_levels, padded to fwd_padded), then the back
+    // substitution's (up to bwd_end, padded to rows.n_levels), the first two levels again
+    DevRows rows;
+    int32_t fwd_levels, fwd_padded, bwd_end;
   };
 
   // Tables of the cooperative (one workgroup per cell) form; see MechanismTables.
@@ -173,6 +175,18 @@ namespace micm_hip
     int32_t status;  // MICM_HIP_STATE_*
     int64_t stats[7];
   };
+
+  // Checkpoints of recorded Solves: per cell max_records records of n_species + 1 doubles,
+  // (H, y at the start of an accepted step) or (kClampTag, y before the post-solve clamp);
+  // counts[cell] records written so far (above max_records: the tape overflowed and later
+  // records were dropped).
+  struct Tape
+  {
+    double* records;
+    int64_t* counts;
+    int64_t max_records;
+  };
+  constexpr double kClampTag = -1.0;
 
   constexpr int32_t kRejectLast = 1, kRejectMore = 2, kNewStep = 4, kJacobianDue = 8;
 

@@ -214,8 +214,8 @@ namespace micm_hip
     // in the same order and with the same rounding as in one long task, but the sum
     // starts as soon as its first operands exist instead of when its last one does.
     // The last segment runs no earlier than `final_min` and carries the divisor; an
-    // element without products gets one task that only divides.  Returns the level
-    // of the last segment.
+    // element without products gets one task that only divides.  No segment is longer than
+    // max_len.  Returns the level of the last segment.
     // Shortest segment (except an element's last) of the substitution sums; the LU's is a
     // choice (kLuBlockings): its many short segments can cost more in per-task overhead
     // than they save in chain length, the substitutions' do not (measured on MI355X for
@@ -223,7 +223,8 @@ namespace micm_hip
     constexpr size_t kSolveSegmentMin = 1;
 
     int32_t add_segments(std::vector<LevelTask>& out, uint32_t pos, uint32_t diag, const std::vector<uint32_t>& terms,
-                         const std::vector<int32_t>& ready, int32_t final_min, size_t min_len)
+                         const std::vector<int32_t>& ready, int32_t final_min, size_t min_len,
+                         size_t max_len = ~size_t(0))
     {
       const size_t first = out.size();
       int32_t lv = 0;
@@ -231,7 +232,7 @@ namespace micm_hip
       {
         lv = std::max(lv, ready[q]);
         size_t e = q + 1;
-        while (e < terms.size() && (ready[e] <= lv || e - q < min_len))
+        while (e < terms.size() && e - q < max_len && (ready[e] <= lv || e - q < min_len))
         {
           lv = std::max(lv, ready[e]);
           ++e;
@@ -243,6 +244,7 @@ namespace micm_hip
         seg.terms.assign(terms.begin() + static_cast<std::ptrdiff_t>(q), terms.begin() + static_cast<std::ptrdiff_t>(e));
         out.push_back(std::move(seg));
         q = e;
+        ++lv;  // the next segment continues the partial sum
       }
       if (out.size() == first)
       {
@@ -838,7 +840,6 @@ namespace micm_hip
           return tasks[a].count > tasks[b].count;
         });
         const size_t take = std::min<size_t>(ready.size(), kRowSlots);
-        int32_t groups = 0;
         next.assign(ready.begin() + static_cast<std::ptrdiff_t>(take), ready.end());
         for (size_t s = 0; s < static_cast<size_t>(kRowSlots); ++s)
         {
@@ -853,7 +854,6 @@ namespace micm_hip
             head = r.out | ((t.last ? r.diag : kNoDivisor) << 16);
             for (uint32_t q = 0; q < t.count; ++q)
               words[4 * (q % kRowSlots) + q / kRowSlots] = r.terms[t.first + q];
-            groups = std::max(groups, static_cast<int32_t>((t.count + kRowSlots - 1) / kRowSlots));
             for (uint32_t x : succ[ready[s]])
               if (--left[x] == 0)
                 next.push_back(x);
@@ -861,7 +861,7 @@ namespace micm_hip
           out.heads.push_back(head);
           out.terms.insert(out.terms.end(), words.begin(), words.end());
         }
-        out.groups.push_back(groups);
+        ++out.n_levels_;
         ready.swap(next);
       }
       return out;
@@ -1002,7 +1002,9 @@ namespace micm_hip
         tail.diag_pos.push_back(pos[p]);
       const uint32_t zero = static_cast<uint32_t>(tail.nnz), zero_x = static_cast<uint32_t>(n);
       // LU: the products with pivots before the block; elements outside the block complete,
-      // with their division, the block's without one
+      // with their division, the block's without one.  Sums in runs of the terms that a
+      // task's record carries: with short blocks of products split off as they become
+      // ready (kLuBlockingDefault) 210/560 takes 56 levels of 256 tasks, in whole runs 36.
       {
         std::vector<int32_t> level(t.alu_col.size(), 0), ready;
         std::vector<uint32_t> terms;
@@ -1027,7 +1029,7 @@ namespace micm_hip
             continue;
           level[out] = add_segments(tasks, static_cast<uint32_t>(pos[out]),
                                     divides ? static_cast<uint32_t>(pos[diag]) : kNoDivisor, terms, ready,
-                                    divides ? level[diag] : 0, kLuBlockingDefault) + 1;
+                                    divides ? level[diag] : 0, kInlineTerms, kInlineTerms) + 1;
         }
         const TaskOrder order = task_order(tasks);
         const std::vector<int32_t> capped = cap_levels(tasks, order, 256);
@@ -1047,7 +1049,20 @@ namespace micm_hip
           if (!r.terms.empty())
             rows.push_back(std::move(r));
         }
-        tail.fwd = row_levels(rows, n, zero, zero_x);
+        tail.rows = row_levels(rows, n, zero, zero_x);
+        // empty levels up to a multiple of kRowPadding (at least that many in all, for the
+        // read ahead)
+        auto pad_levels = [&](int32_t least) {
+          while (tail.rows.n_levels() % kRowPadding != 0 || tail.rows.n_levels() < least)
+          {
+            tail.rows.heads.insert(tail.rows.heads.end(), kRowSlots, zero_x | (kNoDivisor << 16));
+            tail.rows.terms.insert(tail.rows.terms.end(), kRowSlots * kRowTerms, zero | (zero_x << 16));
+            ++tail.rows.n_levels_;
+          }
+          return tail.rows.n_levels();
+        };
+        tail.fwd_levels = tail.rows.n_levels();
+        tail.fwd_padded = pad_levels(0);
         rows.clear();
         for (int32_t i = first - 1; i >= 0; --i)
         {
@@ -1059,7 +1074,17 @@ namespace micm_hip
                               (static_cast<uint32_t>(t.bwd_col[q]) << 16));
           rows.push_back(std::move(r));
         }
-        tail.bwd = row_levels(rows, n, zero, zero_x);
+        const RowLevels back = row_levels(rows, n, zero, zero_x);
+        tail.rows.heads.insert(tail.rows.heads.end(), back.heads.begin(), back.heads.end());
+        tail.rows.terms.insert(tail.rows.terms.end(), back.terms.begin(), back.terms.end());
+        tail.rows.n_levels_ += back.n_levels_;
+        tail.bwd_end = tail.rows.n_levels();
+        pad_levels(kRowPadding);
+        // the next solve's first records
+        for (int32_t k = 0; k < 2 * kRowSlots; ++k)
+          tail.rows.heads.push_back(tail.rows.heads[static_cast<size_t>(k)]);
+        for (int32_t k = 0; k < 2 * kRowSlots * kRowTerms; ++k)
+          tail.rows.terms.push_back(tail.rows.terms[static_cast<size_t>(k)]);
       }
     }
 

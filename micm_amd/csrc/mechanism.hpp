@@ -97,11 +97,14 @@ namespace micm_hip
   struct RowLevels
   {
     std::vector<uint32_t> heads;   // per slot: out | diag << 16 (kNoDivisor: no division)
-    std::vector<uint32_t> terms;   // per slot 16 lanes x 4 words: term 16 g + lane (ALU position | x position << 16)
-    std::vector<int32_t> groups;   // per level: groups of sixteen terms of its longest task
-    int32_t n_levels() const { return static_cast<int32_t>(groups.size()); }
+    // per slot 16 lanes x 4 words: term 16 g + lane (ALU position | x position << 16), past a
+    // task's last term the factor's zero and a zero of x
+    std::vector<uint32_t> terms;
+    int32_t n_levels_ = 0;
+    int32_t n_levels() const { return n_levels_; }
   };
   constexpr int kRowSlots = 16;
+  constexpr int kRowPadding = 3;
   constexpr int kRowTerms = 64;  // a longer row continues in a task of a later level
 
   // The last `size` rows and columns of the factor as a dense block (see tail.hpp): the
@@ -119,7 +122,11 @@ namespace micm_hip
     std::vector<int32_t> jac_pos, diag_pos;  // of a Jacobian element, of a species' diagonal
     std::vector<uint64_t> row_mask;          // per block row: its columns in the fill pattern
     LevelSchedule lu;                        // products with pivots before the block
-    RowLevels fwd, bwd;
+    // the forward substitution's levels, empty ones up to fwd_padded, the back substitution's
+    // up to bwd_end, empty ones, the first two levels again; both padded counts are multiples
+    // of kRowPadding (tail_solve's unrolling)
+    RowLevels rows;
+    int32_t fwd_levels = 0, fwd_padded = 0, bwd_end = 0;
   };
   constexpr int kTailBlock = 16;
   constexpr int kTailMax = 64;

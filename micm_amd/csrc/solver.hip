@@ -17,7 +17,7 @@
 //   COOPERATIVE -- per-cell step size; one workgroup per cell (coop.hpp), cells from
 //                 a work queue, in the previous Solve's cost order once there was one.
 #include "adjoint.hpp"
-#include "tail.hpp"
+#include "coop_tail.hpp"
 #include "coop.hpp"
 #include "device.hpp"
 #include "mechanism.hpp"
@@ -1648,267 +1648,6 @@ namespace
       coop_sync<NT>();
     }
   }
-
-  // ---- cooperative form with the factor's dense block (tail.hpp): one workgroup of 256
-  // threads per cell, for mechanisms of up to 256 species.  LDS holds what other threads
-  // read: the factor (head, block, zero), y, one vector x (stage inputs, right-hand sides
-  // and solutions, x[n] = 0) and a scratch area shared in time by the reaction rates, the
-  // Jacobian's partial products, the block's pivots and the error terms.  Thread i keeps
-  // species i's stage vectors, f(y) and accumulated Jacobian diagonal in registers; rate
-  // constants are read from a per-workgroup copy in global memory.
-  //
-  // Bound by the dependency chain of one attempt.  An attempt of the slowest cell, two waves
-  // per SIMD, against the level-scheduled compact layout it replaced: 210/560 366 -> 154 us,
-  // 60/200 110 -> 53 us, TS1 190 -> 79 us.
-  __host__ __device__ inline size_t tail_scratch_doubles(int n, int n_reactions, int n_terms)
-  {
-    int scratch = kTailBuffer;
-    if (n_reactions > scratch)
-      scratch = n_reactions;
-    if (n_terms > scratch)
-      scratch = n_terms;
-    const int padded = (n + kTailBlock - 1) / kTailBlock * kTailBlock;
-    return static_cast<size_t>(scratch > padded ? scratch : padded);
-  }
-  // y starts at an even position, so that the scratch area (16-byte accesses) does too
-  __host__ __device__ inline size_t tail_lds_doubles(int nnz, int n, int n_reactions, int n_terms)
-  {
-    return ((static_cast<size_t>(nnz) + 1 + 2 * static_cast<size_t>(n) + 1 + 1) & ~size_t(1)) +
-           tail_scratch_doubles(n, n_reactions, n_terms);
-  }
-
-  template<int MINW, bool RECORD>
-  __global__ void __launch_bounds__(kTailThreads, MINW)
-      k_coop_tail(DevMech m, DevCoop c, DevTail t, DevParams p, int64_t n_fixed, const int32_t* __restrict__ list,
-                  const int* list_count, int* next, const CellControl* resume, double* __restrict__ y_state,
-                  double* __restrict__ k_state, const double* __restrict__ atol, int32_t* status_out,
-                  int64_t* stats_out, double* final_time_out, const double* __restrict__ cond_state,
-                  const double* __restrict__ custom_state, double* __restrict__ k_wg, Tape tape)
-  {
-    constexpr int NT = kTailThreads;
-    extern __shared__ double lds[];
-    __shared__ int s_idx;
-    __shared__ int s_flags[NT / kWave];
-    const int tid = threadIdx.x;
-    const int n = m.n_species;
-    const bool mine = tid < n;  // this thread has a species
-    CoopLds L{};
-    L.alu = lds;
-    L.y = lds + t.nnz + 1;
-    double* const x = L.y + n;
-    L.scratch = lds + ((static_cast<size_t>(t.nnz) + 1 + 2 * static_cast<size_t>(n) + 1 + 1) & ~size_t(1));
-    L.jterm = L.scratch;
-    L.k = k_wg + static_cast<size_t>(blockIdx.x) * m.n_reactions;
-    c.jac_to_alu = t.jac_pos;
-    const int64_t count = list ? static_cast<int64_t>(*list_count) : n_fixed;
-    const int diag = mine ? t.diag_pos[tid] : 0;
-    const double atol_r = mine ? atol[tid] : 1.0;
-    const int sum_groups = (n + kTailBlock - 1) / kTailBlock;
-    double one = 1.0;
-    asm("" : "+v"(one));
-    while (true)
-    {
-      if (tid == 0)
-        s_idx = atomicAdd(next, 1);
-      coop_sync<NT>();
-      const int64_t idx = s_idx;
-      coop_sync<NT>();
-      if (idx >= count)
-        return;
-      const int64_t cell = list ? list[idx] : idx;
-      const size_t g = cell / kGroup;
-      const int cl = cell % kGroup;
-      {
-        Lane ys = lane_view(y_state, g, n, cl);
-        Lane ks = lane_view(k_state, g, m.n_reactions, cl);
-        if (mine)
-          L.y[tid] = ys[tid];
-        if (tid == 0)
-          x[n] = 0.0;
-        if (cond_state)
-        {
-          // UpdateStateParameters fused into the launch
-          Lane cd = lane_view(const_cast<double*>(cond_state), g, 3, cl);
-          Lane cu = lane_view(const_cast<double*>(custom_state), g, m.n_custom, cl);
-          const double T = cd[0], P = cd[1], rho = cd[2];
-          for (int r = tid; r < m.n_reactions; r += NT)
-          {
-            const double kr = rate_constant(m, r, T, P, rho, cu);
-            L.k[r] = kr;
-            ks[r] = kr;
-          }
-        }
-        else
-        {
-          for (int r = tid; r < m.n_reactions; r += NT)
-            L.k[r] = ks[r];
-        }
-      }
-      CellControl cc;
-      if (resume)
-        cc = resume[cell];
-      else
-        control_init(p, cc);
-      // recorded Solve: the cell's checkpoints are appended to its tape
-      int64_t n_rec = RECORD ? tape.counts[cell] : 0;
-      double* const rec_base =
-          RECORD ? tape.records + static_cast<size_t>(cell) * tape.max_records * (static_cast<size_t>(n) + 1) : nullptr;
-      auto record = [&](double tag) {
-        if (n_rec < tape.max_records)
-        {
-          double* rec = rec_base + static_cast<size_t>(n_rec) * (static_cast<size_t>(n) + 1);
-          if (tid == 0)
-            rec[0] = tag;
-          if (mine)
-            rec[1 + tid] = L.y[tid];
-        }
-        ++n_rec;
-      };
-      coop_sync<NT>();
-      double f0 = 0.0, jdiag = 0.0;
-      while (true)
-      {
-        bool fresh = false;
-        if (cc.flags & kNewStep)
-        {
-          if (!begin_step(p, cc))
-            break;
-          f0 = coop_forcing_own<NT>(m, c, L, L.y);
-          coop_sync<NT>();
-          cc.stats[MICM_HIP_STAT_FUNCTION_CALLS] += 1;
-          cc.stats[MICM_HIP_STAT_JACOBIAN_UPDATES] += 1;
-          cc.last_alpha = 0.0;
-          cc.flags &= ~kNewStep;
-          fresh = true;
-        }
-        const double alpha = next_alpha(p, cc);
-        // -J(y) again (y and k are those of the step), its diagonal replaced by the
-        // accumulated one: the same values as keeping -J and adding alpha in place.  A
-        // factor with values that are not finite is formed again with the block's products
-        // tested one by one.
-        bool masked = false;
-        while (true)
-        {
-          for (int q = tid; q <= t.nnz; q += NT)
-            L.alu[q] = 0.0;
-          coop_jacobian<NT, true>(m, c, L);
-          if (mine)
-          {
-            if (fresh && !masked)
-              jdiag = L.alu[diag];
-            if (!masked)
-              jdiag += alpha * 1.0;
-            L.alu[diag] = jdiag;
-          }
-          coop_sync<NT>();
-          coop_levels_piped<NT, true>(t.lu, t.lu.terms, L.alu, L.alu, L.alu);
-          if (masked)
-          {
-            tail_factor<true>(t, L.alu, L.scratch, s_flags);
-            break;
-          }
-          if (tail_factor<false>(t, L.alu, L.scratch, s_flags))
-            break;
-          masked = true;
-        }
-        cc.stats[MICM_HIP_STAT_DECOMPOSITIONS] += 1;
-        // stage vectors of this thread's species (indexed by unrolled loops only)
-        double K[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
-        double f = f0;
-        const double y_r = mine ? L.y[tid] : 0.0;
-        for (int s = 0; s < p.stages; ++s)
-        {
-          const int sc = s * (s - 1) / 2;
-          if (s > 0 && p.new_f[s])
-          {
-            double v = y_r;
-#pragma unroll
-            for (int j = 0; j < 5; ++j)
-              if (j < s)
-                v += p.a[sc + j] * K[j];
-            if (mine)
-              x[tid] = v;
-            coop_sync<NT>();
-            f = coop_forcing_own<NT>(m, c, L, x);
-            cc.stats[MICM_HIP_STAT_FUNCTION_CALLS] += 1;
-          }
-          double v = f;
-#pragma unroll
-          for (int j = 0; j < 5; ++j)
-            if (j < s)
-              v += (p.c[sc + j] / cc.H) * K[j];
-          if (mine)
-            x[tid] = v;
-          coop_sync<NT>();
-          tail_solve(t, L.alu, x, masked);
-          const double Ks = mine ? x[tid] : 0.0;
-#pragma unroll
-          for (int j = 0; j < 6; ++j)
-            K[j] = j == s ? Ks : K[j];
-          cc.stats[MICM_HIP_STAT_SOLVES] += 1;
-        }
-        double ynew = y_r, e = 0.0;
-#pragma unroll
-        for (int s = 0; s < 6; ++s)
-          if (s < p.stages)
-            ynew += p.m[s] * K[s];
-#pragma unroll
-        for (int s = 0; s < 6; ++s)
-          if (s < p.stages)
-            e += p.e[s] * K[s];
-        if (tid < sum_groups * kTailBlock)
-        {
-          const double a = fabs(y_r), b = fabs(ynew);
-          const double q = e / (atol_r + p.rtol * (a > b ? a : b));
-          L.scratch[tid] = mine ? q * q : 0.0;
-        }
-        coop_sync<NT>();
-        // every wavefront adds the terms in species order
-        double acc = 0.0;
-        {
-          const double* terms = L.scratch + (tid & (kTailBlock - 1));
-          double q = terms[0];
-          for (int h = 0; h < sum_groups; ++h)
-          {
-            const double qn = terms[kTailBlock * (h + 1 < sum_groups ? h + 1 : h)];
-            acc = ordered_sub16<0>(acc, q, one);
-            q = qn;
-          }
-        }
-        const double error = smax(sqrt(acc / static_cast<double>(n > 0 ? n : 1)), 1.0e-10);
-        const double h_used = cc.H;
-        if (control_update(p, cc, error))
-        {
-          if constexpr (RECORD)
-            record(h_used);
-          if (mine)
-            L.y[tid] = ynew;
-        }
-        coop_sync<NT>();
-        if (cc.status != MICM_HIP_STATE_RUNNING)
-          break;
-      }
-      if constexpr (RECORD)
-      {
-        record(kClampTag);
-        if (tid == 0)
-          tape.counts[cell] = n_rec;
-      }
-      if (mine)
-      {
-        Lane ys = lane_view(y_state, g, n, cl);
-        ys[tid] = smax(L.y[tid], 0.0);
-      }
-      if (tid == 0)
-      {
-        status_out[cell] = cc.status;
-        for (int i = 0; i < 7; ++i)
-          stats_out[cell * 7 + i] = cc.stats[i];
-        final_time_out[cell] = cc.t;
-      }
-      coop_sync<NT>();
-    }
-  }
 }  // namespace
 
 // ====================================================================== C-ABI
@@ -2086,7 +1825,6 @@ namespace
     const uint32_t* terms = nullptr;
     upload(blob, off, r.terms, terms, staging);
     d.terms = reinterpret_cast<const uint4*>(terms);
-    upload(blob, off, r.groups, d.groups, staging);
     d.n_levels = r.n_levels();
   }
 
@@ -2097,10 +1835,8 @@ namespace
 
   size_t tail_bytes(const TailTables& t)
   {
-    size_t bytes = padded_bytes(t.jac_pos) + padded_bytes(t.diag_pos) + padded_bytes(t.row_mask) + level_bytes(t.lu);
-    for (const RowLevels* r : { &t.fwd, &t.bwd })
-      bytes += padded_bytes(r->heads) + padded_bytes(r->terms) + padded_bytes(r->groups);
-    return bytes;
+    return padded_bytes(t.jac_pos) + padded_bytes(t.diag_pos) + padded_bytes(t.row_mask) + level_bytes(t.lu) +
+           padded_bytes(t.rows.heads) + padded_bytes(t.rows.terms);
   }
 
   size_t blocked_level_bytes(const MechanismTables& t)
@@ -2389,8 +2125,10 @@ namespace
       upload(m->blob, off, t.tail.diag_pos, tl.diag_pos, staging);
       upload(m->blob, off, t.tail.row_mask, tl.row_mask, staging);
       upload_levels(m->blob, off, t.tail.lu, tl.lu, staging);
-      upload_rows(m->blob, off, t.tail.fwd, tl.fwd, staging);
-      upload_rows(m->blob, off, t.tail.bwd, tl.bwd, staging);
+      upload_rows(m->blob, off, t.tail.rows, tl.rows, staging);
+      tl.fwd_levels = t.tail.fwd_levels;
+      tl.fwd_padded = t.tail.fwd_padded;
+      tl.bwd_end = t.tail.bwd_end;
     }
     DevAdjoint& a = m->adj;
     upload_levels(m->blob, off, t.lv_ut, a.ut, staging);
@@ -2451,15 +2189,6 @@ namespace
       case 1024: return coop_occupancy_nt<1024>(stage, compact, lds);
       default: return coop_occupancy_nt<kWave>(stage, compact, lds);
     }
-  }
-
-  int tail_occupancy(int min_waves, size_t lds)
-  {
-    int per_cu = 0;
-    const hipError_t e =
-        min_waves == 3 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_coop_tail<3, false>, kTailThreads, lds)
-                       : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_coop_tail<2, false>, kTailThreads, lds);
-    return e == hipSuccess ? per_cu : 0;
   }
 
   size_t lds_limit()
@@ -2604,8 +2333,8 @@ namespace
     {
       const size_t lds =
           tail_lds_doubles(m->tail.nnz, m->dev.n_species, m->dev.n_reactions, c.n_terms) * sizeof(double);
-      const int occ3 = lds <= lds_limit() ? tail_occupancy(3, lds) : 0;
-      const int occ2 = lds <= lds_limit() ? tail_occupancy(2, lds) : 0;
+      const int occ3 = lds <= lds_limit() ? coop_tail_occupancy(3, lds) : 0;
+      const int occ2 = lds <= lds_limit() ? coop_tail_occupancy(2, lds) : 0;
       if (occ3 > 0 || occ2 > 0)
       {
         plan.lds = lds;
@@ -2697,7 +2426,7 @@ namespace
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     blocks = static_cast<int64_t>(cus) *
-             std::max(plan.tail ? tail_occupancy(plan.min_waves, plan.lds)
+             std::max(plan.tail ? coop_tail_occupancy(plan.min_waves, plan.lds)
                                 : coop_occupancy(plan.threads, plan.stage, plan.compact, plan.lds),
                       1);
     return MICM_HIP_OK;
@@ -2759,29 +2488,26 @@ namespace
     }
   }
 
-  template<int MINW, bool RECORD>
   int launch_coop_tail(micm_hip_state* s, const DevParams& p, const CoopPlan& plan, const int32_t* list,
                        const int* count, int64_t n_fixed, const CellControl* resume, bool update_rates, hipStream_t st)
   {
     const micm_hip_mechanism* m = s->mech;
-    const void* fn = reinterpret_cast<const void*>(k_coop_tail<MINW, RECORD>);
-    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(plan.lds)));
     int64_t blocks = 0;
     if (int rc = coop_blocks(plan, blocks))
       return rc;
     const bool ext = s->ext_next != nullptr;
-    int* next = ext ? s->ext_next : s->coop_next;
-    double* k_rows = ext ? s->ext_k : s->coop_k;
     if ((ext ? s->ext_k_rows : s->coop_k_rows) < blocks)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "cooperative scratch not prepared");
     if (!list)
       blocks = std::max<int64_t>(1, std::min(blocks, n_fixed));
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, next);
-    hipLaunchKernelGGL((k_coop_tail<MINW, RECORD>), dim3(static_cast<unsigned>(blocks)), dim3(kTailThreads), plan.lds,
-                       st, m->dev, m->coop, m->tail, p, n_fixed, list, count, next, resume, s->y, s->k, s->atol,
-                       s->status, s->stats, s->final_time, update_rates ? s->cond : nullptr,
-                       update_rates ? s->custom : nullptr, k_rows, s->recording);
-    HIP_TRY(hipGetLastError());
+    const CoopTailArgs a{ m->dev,          m->coop,  m->tail,   p,        n_fixed,
+                          list,            count,    ext ? s->ext_next : s->coop_next,
+                          resume,          s->y,     s->k,      s->atol,  s->status,
+                          s->stats,        s->final_time,       update_rates ? s->cond : nullptr,
+                          update_rates ? s->custom : nullptr,   ext ? s->ext_k : s->coop_k,
+                          s->recording };
+    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, a.next);
+    HIP_TRY(coop_tail_launch(plan.min_waves, static_cast<unsigned>(blocks), plan.lds, st, a));
     return MICM_HIP_OK;
   }
 
@@ -2792,14 +2518,7 @@ namespace
     if (plan.lds == 0)
       return fail(MICM_HIP_ERR_UNSUPPORTED, "the cooperative form does not fit this mechanism in LDS");
     if (plan.tail)
-    {
-      if (s->recording.records)
-        return plan.min_waves == 3
-                   ? launch_coop_tail<3, true>(s, p, plan, list, count, n_fixed, resume, update_rates, st)
-                   : launch_coop_tail<2, true>(s, p, plan, list, count, n_fixed, resume, update_rates, st);
-      return plan.min_waves == 3 ? launch_coop_tail<3, false>(s, p, plan, list, count, n_fixed, resume, update_rates, st)
-                                 : launch_coop_tail<2, false>(s, p, plan, list, count, n_fixed, resume, update_rates, st);
-    }
+      return launch_coop_tail(s, p, plan, list, count, n_fixed, resume, update_rates, st);
     switch (plan.threads)
     {
       case 128: return launch_coop_nt<128>(s, p, plan, list, count, n_fixed, resume, update_rates, st);

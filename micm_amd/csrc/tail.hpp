@@ -18,16 +18,17 @@
 // right-hand sides and every difference of unlike values round to +0) -- unless u is
 // infinite or NaN.  Every result of the block is therefore checked to be finite, and a cell
 // with one that is not is done again with each product tested against the fill pattern
-// (MASKED), which is exact for every operand.
+// (tail_factor_masked, tail_masked), which is exact for every operand.
 #pragma once
 
 #include "coop.hpp"
+#include "coop_tail.hpp"
 
 #include <type_traits>
 
 namespace micm_hip
 {
-  constexpr int kTailThreads = 256;
+  static_assert(kTailBuffer == 4 * kTailMax && kTailBlock == 16, "as coop_tail.hpp has them");
 
   // v - p[K0] - ... - p[15], subtracted in that order, p[k] being lane k's p of the reader's
   // DPP row of sixteen lanes.  One instruction a product: the multiply by m1 = -1 is exact,
@@ -68,20 +69,16 @@ namespace micm_hip
     return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
   }
 
-  // Doubles of LDS that tail_factor uses besides the factor: two buffers of a pivot row and
-  // a pivot column.
-  constexpr int kTailBuffer = 4 * kTailMax;
-
   // Pivots 16 (PA - p0) ... + 15 of a block of 4 - p0 sixteens: thread (ti, tj) holds the
   // elements (ti + 16 (a - p0), tj + 16 (b - p0)) as e[a][b].  At a pivot its row and column
   // go through LDS (two buffers, so one barrier a pivot); every four lanes divide one
   // column value each and pass the quotients on by DPP, and each thread updates its
   // elements below and right of the pivot.  Elements that are final already see a zero
   // factor.
-  template<int PA, bool MASKED>
-  __device__ __forceinline__ void tail_pivots(double (&e)[4][4], const DevTail& t, int p0, int ti, int tj, double* buf,
-                                              const uint64_t (&rm)[4])
+  template<int PA>
+  __device__ __forceinline__ void tail_pivots(double (&e)[4][4], int ti, int tj, double* buf)
   {
+#pragma unroll 1
     for (int kk = 0; kk < kTailBlock; ++kk)
     {
       double* row = buf + (kk & 1) * (2 * kTailMax);
@@ -120,48 +117,28 @@ namespace micm_hip
         l[2] = quad_lane<2>(q);
         l[3] = quad_lane<3>(q);
       }
-      if constexpr (!MASKED)
+      const double u_pa = tj > kk ? u[PA] : 0.0, l_pa = ti > kk ? l[PA] : 0.0;
+#pragma unroll
+      for (int a = PA; a < 4; ++a)
       {
-        const double u_pa = tj > kk ? u[PA] : 0.0, l_pa = ti > kk ? l[PA] : 0.0;
+        const double la = a == PA ? l_pa : l[a];
 #pragma unroll
-        for (int a = PA; a < 4; ++a)
-        {
-          const double la = a == PA ? l_pa : l[a];
-#pragma unroll
-          for (int b = PA; b < 4; ++b)
-            e[a][b] -= la * (b == PA ? u_pa : u[b]);
-          if (tj == kk && (a > PA || ti > kk))
-            e[a][PA] = l[a];
-        }
-      }
-      else
-      {
-        const int k = kTailBlock * (PA - p0) + kk;
-        const uint64_t rk = const_load(t.row_mask, k);
-#pragma unroll
-        for (int a = PA; a < 4; ++a)
-          if ((a > PA || ti > kk) && ((rm[a] >> k) & 1u))
-          {
-#pragma unroll
-            for (int b = PA; b < 4; ++b)
-              if ((b > PA || tj > kk) && ((rk >> (tj + kTailBlock * (b - p0))) & 1u))
-                e[a][b] -= l[a] * u[b];
-            if (tj == kk)
-              e[a][PA] = l[a];
-          }
+        for (int b = PA; b < 4; ++b)
+          e[a][b] -= la * (b == PA ? u_pa : u[b]);
+        if (tj == kk && (a > PA || ti > kk))
+          e[a][PA] = l[a];
       }
     }
   }
 
   // The block's own factorisation in place (A: the factor, its head and the block's sums
-  // over the head's pivots final), 256 threads.  False (on every thread) when an element is
-  // not finite; the block is then left as it is, if not MASKED.  buf: kTailBuffer doubles;
-  // flags: one int per wave.  Ends with a barrier.
+  // over the head's pivots final), 256 threads.  False (on every thread), the block left as
+  // it is, when an element is not finite.  buf: kTailBuffer doubles; flags: one int per
+  // wave.  Ends with a barrier.
   //
   // One pivot costs an LDS round trip with a barrier (140 clocks), a division (53) and ten
   // clocks for each of a thread's elements, whatever the fill; the level schedule of the
   // same rows takes two levels a pivot at 1,400 each.
-  template<bool MASKED>
   __device__ inline bool tail_factor(const DevTail& t, double* A, double* buf, int* flags)
   {
     const int tid = threadIdx.x;
@@ -170,7 +147,6 @@ namespace micm_hip
     const int stride = t.size + 1;
     double* base = A + t.head + ti * stride + tj;
     double e[4][4];
-    uint64_t rm[4] = { 0, 0, 0, 0 };
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -180,20 +156,13 @@ namespace micm_hip
         if (a >= p0 && b >= p0)
           e[a][b] = base[kTailBlock * (stride * (a - p0) + (b - p0))];
       }
-    if constexpr (MASKED)
-    {
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-        if (a >= p0)
-          rm[a] = t.row_mask[ti + kTailBlock * (a - p0)];
-    }
     if (p0 <= 0)
-      tail_pivots<0, MASKED>(e, t, p0, ti, tj, buf, rm);
+      tail_pivots<0>(e, ti, tj, buf);
     if (p0 <= 1)
-      tail_pivots<1, MASKED>(e, t, p0, ti, tj, buf, rm);
+      tail_pivots<1>(e, ti, tj, buf);
     if (p0 <= 2)
-      tail_pivots<2, MASKED>(e, t, p0, ti, tj, buf, rm);
-    tail_pivots<3, MASKED>(e, t, p0, ti, tj, buf, rm);
+      tail_pivots<2>(e, ti, tj, buf);
+    tail_pivots<3>(e, ti, tj, buf);
     bool finite = true;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -205,7 +174,7 @@ namespace micm_hip
       flags[tid / kWave] = bad != 0;
     lds_barrier<kTailThreads>();
     const bool ok = (flags[0] | flags[1] | flags[2] | flags[3]) == 0;
-    if (MASKED || ok)
+    if (ok)
     {
 #pragma unroll
       for (int a = 0; a < 4; ++a)
@@ -218,220 +187,304 @@ namespace micm_hip
     return ok;
   }
 
-  // Rows of a substitution in levels of sixteen (DevRows), one task to a DPP row: lane k
-  // forms the products 16 g + k, the row subtracts them in order.  Records are read two
-  // levels ahead, as in coop_levels_piped; x[n] is a zero for the empty slots' lanes.
-  __device__ inline void tail_rows(const DevRows& r, const double* A, double* x, double m1)
+  // The block's factorisation in LDS with every product tested against the fill pattern
+  // (for values that are not finite; small code, not speed).  Ends with a barrier.
+  __device__ inline void tail_factor_masked(const DevTail& t, double* A)
   {
     const int tid = threadIdx.x;
-    const int nl = r.n_levels;
-    struct Rec
+    const int d = t.size, stride = d + 1;
+    double* B = A + t.head;
+#pragma unroll 1
+    for (int k = 0; k < d; ++k)
     {
-      uint32_t h;
-      uint4 t;
-    };
-    auto load = [&](int l) {
-      const int at = l < nl ? l : 0;
-      Rec c;
-      c.h = r.heads[at * kRowSlots + (tid >> 4)];
-      c.t = r.terms[at * kTailThreads + tid];
-      return c;
-    };
-    if (nl == 0)
-      return;
-    auto step = [&](int l, const Rec& cur, Rec& ahead) {
-      if (l >= nl)
-        return;
-      const int groups = const_load(r.groups, l);
-      ahead = load(l + 2);
-      settle(cur.t);
-      settle(uint4{ cur.h, 0u, 0u, 0u });
-      const uint32_t o = cur.h & 0xffffu, d = cur.h >> 16;
-      double v = x[o];
-      const double dv = d < kUnitDivisor ? A[d] : 1.0;
-      const double p0 = A[cur.t.x & 0xffffu] * x[cur.t.x >> 16];
-      if (groups <= 1)
+      const uint64_t rk = const_load(t.row_mask, k);
+      if (tid > k && tid < d && ((t.row_mask[tid] >> k) & 1u))
+        B[tid * stride + k] = B[tid * stride + k] / B[k * stride + k];
+      __syncthreads();
+#pragma unroll 1
+      for (int q = tid; q < d * kTailMax; q += kTailThreads)
       {
-        v = ordered_sub16<0>(v, p0, m1);
+        const int i = q / kTailMax, j = q % kTailMax;
+        if (i > k && j > k && j < d && ((t.row_mask[i] >> k) & 1u) && ((rk >> j) & 1u))
+          B[i * stride + j] -= B[i * stride + k] * B[k * stride + j];
       }
-      else
-      {
-        const double p1 = A[cur.t.y & 0xffffu] * x[cur.t.y >> 16];
-        if (groups == 2)
-        {
-          v = ordered_sub16<0>(v, p0, m1);
-          v = ordered_sub16<0>(v, p1, m1);
-        }
-        else
-        {
-          const double p2 = A[cur.t.z & 0xffffu] * x[cur.t.z >> 16];
-          const double p3 = A[cur.t.w & 0xffffu] * x[cur.t.w >> 16];
-          v = ordered_sub16<0>(v, p0, m1);
-          v = ordered_sub16<0>(v, p1, m1);
-          v = ordered_sub16<0>(v, p2, m1);
-          v = ordered_sub16<0>(v, p3, m1);
-        }
-      }
-      if (d < kUnitDivisor)
-        v = v / dv;
-      if ((tid & 15) == 0)
-        x[o] = v;
-      lds_barrier<kTailThreads>();
-    };
-    Rec r0 = load(0), r1 = load(1), r2;
-    for (int l = 0; l < nl; l += 3)
-    {
-      step(l, r0, r2);
-      step(l + 1, r1, r0);
-      step(l + 2, r2, r1);
+      __syncthreads();
     }
   }
 
-  // Rows 16 (G - p0) + 15 down to 16 (G - p0) of the block's back substitution.  xg[g]: lane
-  // l holds x of column 16 (g - p0) + l % 16, zero until it is known, so the products of the
-  // columns up to the row's own are zeros; z: lane i holds the forward result of row i.
-  template<int G, bool MASKED>
-  __device__ __forceinline__ void tail_back(double (&xg)[4], const DevTail& t, int p0, const double* block, double z,
-                                            double m1)
+  // Record of one thread in a level of DevRows: its DPP row's task and the lane's four terms.
+  struct RowRecord
   {
-    const int l16 = threadIdx.x & 15;
-    const int stride = t.size + 1;
-    const int first = kTailBlock * (G - p0);
-    const double* row = block + (first + kTailBlock - 1) * stride;  // the current row
-    double u[4], diag;
-#pragma unroll
-    for (int g = G; g < 4; ++g)
-      u[g] = row[kTailBlock * (g - p0) + l16];
-    diag = row[first + kTailBlock - 1];
-    auto rows = [&](auto quad) {
-      constexpr int K0 = decltype(quad)::value;
-      for (int rr = K0 + 3; rr >= K0; --rr)
-      {
-        const int i = first + rr;
-        // the next row's operands (the last row reads row 0 of the block again, unused)
-        const double* next = i > 0 ? row - stride : block;
-        double un[4];
-#pragma unroll
-        for (int g = G; g < 4; ++g)
-          un[g] = next[kTailBlock * (g - p0) + l16];
-        const double dn = next[i > 0 ? i - 1 : 0];
-        double v = readlane_f64(z, static_cast<uint32_t>(i));
-        double p[4];
-        const uint64_t rm = MASKED ? const_load(t.row_mask, i) : 0;
-#pragma unroll
-        for (int g = G; g < 4; ++g)
-        {
-          p[g] = u[g] * xg[g];
-          if constexpr (MASKED)
-          {
-            const int j = kTailBlock * (g - p0) + l16;
-            p[g] = j > i && ((rm >> j) & 1u) ? p[g] : 0.0;
-          }
-        }
-        v = ordered_sub16<K0>(v, p[G], m1);
-#pragma unroll
-        for (int g = G + 1; g < 4; ++g)
-          v = ordered_sub16<0>(v, p[g], m1);
-        v = v / diag;
-        xg[G] = l16 == rr ? v : xg[G];
-#pragma unroll
-        for (int g = G; g < 4; ++g)
-          u[g] = un[g];
-        diag = dn;
-        row = next;
-      }
-    };
-    rows(std::integral_constant<int, 12>{});
-    rows(std::integral_constant<int, 8>{});
-    rows(std::integral_constant<int, 4>{});
-    rows(std::integral_constant<int, 0>{});
+    uint32_t head;
+    uint4 terms;
+  };
+
+  __device__ __forceinline__ RowRecord row_record(const DevRows& r, int l)
+  {
+    // a uniform base and an unsigned lane offset: scalar address arithmetic
+    const uint32_t* heads = r.heads + l * kRowSlots;
+    const uint4* terms = r.terms + l * kTailThreads;
+    return RowRecord{ heads[threadIdx.x >> 4], terms[threadIdx.x] };
   }
 
-  // The block's forward columns and back rows by one wavefront; xt: x of the block's first
-  // row, replaced by the solution.  False (x unchanged) when a result is not finite, if not
-  // MASKED.
-  template<bool MASKED>
-  __device__ inline bool tail_substitute(const DevTail& t, const double* block, double* xt, double m1)
+  // The records of a substitution's first two levels, read before it starts.
+  struct RowsAhead
   {
-    const int lane = threadIdx.x & (kWave - 1), l16 = lane & 15;
-    const int d = t.size, stride = d + 1;
-    const int p0 = 4 - d / kTailBlock;
-    const bool has = lane < d;
-    const int r = has ? lane : 0;  // lanes past the block hold row 0, which no column changes
+    RowRecord r0, r1;
+  };
+
+  __device__ __forceinline__ RowsAhead rows_ahead(const DevRows& r)
+  {
+    return RowsAhead{ row_record(r, 0), row_record(r, 1) };
+  }
+
+  // One level of sixteen tasks, one to a DPP row: lane k forms the products 16 g + k, the
+  // row subtracts them in order; DIV: and divides (by one where a task has no divisor).  A
+  // wavefront skips the groups that none of its tasks has (its lanes' words are all `pad`).
+  // Every lane of a row writes the row's result: an exec mask around the write costs 70 of a
+  // level's 570 clocks.
+  template<bool DIV>
+  __device__ __forceinline__ void tail_level(const RowRecord& rec, uint32_t pad, const double* A, double* x, double m1)
+  {
+    const uint32_t o = rec.head & 0xffffu, d = rec.head >> 16;
+    const uint32_t w[4] = { rec.terms.x, rec.terms.y, rec.terms.z, rec.terms.w };
+    double v = x[o], dv = 1.0;
+    if constexpr (DIV)
+      dv = A[d < kUnitDivisor ? d : 0];
+    auto product = [&](int g) { return A[w[g] & 0xffffu] * x[w[g] >> 16]; };
+    const double p0 = product(0);
+    if (!__any(w[1] != pad))
+    {
+      v = ordered_sub16<0>(v, p0, m1);
+    }
+    else if (!__any(w[2] != pad))
+    {
+      const double p1 = product(1);
+      v = ordered_sub16<0>(v, p0, m1);
+      v = ordered_sub16<0>(v, p1, m1);
+    }
+    else
+    {
+      const double p1 = product(1), p2 = product(2), p3 = product(3);
+      v = ordered_sub16<0>(v, p0, m1);
+      v = ordered_sub16<0>(v, p1, m1);
+      v = ordered_sub16<0>(v, p2, m1);
+      v = ordered_sub16<0>(v, p3, m1);
+    }
+    if constexpr (DIV)
+    {
+      v = v / (d < kUnitDivisor ? dv : 1.0);
+      asm("" : "+v"(v));
+    }
+    x[o] = v;
+    lds_barrier<kTailThreads>();
+  }
+
+  // Rows 16 G + 15 down to 16 G of the back substitution of a block of D rows.  xg[g]: lane l
+  // holds x of column 16 g + l % 16, zero until it is known, so the products of the columns
+  // up to the row's own are zeros; zs: the forward result in LDS.  A row's operands are read
+  // while the row before it is summed.  Every address is a lane's base and a constant: the
+  // one wavefront issues an instruction every five clocks, so a row costs its products (5.4
+  // clocks each) and its instructions: 9.6 us for both triangles of 64 rows, 3.6 us of 32
+  // (13.6 and 5.7 us with the rows in a loop and their addresses formed in it).
+  template<int D, int G>
+  __device__ __forceinline__ void tail_back(double (&xg)[D / kTailBlock], const double* block, const double* zs,
+                                            double m1)
+  {
+    constexpr int Q = D / kTailBlock, S = D + 1;
+    const int l16 = threadIdx.x & 15;
+    const double* lane = block + l16;
+    double u[Q], diag, z;
+    constexpr int last = kTailBlock * G + kTailBlock - 1;
+#pragma unroll
+    for (int g = G; g < Q; ++g)
+      u[g] = lane[last * S + kTailBlock * g];
+    diag = block[last * S + last];
+    z = zs[last];
+#pragma unroll
+    for (int rr = kTailBlock - 1; rr >= 0; --rr)
+    {
+      const int i = kTailBlock * G + rr;
+      double v = z, p[Q];
+#pragma unroll
+      for (int g = G; g < Q; ++g)
+        p[g] = u[g] * xg[g];
+      const double d = diag;
+      if (rr > 0)
+      {
+#pragma unroll
+        for (int g = G; g < Q; ++g)
+          u[g] = lane[(i - 1) * S + kTailBlock * g];
+        diag = block[(i - 1) * S + i - 1];
+        z = zs[i - 1];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (rr >= 12)
+        v = ordered_sub16<12>(v, p[G], m1);
+      else if (rr >= 8)
+        v = ordered_sub16<8>(v, p[G], m1);
+      else if (rr >= 4)
+        v = ordered_sub16<4>(v, p[G], m1);
+      else
+        v = ordered_sub16<0>(v, p[G], m1);
+#pragma unroll
+      for (int g = G + 1; g < Q; ++g)
+        v = ordered_sub16<0>(v, p[g], m1);
+      v = v / d;
+      asm("" : "+v"(v));  // on every lane: no branch around the division
+      xg[G] = l16 == rr ? v : xg[G];
+    }
+  }
+
+  // The block's forward columns by one wavefront, lane = row; xt: x of the block's first row,
+  // replaced by the result.  False (xt unchanged) when a result is not finite.
+  template<int D>
+  __device__ __forceinline__ bool tail_forward(const double* block, double* xt)
+  {
+    constexpr int S = D + 1;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int r = lane < D ? lane : 0;  // lanes past the block hold row 0, which no column changes
     double v = xt[r];
-    const double* row = block + r * stride;
-    const uint64_t rm = MASKED ? t.row_mask[r] : 0;
+    const double* row = block + r * S;
     double a[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q)
       a[q] = row[q];
-    for (int c0 = 0; c0 < d; c0 += 8)
+#pragma unroll
+    for (int c0 = 0; c0 < D; c0 += 8)
     {
       double an[8];
-      const int n0 = c0 + 8 < d ? c0 + 8 : 0;
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        an[q] = row[n0 + q];
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
+      if (c0 + 8 < D)
       {
-        const int c = c0 + q;
-        const double xc = readlane_f64(v, static_cast<uint32_t>(c));
-        if constexpr (MASKED)
-        {
-          const double nv = v - a[q] * xc;
-          v = r > c && ((rm >> c) & 1u) ? nv : v;
-        }
-        else
-        {
-          v -= (r > c ? a[q] : 0.0) * xc;
-        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+          an[q] = row[c0 + 8 + q];
       }
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (c0 + q < D - 1)
+          v -= (r > c0 + q ? a[q] : 0.0) * readlane_f64(v, static_cast<uint32_t>(c0 + q));
 #pragma unroll
       for (int q = 0; q < 8; ++q)
         a[q] = an[q];
     }
-    double xg[4] = { 0.0, 0.0, 0.0, 0.0 };
-    bool finite = !has || __builtin_isfinite(v);
-    tail_back<3, MASKED>(xg, t, p0, block, v, m1);
-    if (p0 <= 2)
-      tail_back<2, MASKED>(xg, t, p0, block, v, m1);
-    if (p0 <= 1)
-      tail_back<1, MASKED>(xg, t, p0, block, v, m1);
-    if (p0 <= 0)
-      tail_back<0, MASKED>(xg, t, p0, block, v, m1);
+    const bool ok = __ballot(!__builtin_isfinite(v)) == 0;
+    if (ok && lane < D)
+      xt[lane] = v;
+    return ok;
+  }
+
+  // The block's back rows by one wavefront, as tail_forward.
+  template<int D>
+  __device__ __forceinline__ bool tail_backward(const double* block, double* xt, double m1)
+  {
+    constexpr int Q = D / kTailBlock;
+    double xg[Q];
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+    for (int g = 0; g < Q; ++g)
+      xg[g] = 0.0;
+    if constexpr (Q > 3)
+      tail_back<D, 3>(xg, block, xt, m1);
+    if constexpr (Q > 2)
+      tail_back<D, 2>(xg, block, xt, m1);
+    if constexpr (Q > 1)
+      tail_back<D, 1>(xg, block, xt, m1);
+    tail_back<D, 0>(xg, block, xt, m1);
+    bool finite = true;
+#pragma unroll
+    for (int g = 0; g < Q; ++g)
       finite = finite && __builtin_isfinite(xg[g]);
     const bool ok = __ballot(!finite) == 0;
-    if (MASKED || ok)
+    if (ok && (threadIdx.x & (kWave - 1)) < kTailBlock)
     {
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        if (g >= p0 && lane < kTailBlock)
-          xt[kTailBlock * (g - p0) + l16] = xg[g];
+      for (int g = 0; g < Q; ++g)
+        xt[kTailBlock * g + (threadIdx.x & 15)] = xg[g];
     }
     return ok;
   }
 
+  // tail_forward (DIR 0) or tail_backward (1) with every product tested against the fill
+  // pattern, row by row (for values that are not finite; small code, not speed).
+  template<int DIR>
+  __device__ inline void tail_masked(const DevTail& t, const double* block, double* xt)
+  {
+    const int d = t.size, stride = d + 1;
+    if ((threadIdx.x & (kWave - 1)) == 0)
+    {
+#pragma unroll 1
+      for (int q = 0; q < d; ++q)
+      {
+        const int i = DIR == 0 ? q : d - 1 - q;
+        double v = xt[i];
+#pragma unroll 1
+        for (int j = DIR == 0 ? 0 : i + 1; j < (DIR == 0 ? i : d); ++j)
+          if ((t.row_mask[i] >> j) & 1u)
+            v -= block[i * stride + j] * xt[j];
+        xt[i] = DIR == 0 ? v : v / block[i * stride + i];
+      }
+    }
+    coop_sync<kWave>();
+  }
+
+  // Both triangles of the block by one wavefront.
+  template<int D>
+  __device__ __forceinline__ void tail_substitute(const DevTail& t, const double* block, double* xt, bool masked,
+                                                  double m1)
+  {
+    if (masked || !tail_forward<D>(block, xt))
+      tail_masked<0>(t, block, xt);
+    coop_sync<kWave>();
+    if (masked || !tail_backward<D>(block, xt, m1))
+      tail_masked<1>(t, block, xt);
+  }
+
   // x <- U^-1 L^-1 x (x[n] = 0 behind it); masked: the factor holds values that are not
-  // finite.  Ends with a barrier.
-  __device__ inline void tail_solve(const DevTail& t, const double* A, double* x, bool masked)
+  // finite.  The record of level l + 2 is read while level l runs; the levels before and
+  // after the block are one list that ends in its first two levels again, whose records the
+  // next solve starts with (`ahead`).  Three records rotate, unrolled by three so that none
+  // moves; both passes' level counts are padded to multiples of three, so that each pass and
+  // the next solve start with the same record.  Ends with a barrier.
+  __device__ inline void tail_solve(const DevTail& t, const double* A, double* x, bool masked, RowsAhead& ahead)
   {
     double m1 = -1.0;
     asm("" : "+v"(m1));
-    tail_rows(t.fwd, A, x, m1);
+    const DevRows& r = t.rows;
+    const uint32_t pad = static_cast<uint32_t>(t.nnz) | (static_cast<uint32_t>(t.first + t.size) << 16);
+    RowRecord spare;
+    auto levels = [&](auto div, int begin, int end) {
+      constexpr bool DIV = decltype(div)::value;
+      auto step = [&](int l, const RowRecord& cur, RowRecord& next) {
+        next = row_record(r, l + 2);
+        if (l < end)
+        {
+          settle(cur.terms);
+          settle(uint4{ cur.head, 0u, 0u, 0u });
+          tail_level<DIV>(cur, pad, A, x, m1);
+        }
+      };
+#pragma unroll 1
+      for (int l = begin; l < end; l += kRowPadding)
+      {
+        step(l, ahead.r0, spare);
+        step(l + 1, ahead.r1, ahead.r0);
+        step(l + 2, spare, ahead.r1);
+      }
+    };
+    levels(std::false_type{}, 0, t.fwd_levels);
     if (threadIdx.x < kWave)
     {
-      const double* block = A + t.head;
+      const double* b = A + t.head;
       double* xt = x + t.first;
-      bool done = false;
-      if (!masked)
-        done = tail_substitute<false>(t, block, xt, m1);
-      if (!done)
-        tail_substitute<true>(t, block, xt, m1);
+      switch (t.size)
+      {
+        case 16: tail_substitute<16>(t, b, xt, masked, m1); break;
+        case 32: tail_substitute<32>(t, b, xt, masked, m1); break;
+        case 48: tail_substitute<48>(t, b, xt, masked, m1); break;
+        default: tail_substitute<64>(t, b, xt, masked, m1); break;
+      }
     }
     lds_barrier<kTailThreads>();
-    tail_rows(t.bwd, A, x, m1);
+    levels(std::true_type{}, t.fwd_padded, t.bwd_end);
   }
 }  // namespace micm_hip

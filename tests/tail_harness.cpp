@@ -51,9 +51,10 @@ namespace
     return true;
   }
 
-  bool run_rows(const RowLevels& r, const std::vector<double>& A, std::vector<double>& x, uint32_t zero_x)
+  bool run_rows(const RowLevels& r, int32_t first, int32_t last, const std::vector<double>& A, std::vector<double>& x,
+                uint32_t zero_x)
   {
-    for (int32_t l = 0; l < r.n_levels(); ++l)
+    for (int32_t l = first; l < last; ++l)
     {
       const std::vector<double> x0 = x;
       std::vector<char> written(x.size(), 0);
@@ -63,22 +64,18 @@ namespace
         if (o != zero_x && written.at(o)++)
           return false;
       }
-      if (r.groups[l] < 0 || r.groups[l] > 4)
-        return false;
       for (int s = 0; s < kRowSlots; ++s)
       {
         const size_t slot = static_cast<size_t>(l) * kRowSlots + s;
         const uint32_t o = r.heads[slot] & 0xffffu, d = r.heads[slot] >> 16;
         double v = x0.at(o);
-        const int run = r.groups[l] <= 1 ? 1 : r.groups[l] == 2 ? 2 : 4;  // as tail_rows
         for (int q = 0; q < 64; ++q)
         {
           const uint32_t tr = r.terms.at(slot * 64 + 4 * (q % 16) + q / 16);
           const bool pad = (tr >> 16) == zero_x;
-          if (!pad && (q >= 16 * r.groups[l] || written.at(tr >> 16)))
+          if (!pad && written.at(tr >> 16))
             return false;
-          if (q < 16 * run)
-            v -= A.at(tr & 0xffffu) * x0.at(tr >> 16);
+          v -= A.at(tr & 0xffffu) * x0.at(tr >> 16);
         }
         if (d < kUnitDivisor)
           v /= A.at(d);
@@ -140,7 +137,12 @@ extern "C"
     std::vector<double> x(b, b + n);
     x.push_back(0.0);
     const uint32_t zero_x = static_cast<uint32_t>(n);
-    if (!run_rows(T.fwd, A, x, zero_x))
+    if (T.fwd_padded % kRowPadding != 0 || T.rows.n_levels() % kRowPadding != 0 || T.rows.n_levels() < kRowPadding || T.fwd_levels > T.fwd_padded ||
+        T.bwd_end > T.rows.n_levels() ||
+        T.rows.heads.size() != static_cast<size_t>(T.rows.n_levels() + 2) * kRowSlots ||
+        T.rows.terms.size() != T.rows.heads.size() * 64)
+      return -1;
+    if (!run_rows(T.rows, 0, T.fwd_levels, A, x, zero_x))
       return -1;
     double* xt = x.data() + T.first;
     for (int c = 0; c < d; ++c)
@@ -155,7 +157,7 @@ extern "C"
           v -= B[i * stride + j] * xt[j];
       xt[i] = v / B[i * stride + i];
     }
-    if (!run_rows(T.bwd, A, x, zero_x) || x[n] != 0.0)
+    if (!run_rows(T.rows, T.fwd_padded, T.bwd_end, A, x, zero_x) || x[n] != 0.0)
       return -1;
     std::memcpy(b, x.data(), sizeof(double) * n);
     return d;
@@ -167,8 +169,8 @@ extern "C"
     const MechanismTables t = compile_mechanism(*desc);
     out[0] = t.tail.size;
     out[1] = t.tail.lu.n_levels();
-    out[2] = t.tail.fwd.n_levels();
-    out[3] = t.tail.bwd.n_levels();
+    out[2] = t.tail.fwd_levels;
+    out[3] = t.tail.rows.n_levels();
     out[4] = t.tail.nnz;
     out[5] = static_cast<int64_t>(t.term_process.size());
     out[6] = t.tail.lu.max_terms;
