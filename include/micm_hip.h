@@ -311,8 +311,8 @@ int micm_hip_state_set_handoff(micm_hip_state* state, int64_t steps);
  * per-cell layout (no tables staged, fewer arrays in LDS so that more cells fit a CU;
  * needs more than 64 threads and at least one thread per species, else ignored).  With 256
  * threads and 16 to 256 species the compact layout is the kernel that takes the factor's last
- * rows as a dense block, which the library's choice of staging (-1) also picks; 5 / 6 / 7: that
- * kernel built for three waves per SIMD (168 registers) / two (256) / two, 4 leaving the choice
+ * rows as a dense block, which the library's choice of staging (-1) also picks for 256 threads or
+ * its own choice of threads; 5 / 6 / 7: that kernel built for three waves per SIMD (168 registers) / two (256) / two, 4 leaving the choice
  * to the occupancy.  A tuning
  * knob in the role of the vector length L of the reference's GPU policies
  * (cuda_solver_builder.hpp:24-38); results do not depend on it. */
@@ -342,8 +342,8 @@ int micm_hip_solve(const micm_hip_mechanism* mechanism, micm_hip_state* state, d
  * MICM_HIP_SOLVE_UPDATE_RATES) without allocating: no counterpart in the reference; for callers
  * that cannot allocate device memory (code under stream capture, tight serving loops).  The
  * launch's scratch (queue counter, the compact layout's rate-constant rows) lives in one static
- * 4 MiB device array per GPU; a launch shape needing more is refused with
- * MICM_HIP_ERR_INVALID_ARGUMENT.  Enqueued on the state's stream without waiting; results are
+ * 4 MiB device array per GPU; a requested launch shape needing more is refused with
+ * MICM_HIP_ERR_INVALID_ARGUMENT (the library's own choice takes a smaller grid).  Enqueued on the state's stream without waiting; results are
  * those of micm_hip_solve once the stream has finished.  Every call on one GPU shares that
  * array: calls that overlap on a GPU (other threads or streams) race. */
 int micm_hip_solve_noalloc(const micm_hip_mechanism* mechanism, micm_hip_state* state, double time_step,

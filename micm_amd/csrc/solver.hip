@@ -2310,9 +2310,43 @@ namespace
   CoopPlan plan_coop_full(const micm_hip_mechanism* m, int stages, int stage_request, int threads_request,
                           int lu_blocking);
 
-  // stage_request < 0: stage the substitution tables when they fit and the LU tables
-  // when that costs no resident cell per CU, or take the compact layout when that fits
-  // more cells per CU; 4: the compact layout; threads_request 0: one wavefront.
+  // The kernel with the factor's dense block (256 threads), where it takes the mechanism.
+  bool plan_tail(const micm_hip_mechanism* m, int stage_request, CoopPlan& plan)
+  {
+    if (m->tail.size == 0 || m->dev.n_species > kTailThreads)
+      return false;
+    const size_t lds =
+        tail_lds_doubles(m->tail.nnz, m->dev.n_species, m->dev.n_reactions, m->coop.n_terms) * sizeof(double);
+    if (lds > lds_limit())
+      return false;
+    const int occ3 = coop_tail_occupancy(3, lds), occ2 = coop_tail_occupancy(2, lds);
+    if (occ3 == 0 && occ2 == 0)
+      return false;
+    plan.lds = lds;
+    plan.stage = 0;
+    plan.threads = kTailThreads;
+    plan.p_capacity = 0;
+    plan.compact = true;
+    plan.tail = true;
+    // the register budget that fits the most cells per CU, the larger one among equals
+    plan.min_waves = occ3 > occ2 ? 3 : 2;
+    if (stage_request == 5 && occ3 > 0)
+      plan.min_waves = 3;
+    if (stage_request >= 6 && occ2 > 0)
+      plan.min_waves = 2;
+    return true;
+  }
+
+  // stage_request < 0: the kernel with the dense block for 256 threads, else stage the
+  // substitution tables when they fit and the LU tables when that costs no resident cell per
+  // CU, or take the compact layout when that fits more cells per CU; 4: the compact layout.
+  //
+  // threads_request 0 (with stage_request < 0): the kernel with the dense block where it takes
+  // the mechanism (16 to 256 species), else one wavefront.  The dense block beats one wavefront
+  // from the smallest such mechanism on: 20,000 cells of 20/50 in 28 ms instead of 44, 10,000
+  // of 30/90 in 33 instead of 74, of 60/200 in 47 instead of 148 (bound by their slowest
+  // cells); below 16 species one wavefront is faster than 256 threads (README system, 1,000
+  // cells: 0.23 ms against 0.37).
   CoopPlan plan_coop(const micm_hip_mechanism* m, int stages, int stage_request = -1, int threads_request = 0,
                      int lu_blocking = 0)
   {
@@ -2322,36 +2356,19 @@ namespace
     CoopPlan plan = plan_coop_full(m, stages, compact_request ? -1 : stage_request, threads_request, lu_blocking);
     if (!m->t.coop_levels_ok || (stage_request >= 0 && !compact_request))
       return plan;
+    if (threads_request == 0 && stage_request < 0 && plan.lds > 0)
+    {
+      (void)plan_tail(m, stage_request, plan);
+      return plan;
+    }
     // the compact layout keeps one species per thread in registers and publishes the
     // rate constants through global memory, so it needs a workgroup barrier
     const int threads = coop_threads_of(threads_request);
     const DevCoop c = coop_with_blocking(m, lu_blocking, threads);
     if (threads <= kWave || threads < m->dev.n_species)
       return plan;
-    // 256 threads: the kernel with the factor's dense block wherever it fits
-    if (threads == kTailThreads && m->tail.size > 0)
-    {
-      const size_t lds =
-          tail_lds_doubles(m->tail.nnz, m->dev.n_species, m->dev.n_reactions, c.n_terms) * sizeof(double);
-      const int occ3 = lds <= lds_limit() ? coop_tail_occupancy(3, lds) : 0;
-      const int occ2 = lds <= lds_limit() ? coop_tail_occupancy(2, lds) : 0;
-      if (occ3 > 0 || occ2 > 0)
-      {
-        plan.lds = lds;
-        plan.stage = 0;
-        plan.threads = threads;
-        plan.p_capacity = 0;
-        plan.compact = true;
-        plan.tail = true;
-        // the register budget that fits the most cells per CU, the larger one among equals
-        plan.min_waves = occ3 > occ2 ? 3 : 2;
-        if (stage_request == 5 && occ3 > 0)
-          plan.min_waves = 3;
-        if (stage_request >= 6 && occ2 > 0)
-          plan.min_waves = 2;
-        return plan;
-      }
-    }
+    if (threads == kTailThreads && plan_tail(m, stage_request, plan))
+      return plan;
     const size_t compact = coop_compact_lds_doubles(c.nnz_alu, m->dev.n_species, stages, m->dev.n_reactions,
                                                     c.n_terms, c.bwd.max_level_terms) *
                            sizeof(double);
@@ -2496,10 +2513,12 @@ namespace
     if (int rc = coop_blocks(plan, blocks))
       return rc;
     const bool ext = s->ext_next != nullptr;
-    if ((ext ? s->ext_k_rows : s->coop_k_rows) < blocks)
+    if (ext ? s->ext_k_rows < 1 : s->coop_k_rows < blocks)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "cooperative scratch not prepared");
     if (!list)
       blocks = std::max<int64_t>(1, std::min(blocks, n_fixed));
+    if (ext)
+      blocks = std::min(blocks, s->ext_k_rows);
     const CoopTailArgs a{ m->dev,          m->coop,  m->tail,   p,        n_fixed,
                           list,            count,    ext ? s->ext_next : s->coop_next,
                           resume,          s->y,     s->k,      s->atol,  s->status,
@@ -2545,11 +2564,30 @@ namespace
     return MICM_HIP_OK;
   }
 
+  // Whether a persistent Solve with the library's hand-off runs every cell in the cooperative
+  // form from its first attempt: with the dense block an attempt costs the cooperative form
+  // less than the per-lane form, whose lanes wait for each other's memory, except for small
+  // factors in numbers that fill the chip's lanes (64 lanes x 4 SIMDs x 256 CUs).  60/200:
+  // 20,011 cells 55 ms against 195 (hand-off after 16 steps) and 351 (48), 120,000 cells 250
+  // against 370 and 519; 210/560, 20,000 cells 394 against 1,424; 20/50: 10,000 cells 28
+  // against 41, 200,000 cells 97 against 67 ms.
+  constexpr int64_t kPerLaneFactor = 300;
+  constexpr int64_t kPerLaneCells = 65536;
+  constexpr int64_t kHandoffBlock = 16, kHandoffLevels = 48;  // default hand-off steps
+
+  bool hands_off_at_once(const micm_hip_state* s, const CoopPlan& plan)
+  {
+    return s->handoff_steps < 0 && plan.tail &&
+           (s->mech->coop.nnz_alu > kPerLaneFactor || s->n_cells < kPerLaneCells);
+  }
+
   int prepare_solve(micm_hip_state* s, int32_t form, int stages)
   {
     if (form == MICM_HIP_SOLVE_COOPERATIVE || form == MICM_HIP_SOLVE_PERSISTENT)
     {
       const CoopPlan plan = plan_coop(s->mech, stages, s->coop_stage, s->coop_threads, s->lu_blocking);
+      if (form == MICM_HIP_SOLVE_PERSISTENT && hands_off_at_once(s, plan))
+        form = MICM_HIP_SOLVE_COOPERATIVE;
       if (plan.compact)
       {
         int64_t rows = 0;
@@ -2622,7 +2660,8 @@ namespace
   {
     const micm_hip_mechanism* m = s->mech;
     const DevMech& d = m->dev;
-    if (form == MICM_HIP_SOLVE_COOPERATIVE)
+    const CoopPlan plan = plan_coop(m, p.stages, s->coop_stage, s->coop_threads, s->lu_blocking);
+    if (form == MICM_HIP_SOLVE_COOPERATIVE || hands_off_at_once(s, plan))
       return s->has_order ? launch_coop(s, p, s->order, s->order_bins + kOrderBins, 0, nullptr, update_rates, st)
                           : launch_coop(s, p, nullptr, nullptr, s->n_cells, nullptr, update_rates, st);
     int64_t blocks = 0;
@@ -2633,7 +2672,9 @@ namespace
     Work w = slot_work(s);
     DevParams pp = p;
     const bool coop_ok = coop_lds_bytes(m, p.stages) > 0;
-    pp.handoff_steps = !coop_ok ? 0 : (s->handoff_steps >= 0 ? s->handoff_steps : 48);
+    pp.handoff_steps = !coop_ok ? 0
+                       : s->handoff_steps >= 0 ? s->handoff_steps
+                       : plan.tail ? kHandoffBlock : kHandoffLevels;
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, s->queue_next);
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, s->handoff_count);
     Queue q{ s->queue_next, s->has_order ? s->order : nullptr };
@@ -3389,6 +3430,13 @@ extern "C"
     if (plan.compact)
       if (int rc = coop_blocks(plan, rows))
         return rc;
+    // where the library picked the kernel with the dense block, its grid is cut to the rows
+    // that fit (a smaller grid gives the same results); a requested compact layout that needs
+    // more is refused
+    if (plan.tail && s->coop_stage < 0)
+      rows = std::min<int64_t>(rows, static_cast<int64_t>((kNoAllocScratchBytes - kNoAllocCounterBytes) /
+                                                          (static_cast<size_t>(std::max(m->dev.n_reactions, 1)) *
+                                                           sizeof(double))));
     const size_t need = kNoAllocCounterBytes + static_cast<size_t>(rows) *
                                                    static_cast<size_t>(std::max(m->dev.n_reactions, 1)) * sizeof(double);
     if (need > kNoAllocScratchBytes)
