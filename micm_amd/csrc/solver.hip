@@ -21,6 +21,7 @@
 #include "coop.hpp"
 #include "device.hpp"
 #include "mechanism.hpp"
+#include "ordered_sum.hpp"
 #include "path.hpp"
 
 #include <hip/hip_runtime.h>
@@ -941,9 +942,12 @@ namespace
   // Ynew = Y + sum m_s K_s and Yerr = sum e_s K_s (combine_and_error's expressions)
   // with one thread per (cell, species) of the running cells, in the grouped layout's
   // order; k_plain_finish or (lockstep) k_lockstep_error and k_lockstep_control
-  // finish the attempt.
+  // finish the attempt.  LOCKSTEP: instead of Yerr, the terms of the State's error sum, at
+  // their places in the order that its dense matrix policy visits them (ordered_error).
+  template<bool LOCKSTEP>
   __global__ void __launch_bounds__(kBlock) k_combine_elem(DevMech m, DevParams p, int64_t n_cells, Work w,
-                                                               const CellControl* __restrict__ ctl)
+                                                               const CellControl* __restrict__ ctl,
+                                                               const double* __restrict__ atol)
   {
     const int64_t per_group = static_cast<int64_t>(m.n_species) * kGroup;
     const int64_t f = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
@@ -958,100 +962,91 @@ namespace
     for (int s = 0; s < p.stages; ++s)
       e += p.e[s] * w.K[static_cast<size_t>(s) * w.k_stride + f];
     w.ynew[f] = v;
-    w.yerr[f] = e;
+    if constexpr (LOCKSTEP)
+    {
+      const int i = static_cast<int>((f % per_group) / kGroup);
+      const int64_t gi = c / p.error_group, first = gi * p.error_group;
+      const int64_t rows = n_cells - first < p.error_group ? n_cells - first : p.error_group;
+      const double a = fabs(w.y[f]), b = fabs(v);
+      const double q = e / (atol[i] + p.rtol * (a > b ? a : b));
+      w.yerr[first * m.n_species + i * rows + (c - first)] = q * q;
+    }
+    else
+    {
+      w.yerr[f] = e;
+    }
   }
 
-  constexpr int kLockstepErrorThreads = 1024;
+  // Threads and terms of a thread per tile of the error sum: few wavefronts, whose runs are
+  // composed one after another, where the kernel only sums.
+  constexpr int kStateErrorThreads = 1024, kStateErrorTerms = 8;
+  constexpr int kLockstepErrorThreads = 512, kLockstepErrorTerms = 16;
 
   // The reference's NormalizedError for one State (rosenbrock.inl:353-402): one running
   // sum of the squared scaled errors in the order the State's dense matrix policy visits
   // them, then max(sqrt(sum / (cells * species)), 1e-10).  `group` is that policy's
   // vector length: 1 for Matrix<Real> (cell by cell, species inner), L for
   // VectorMatrix<L> (each group of L cells species by species, the group's cells inner,
-  // a partial last group over its own cells; vector_matrix.hpp:860-867).  The terms are
-  // formed by the whole workgroup a block at a time and added one after another by
-  // thread 0.  Every thread of the workgroup calls it; the result is thread 0's.
-  __device__ inline double ordered_error(int n, int64_t n_cells, int64_t group, const double* __restrict__ y,
-                                         const double* __restrict__ ynew, const double* __restrict__ yerr,
-                                         const double* __restrict__ atol, double rtol, double* terms)
+  // a partial last group over its own cells; vector_matrix.hpp:860-867).  Every thread of the
+  // workgroup calls it and gets the result.
+  template<int NT, int K, class Term>
+  __device__ inline double ordered_error(int n, int64_t n_cells, const Term& term, SumScratch<NT>& scratch)
   {
     const int64_t n_terms = n_cells * n;
-    const int64_t per_group = group * n;
-    double acc = 0.0;
-    for (int64_t base = 0; base < n_terms; base += kLockstepErrorThreads)
-    {
-      const int64_t f = base + threadIdx.x;
-      double q = 0.0;
-      if (f < n_terms)
-      {
-        const int64_t gi = f / per_group;
-        const int64_t off = f - gi * per_group;
-        const int64_t rows = n_cells - gi * group < group ? n_cells - gi * group : group;
-        const int i = static_cast<int>(off / rows);
-        const int64_t c = gi * group + off % rows;
-        const size_t g = c / kGroup;
-        const int cl = c % kGroup;
-        const double a = fabs(lane_view(const_cast<double*>(y), g, n, cl)[i]);
-        const double b = fabs(lane_view(const_cast<double*>(ynew), g, n, cl)[i]);
-        const double ymax = a > b ? a : b;
-        const double v = lane_view(const_cast<double*>(yerr), g, n, cl)[i] / (atol[i] + rtol * ymax);
-        q = v * v;
-      }
-      terms[threadIdx.x] = q;
-      __syncthreads();
-      if (threadIdx.x == 0)
-      {
-        const int cnt = static_cast<int>(n_terms - base < kLockstepErrorThreads ? n_terms - base
-                                                                                : kLockstepErrorThreads);
-        // sixteen reads in flight, then their additions in order
-        int j = 0;
-        for (; j + 16 <= cnt; j += 16)
-        {
-          double t[16];
-#pragma unroll
-          for (int u = 0; u < 16; ++u)
-            t[u] = terms[j + u];
-#pragma unroll
-          for (int u = 0; u < 16; ++u)
-            acc += t[u];
-        }
-        for (; j < cnt; ++j)
-          acc += terms[j];
-      }
-      __syncthreads();
-    }
     const double N = static_cast<double>(n_terms > 0 ? n_terms : 1);
-    return smax(sqrt(acc / N), 1.0e-10);
+    return smax(sqrt(ordered_sum<NT, K>(n_terms, term, scratch) / N), 1.0e-10);
   }
 
-  // Lockstep error of the state's attempt, in the order of the state's dense matrix policy.
-  __device__ inline double lockstep_error(const DevMech& m, const DevParams& p, int64_t n_cells, const Work& w,
-                                          const double* __restrict__ atol, double* terms)
+  // Term f of that sum from the state's arrays.
+  struct StateTerm
   {
-    return ordered_error(m.n_species, n_cells, p.error_group, w.y, w.ynew, w.yerr, atol, p.rtol, terms);
-  }
+    int n;
+    int64_t n_cells, group;
+    const double *y, *ynew, *yerr, *atol;
+    double rtol;
+    __device__ double operator()(int64_t f) const
+    {
+      const int64_t per_group = group * n;
+      const int64_t gi = f / per_group;
+      const int64_t off = f - gi * per_group;
+      const int64_t rows = n_cells - gi * group < group ? n_cells - gi * group : group;
+      const int i = static_cast<int>(off / rows);
+      const int64_t c = gi * group + off % rows;
+      const size_t g = c / kGroup;
+      const int cl = c % kGroup;
+      const double a = fabs(lane_view(const_cast<double*>(y), g, n, cl)[i]);
+      const double b = fabs(lane_view(const_cast<double*>(ynew), g, n, cl)[i]);
+      const double ymax = a > b ? a : b;
+      const double v = lane_view(const_cast<double*>(yerr), g, n, cl)[i] / (atol[i] + rtol * ymax);
+      return v * v;
+    }
+  };
 
-  __global__ void __launch_bounds__(kLockstepErrorThreads) k_state_error(int n, int64_t n_cells, int64_t group,
-                                                                         const double* y, const double* ynew,
-                                                                         const double* yerr, const double* atol,
-                                                                         double rtol, double* error_out)
+  __global__ void __launch_bounds__(kStateErrorThreads) k_state_error(int n, int64_t n_cells, int64_t group,
+                                                                      const double* y, const double* ynew,
+                                                                      const double* yerr, const double* atol,
+                                                                      double rtol, double* error_out)
   {
-    __shared__ double terms[kLockstepErrorThreads];
-    const double e = ordered_error(n, n_cells, group, y, ynew, yerr, atol, rtol, terms);
+    __shared__ SumScratch<kStateErrorThreads> scratch;
+    const double e = ordered_error<kStateErrorThreads, kStateErrorTerms>(
+        n, n_cells, StateTerm{ n, n_cells, group, y, ynew, yerr, atol, rtol }, scratch);
     if (threadIdx.x == 0)
       *error_out = e;
   }
 
-  __global__ void __launch_bounds__(kLockstepErrorThreads) k_lockstep_error(DevMech m, DevParams p, int64_t n_cells,
-                                                                            Work w, const CellControl* ctl,
-                                                                            const double* __restrict__ atol,
-                                                                            double* error_out)
+  // Lockstep error of the state's attempt from the terms that k_combine_elem<true> left in
+  // w.yerr.  Bound by the sum's order: 100,060 terms (20 species x 5,003 cells) take 677 us
+  // added one by one by a thread, about 225 as a chain of one instruction each, and 84 us in
+  // parallel (ordered_sum).
+  __global__ void __launch_bounds__(kLockstepErrorThreads) k_lockstep_error(int n, int64_t n_cells, const double* terms,
+                                                                            const CellControl* ctl, double* error_out)
   {
-    __shared__ double terms[kLockstepErrorThreads];
+    __shared__ SumScratch<kLockstepErrorThreads> scratch;
     // the cells share one control state: all stopped at the loop-top checks or none
     if (ctl[0].status != MICM_HIP_STATE_RUNNING)
       return;
-    const double e = lockstep_error(m, p, n_cells, w, atol, terms);
+    const double e = ordered_error<kLockstepErrorThreads, kLockstepErrorTerms>(
+        n, n_cells, [=](int64_t f) { return terms[f]; }, scratch);
     if (threadIdx.x == 0)
       *error_out = e;
   }
@@ -1092,7 +1087,7 @@ namespace
   // attempt.  Same operations in the same order, so the results are those of the
   // launch-per-phase loop.  Every exit condition and every barrier is uniform over
   // the workgroup.
-  constexpr int kFusedLockstepThreads = kLockstepErrorThreads;
+  constexpr int kFusedLockstepThreads = kStateErrorThreads;
   constexpr int64_t kFusedLockstepMaxCells = kFusedLockstepThreads;
   constexpr int64_t kFusedLockstepMaxFactor = 256;  // nnz of the in-place factor
 
@@ -1101,8 +1096,7 @@ namespace
                                                                             const double* __restrict__ atol,
                                                                             int64_t max_iterations)
   {
-    __shared__ double s_error;
-    __shared__ double s_terms[kFusedLockstepThreads];
+    __shared__ SumScratch<kFusedLockstepThreads> s_sum;
     const int n = m.n_species;
     for (int64_t it = 0; it < max_iterations; ++it)
     {
@@ -1129,13 +1123,8 @@ namespace
       // the cells share one control state: all stopped at the loop-top checks or none
       if (ctl[0].status != MICM_HIP_STATE_RUNNING)
         break;
-      {
-        const double e = lockstep_error(m, p, n_cells, w, atol, s_terms);
-        if (threadIdx.x == 0)
-          s_error = e;
-      }
-      __syncthreads();
-      const double error = s_error;
+      const double error = ordered_error<kFusedLockstepThreads, kStateErrorTerms>(
+          n, n_cells, StateTerm{ n, n_cells, p.error_group, w.y, w.ynew, w.yerr, atol, p.rtol }, s_sum);
       int running = 0;
       for (int64_t c = threadIdx.x; c < n_cells; c += kFusedLockstepThreads)
       {
@@ -3051,7 +3040,7 @@ extern "C"
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "negative cell count or vector length below 1");
     if (!error || (n_cells > 0 && (!y || !ynew || !errors || !atol)))
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null buffer");
-    hipLaunchKernelGGL(k_state_error, dim3(1), dim3(kLockstepErrorThreads), 0, static_cast<hipStream_t>(stream),
+    hipLaunchKernelGGL(k_state_error, dim3(1), dim3(kStateErrorThreads), 0, static_cast<hipStream_t>(stream),
                        m->dev.n_species, n_cells, vector_length, y, ynew, errors, atol, rtol, error);
     HIP_TRY(hipGetLastError());
     return MICM_HIP_OK;
@@ -3377,14 +3366,19 @@ extern "C"
           for (int stage = 0; stage < p.stages; ++stage)
             hipLaunchKernelGGL(k_plain_stage, dim3(grid), dim3(kBlock), 0, st, d, p, s->n_cells, w, s->ctl, stage);
         }
-        hipLaunchKernelGGL(k_combine_elem, dim3(pair_grid), dim3(kBlock), 0, st, d, p, s->n_cells, w, s->ctl);
+        if (!lockstep)
+          hipLaunchKernelGGL(k_combine_elem<false>, dim3(pair_grid), dim3(kBlock), 0, st, d, p, s->n_cells, w, s->ctl,
+                             s->atol);
+        else
+          hipLaunchKernelGGL(k_combine_elem<true>, dim3(pair_grid), dim3(kBlock), 0, st, d, p, s->n_cells, w, s->ctl,
+                             s->atol);
         if (!lockstep)
           hipLaunchKernelGGL(k_plain_finish, dim3(grid), dim3(kBlock), 0, st, d, p, s->n_cells, w, s->ctl, s->atol,
                              s->active);
         else
         {
-          hipLaunchKernelGGL(k_lockstep_error, dim3(1), dim3(kLockstepErrorThreads), 0, st, d, p, s->n_cells, w,
-                             s->ctl, s->atol, s->lockstep_error);
+          hipLaunchKernelGGL(k_lockstep_error, dim3(1), dim3(kLockstepErrorThreads), 0, st, d.n_species, s->n_cells,
+                             w.yerr, s->ctl, s->lockstep_error);
           hipLaunchKernelGGL(k_lockstep_control, dim3(grid), dim3(kBlock), 0, st, d, p, s->n_cells, w, s->ctl,
                              s->lockstep_error, s->active);
         }
