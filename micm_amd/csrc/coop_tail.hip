@@ -125,34 +125,22 @@ namespace
         }
         const double alpha = next_alpha(p, cc);
         // -J(y) again (y and k are those of the step), its diagonal replaced by the
-        // accumulated one: the same values as keeping -J and adding alpha in place.  A
-        // factor with values that are not finite is formed again with the block's products
-        // tested one by one.
-        bool masked = false;
-        while (true)
+        // accumulated one: the same values as keeping -J and adding alpha in place
+        for (int q = tid; q <= t.nnz; q += NT)
+          L.alu[q] = 0.0;
+        coop_jacobian<NT, true>(m, c, L);
+        if (mine)
         {
-          for (int q = tid; q <= t.nnz; q += NT)
-            L.alu[q] = 0.0;
-          coop_jacobian<NT, true>(m, c, L);
-          if (mine)
-          {
-            if (fresh && !masked)
-              jdiag = L.alu[diag];
-            if (!masked)
-              jdiag += alpha * 1.0;
-            L.alu[diag] = jdiag;
-          }
-          coop_sync<NT>();
-          coop_levels_piped<NT, true>(t.lu, t.lu.terms, L.alu, L.alu, L.alu);
-          if (masked)
-          {
-            tail_factor_masked(t, L.alu);
-            break;
-          }
-          if (tail_factor(t, L.alu, L.scratch, s_flags))
-            break;
-          masked = true;
+          if (fresh)
+            jdiag = L.alu[diag];
+          jdiag += alpha * 1.0;
+          L.alu[diag] = jdiag;
         }
+        coop_sync<NT>();
+        coop_levels_piped<NT, true>(t.lu, t.lu.terms, L.alu, L.alu, L.alu);
+        const bool masked = !tail_factor<false>(t, L.alu, L.scratch, s_flags);
+        if (masked)
+          tail_factor_masked(t, L.alu);
         cc.stats[MICM_HIP_STAT_DECOMPOSITIONS] += 1;
         // stage vectors of this thread's species (indexed by unrolled loops only)
         double K[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
@@ -252,6 +240,150 @@ namespace
     }
   }
 
+  // ---- single phases with the dense block, one cell per workgroup.  The cells of one group
+  // go to one XCD one after another and share the group's 128-byte lines in its L2 (workgroup b
+  // runs on XCD b % 8).
+  __device__ __forceinline__ bool cell_of_block(int64_t n_cells, size_t& g, int& cl)
+  {
+    constexpr unsigned kXcds = 8;
+    const unsigned x = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+    const int64_t grp = static_cast<int64_t>(j / kGroup) * kXcds + x;
+    g = static_cast<size_t>(grp);
+    cl = static_cast<int>(j % kGroup);
+    return grp * kGroup + cl < n_cells;
+  }
+
+  // A[map[p]] = src[p] of the cell for map[p] >= 0, eight loads in flight per thread; true on
+  // the threads that saw a -0.
+  __device__ __forceinline__ bool load_cell(double* A, const int32_t* map, const double* __restrict__ src, size_t g, int cl,
+                                            int n)
+  {
+    constexpr int NT = kTailThreads;
+    const double* base = src + g * static_cast<size_t>(n) * kGroup + cl;
+    bool negative_zero = false;
+    for (int p0 = threadIdx.x; p0 < n; p0 += 8 * NT)
+    {
+      double v[8];
+      int to[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+      {
+        const int p = p0 + j * NT < n ? p0 + j * NT : p0;
+        v[j] = base[static_cast<size_t>(p) * kGroup];
+        to[j] = map ? map[p] : p;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+      {
+        negative_zero = negative_zero || (v[j] == 0.0 && __builtin_signbit(v[j]));
+        if (p0 + j * NT < n && to[j] >= 0)
+          A[to[j]] = v[j];
+      }
+    }
+    return negative_zero;
+  }
+
+  // Whether any thread of the workgroup says so; ends with a barrier.
+  __device__ __forceinline__ bool any_thread(bool v, int* flags)
+  {
+    const uint64_t who = __ballot(v);
+    if ((threadIdx.x & (kWave - 1)) == 0)
+      flags[threadIdx.x / kWave] = who != 0;
+    __syncthreads();
+    const bool any = (flags[0] | flags[1] | flags[2] | flags[3]) != 0;
+    __syncthreads();
+    return any;
+  }
+
+  // LuDecompositionDoolittle::Decompose for one cell (lu_decomposition_doolittle.inl:325-403).
+  // Bound as the Solve's factorisation is by its chain, not by the 87 KB a 210/560 cell reads
+  // and writes: 4,096 cells in 545 us, 1,665 with the level schedule alone.
+  __global__ void __launch_bounds__(kTailThreads, 2)
+      k_lu_decompose_tail(DevMech m, DevTail t, int64_t n_cells, const double* __restrict__ jac,
+                          double* __restrict__ lower, double* __restrict__ upper)
+  {
+    constexpr int NT = kTailThreads;
+    extern __shared__ double lds[];
+    __shared__ int s_flags[NT / kWave];
+    size_t g;
+    int cl;
+    if (!cell_of_block(n_cells, g, cl))
+      return;
+    const int tid = threadIdx.x;
+    double* A = lds;
+    double* buf = lds + ((static_cast<size_t>(t.nnz) + 2) & ~size_t(1));
+    for (int q = tid; q <= t.nnz; q += NT)
+      A[q] = 0.0;
+    __syncthreads();
+    const bool exact = any_thread(load_cell(A, t.jac_pos, jac, g, cl, m.nnz_jac), s_flags);
+    coop_levels_piped<NT, true>(t.lu, t.lu.terms, A, A, A);
+    if (exact || !tail_factor<true>(t, A, buf, s_flags))
+      tail_factor_masked(t, A);
+    double* lo = lower + g * static_cast<size_t>(m.nnz_lower) * kGroup + cl;
+    for (int p = tid; p < m.nnz_lower; p += NT)
+    {
+      const int a = t.lower_pos[p];
+      lo[static_cast<size_t>(p) * kGroup] = a >= 0 ? A[a] : 1.0;
+    }
+    double* up = upper + g * static_cast<size_t>(m.nnz_upper) * kGroup + cl;
+    for (int p = tid; p < m.nnz_upper; p += NT)
+      up[static_cast<size_t>(p) * kGroup] = A[t.upper_pos[p]];
+  }
+
+  // LinearSolver::Solve for one cell (linear_solver.inl:235-294), dividing by L[i][i] as the
+  // reference does where it is not 1.  210/560, 4,096 cells: 341 us, 1,303 with the level
+  // schedules alone.
+  __global__ void __launch_bounds__(kTailThreads, 2)
+      k_lu_solve_tail(DevMech m, DevTail t, int64_t n_cells, const double* __restrict__ lower,
+                      const double* __restrict__ upper, double* __restrict__ xs)
+  {
+    constexpr int NT = kTailThreads;
+    extern __shared__ double lds[];
+    __shared__ int s_flags[NT / kWave];
+    size_t g;
+    int cl;
+    if (!cell_of_block(n_cells, g, cl))
+      return;
+    const int tid = threadIdx.x;
+    const int n = m.n_species;
+    double* A = lds;
+    double* x = A + t.nnz + 1;
+    double* ld = x + n + 1;
+    RowsAhead ahead = rows_ahead(t.rows);
+    // the block's structural zeros and the zero behind it
+    for (int q = t.head + tid; q <= t.nnz; q += NT)
+      A[q] = 0.0;
+    if (tid == 0)
+      x[n] = 0.0;
+    __syncthreads();
+    (void)load_cell(A, t.lower_pos, lower, g, cl, m.nnz_lower);
+    (void)load_cell(A, t.upper_pos, upper, g, cl, m.nnz_upper);
+    const bool exact = load_cell(x, nullptr, xs, g, cl, n);
+    bool diagonal = false;
+    for (int i = tid; i < n; i += NT)
+    {
+      ld[i] = lower[(g * m.nnz_lower + m.lower_diag[i]) * kGroup + cl];
+      diagonal = diagonal || ld[i] != 1.0;
+    }
+    const bool masked = any_thread(exact, s_flags);
+    if (any_thread(diagonal, s_flags))
+    {
+      // rows without off-diagonal L entries only divide; they are inputs of every level
+      for (int i = tid; i < t.first; i += NT)
+        if (m.fwd_offsets[i] == m.fwd_offsets[i + 1])
+          x[i] = x[i] / ld[i];
+      __syncthreads();
+      tail_solve_lower_diagonal(t, A, x, ld, ahead);
+    }
+    else
+    {
+      tail_solve(t, A, x, masked, ahead);
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += NT)
+      xs[(g * n + i) * kGroup + cl] = x[i];
+  }
+
   template<int MINW, bool RECORD>
   hipError_t launch(unsigned blocks, size_t lds, hipStream_t stream, const CoopTailArgs& a)
   {
@@ -281,5 +413,39 @@ namespace
     if (a.tape.records)
       return min_waves == 3 ? launch<3, true>(blocks, lds, stream, a) : launch<2, true>(blocks, lds, stream, a);
     return min_waves == 3 ? launch<3, false>(blocks, lds, stream, a) : launch<2, false>(blocks, lds, stream, a);
+  }
+
+  size_t tail_factor_lds(const DevTail& t)
+  {
+    return sizeof(double) * (((static_cast<size_t>(t.nnz) + 2) & ~size_t(1)) + kTailBuffer);
+  }
+
+  size_t tail_solve_lds(const DevMech& m, const DevTail& t)
+  {
+    return sizeof(double) * (static_cast<size_t>(t.nnz) + 1 + 2 * static_cast<size_t>(m.n_species) + 1);
+  }
+
+  hipError_t lu_decompose_tail(const DevMech& m, const DevTail& t, int64_t n_cells, unsigned blocks, const double* jac,
+                               double* lower, double* upper, hipStream_t stream)
+  {
+    const size_t lds = tail_factor_lds(t);
+    if (const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_lu_decompose_tail),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        e != hipSuccess)
+      return e;
+    hipLaunchKernelGGL(k_lu_decompose_tail, dim3(blocks), dim3(kTailThreads), lds, stream, m, t, n_cells, jac, lower, upper);
+    return hipGetLastError();
+  }
+
+  hipError_t lu_solve_tail(const DevMech& m, const DevTail& t, int64_t n_cells, unsigned blocks, const double* lower,
+                           const double* upper, double* x, hipStream_t stream)
+  {
+    const size_t lds = tail_solve_lds(m, t);
+    if (const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_lu_solve_tail),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        e != hipSuccess)
+      return e;
+    hipLaunchKernelGGL(k_lu_solve_tail, dim3(blocks), dim3(kTailThreads), lds, stream, m, t, n_cells, lower, upper, x);
+    return hipGetLastError();
   }
 }  // namespace micm_hip

@@ -52,4 +52,13 @@ namespace micm_hip
   // Workgroups per CU of the build for min_waves waves per SIMD (3 or 2), 0 where it does not fit.
   int coop_tail_occupancy(int min_waves, size_t lds);
   hipError_t coop_tail_launch(int min_waves, unsigned blocks, size_t lds, hipStream_t stream, const CoopTailArgs& a);
+
+  // The single phases with the block, one cell per workgroup (`blocks`: whole groups of cells
+  // for every XCD), and their LDS.
+  size_t tail_factor_lds(const DevTail& t);
+  size_t tail_solve_lds(const DevMech& m, const DevTail& t);
+  hipError_t lu_decompose_tail(const DevMech& m, const DevTail& t, int64_t n_cells, unsigned blocks, const double* jac,
+                               double* lower, double* upper, hipStream_t stream);
+  hipError_t lu_solve_tail(const DevMech& m, const DevTail& t, int64_t n_cells, unsigned blocks, const double* lower,
+                           const double* upper, double* x, hipStream_t stream);
 }  // namespace micm_hip

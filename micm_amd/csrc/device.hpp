@@ -102,6 +102,8 @@ namespace micm_hip
     int32_t first, head, nnz;
     const int32_t* jac_pos;
     const int32_t* diag_pos;
+    const int32_t* lower_pos;
+    const int32_t* upper_pos;
     const uint64_t* row_mask;
     DevLevels lu;
     // the forward substitution's levels (fwd_levels, padded to fwd_padded), then the back

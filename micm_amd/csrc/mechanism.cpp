@@ -1000,6 +1000,10 @@ namespace micm_hip
         tail.jac_pos.push_back(pos[p]);
       for (int32_t p : t.alu_diag)
         tail.diag_pos.push_back(pos[p]);
+      for (int32_t p : t.alu_lower)
+        tail.lower_pos.push_back(p >= 0 ? pos[p] : -1);
+      for (int32_t p : t.alu_upper)
+        tail.upper_pos.push_back(pos[p]);
       const uint32_t zero = static_cast<uint32_t>(tail.nnz), zero_x = static_cast<uint32_t>(n);
       // LU: the products with pivots before the block; elements outside the block complete,
       // with their division, the block's without one.  Sums in runs of the terms that a
@@ -1043,6 +1047,7 @@ namespace micm_hip
         {
           SubstitutionRow r;
           r.out = static_cast<uint32_t>(i);
+          r.diag = i < first ? kUnitDivisor : kNoDivisor;
           for (int32_t q = t.fwd_offsets[i]; q < t.fwd_offsets[i + 1] && t.fwd_col[q] < first; ++q)
             r.terms.push_back(static_cast<uint32_t>(pos[t.alu_lower[t.fwd_mat[q]]]) |
                               (static_cast<uint32_t>(t.fwd_col[q]) << 16));

@@ -120,7 +120,8 @@ namespace micm_hip
     int32_t head = 0;  // elements outside the block
     int32_t nnz = 0;   // positions without the zero
     std::vector<int32_t> jac_pos, diag_pos;  // of a Jacobian element, of a species' diagonal
-    std::vector<uint64_t> row_mask;          // per block row: its columns in the fill pattern
+    std::vector<int32_t> lower_pos, upper_pos;  // of an element of L (-1: the unit diagonal), of U
+    std::vector<uint64_t> row_mask;             // per block row: its columns in the fill pattern
     LevelSchedule lu;                        // products with pivots before the block
     // the forward substitution's levels, empty ones up to fwd_padded, the back substitution's
     // up to bwd_end, empty ones, the first two levels again; both padded counts are multiples

@@ -526,15 +526,17 @@ namespace
     }
   }
 
+  // One thread per (diagonal element, cell): a thread per cell walking the diagonal leaves all
+  // but n_cells lanes idle (210 species, 4,096 cells: 64 us).
   __global__ void __launch_bounds__(kBlock) k_alpha_minus_jacobian(DevMech m, int64_t n_cells, double* __restrict__ jac,
                                                                    double alpha)
   {
-    const int64_t c = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (c >= n_cells)
+    const int64_t f = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    const int64_t q = f / kGroup, g = q / m.n_species;
+    const int l = static_cast<int>(f % kGroup);
+    if (g * kGroup + l >= n_cells)
       return;
-    Lane J = lane_view(jac, c / kGroup, m.nnz_jac, c % kGroup);
-    for (int i = 0; i < m.n_species; ++i)
-      J[m.jac_diag[i]] += alpha * 1.0;
+    lane_view(jac, static_cast<size_t>(g), m.nnz_jac, l)[m.jac_diag[q % m.n_species]] += alpha * 1.0;
   }
 
   __global__ void __launch_bounds__(kBlock) k_lu_decompose(DevMech m, int64_t n_cells, const double* __restrict__ jac,
@@ -561,21 +563,57 @@ namespace
                     lane_view(const_cast<double*>(upper), g, m.nnz_upper, l), lane_view(x, g, m.n_species, l));
   }
 
+  // The per-cell norm (path.hpp, error_sum): a workgroup takes kErrorCells cells of a group, its
+  // threads form the squares of kErrorSpecies species at a time into LDS, and one lane per cell
+  // adds them in species order.  A thread per cell forming and adding its own terms leaves the
+  // chip idle below 100,000 cells (210 species, 4,096 cells: 154 us).
+  constexpr int kErrorCells = 16;
+  constexpr int kErrorSpecies = 64;
+
   __global__ void __launch_bounds__(kBlock) k_normalized_error(int n_species, int64_t n_cells, const double* __restrict__ y,
                                                                const double* __restrict__ ynew,
                                                                const double* __restrict__ yerr,
                                                                const double* __restrict__ atol, double rtol,
                                                                double* __restrict__ err)
   {
-    const int64_t c = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (c >= n_cells)
+    __shared__ double terms[2][kErrorSpecies * kErrorCells];
+    constexpr int kTiles = kGroup / kErrorCells;
+    const size_t g = blockIdx.x / kTiles;
+    const int q0 = static_cast<int>(blockIdx.x % kTiles) * kErrorCells;
+    const int cc = threadIdx.x % kErrorCells, sp = threadIdx.x / kErrorCells;
+    const size_t base = g * static_cast<size_t>(n_species) * kGroup + q0 + cc;
+    const int64_t cell = static_cast<int64_t>(g) * kGroup + q0 + cc;
+    if (static_cast<int64_t>(g) * kGroup + q0 >= n_cells)
       return;
-    const size_t g = c / kGroup;
-    const int l = c % kGroup;
-    const double s = error_sum(n_species, lane_view(const_cast<double*>(y), g, n_species, l),
-                               lane_view(const_cast<double*>(ynew), g, n_species, l),
-                               lane_view(const_cast<double*>(yerr), g, n_species, l), atol, rtol);
-    err[c] = smax(sqrt(s / static_cast<double>(n_species > 0 ? n_species : 1)), 1.0e-10);
+    double acc = 0.0;
+    int buffer = 0;
+    for (int i0 = 0; i0 < n_species; i0 += kErrorSpecies, buffer ^= 1)
+    {
+#pragma unroll
+      for (int k = 0; k < kErrorSpecies * kErrorCells / kBlock; ++k)
+      {
+        const int i = i0 + sp + k * (kBlock / kErrorCells);
+        double t = 0.0;  // past the last species: adds nothing to a sum that is never -0
+        if (i < n_species && cell < n_cells)
+        {
+          const size_t f = base + static_cast<size_t>(i) * kGroup;
+          const double a = fabs(y[f]), b = fabs(ynew[f]);
+          const double ymax = a > b ? a : b;
+          const double q = yerr[f] / (atol[i] + rtol * ymax);
+          t = q * q;
+        }
+        terms[buffer][(sp + k * (kBlock / kErrorCells)) * kErrorCells + cc] = t;
+      }
+      __syncthreads();
+      if (threadIdx.x < kErrorCells)
+      {
+#pragma unroll 16
+        for (int i = 0; i < kErrorSpecies; ++i)
+          acc += terms[buffer][i * kErrorCells + cc];
+      }
+    }
+    if (threadIdx.x < kErrorCells && cell < n_cells)
+      err[cell] = smax(sqrt(acc / static_cast<double>(n_species > 0 ? n_species : 1)), 1.0e-10);
   }
 
   // ------------------------------------------------------------------ solver state
@@ -1824,7 +1862,8 @@ namespace
 
   size_t tail_bytes(const TailTables& t)
   {
-    return padded_bytes(t.jac_pos) + padded_bytes(t.diag_pos) + padded_bytes(t.row_mask) + level_bytes(t.lu) +
+    return padded_bytes(t.jac_pos) + padded_bytes(t.diag_pos) + padded_bytes(t.lower_pos) +
+           padded_bytes(t.upper_pos) + padded_bytes(t.row_mask) + level_bytes(t.lu) +
            padded_bytes(t.rows.heads) + padded_bytes(t.rows.terms);
   }
 
@@ -2112,6 +2151,8 @@ namespace
       tl.nnz = t.tail.nnz;
       upload(m->blob, off, t.tail.jac_pos, tl.jac_pos, staging);
       upload(m->blob, off, t.tail.diag_pos, tl.diag_pos, staging);
+      upload(m->blob, off, t.tail.lower_pos, tl.lower_pos, staging);
+      upload(m->blob, off, t.tail.upper_pos, tl.upper_pos, staging);
       upload(m->blob, off, t.tail.row_mask, tl.row_mask, staging);
       upload_levels(m->blob, off, t.tail.lu, tl.lu, staging);
       upload_rows(m->blob, off, t.tail.rows, tl.rows, staging);
@@ -2204,6 +2245,21 @@ namespace
       if (2 * doubles_per_cell * tc * sizeof(double) <= limit)
         return tc;
     return doubles_per_cell * sizeof(double) <= limit ? 1 : 0;
+  }
+
+  // Whether the single-phase LU and substitution take the kernels with the factor's dense block
+  // (one cell per workgroup) rather than the tiled ones: for factors of at least kTailFactor
+  // entries, and for smaller ones below kTailCells cells, where a tile of many cells leaves most
+  // CUs idle.  LU, us, block / tiled: 210/560 (8,548 entries) 77 / 214 for 64 cells and 545 /
+  // 1,665 for 4,096; TS1 (2,381) 135 / 166, 60/200 (1,304) 98 / 118 for 4,096 and 433 / 440 for
+  // 20,000; 50 species (989) 32 / 55 for 1,000 and 374 / 359 for 20,000; 24 species (238) 19 / 23
+  // for 1,000 and 51 / 24 for 4,096.
+  constexpr int kTailFactor = 1200;
+  constexpr int64_t kTailCells = 768;
+
+  bool phases_with_tail(const micm_hip_mechanism* m, int64_t n_cells, size_t lds)
+  {
+    return m->tail.size > 0 && (m->coop.nnz_alu >= kTailFactor || n_cells <= kTailCells) && lds <= lds_limit();
   }
 
   // Cells per workgroup of the tiled forcing / Jacobian kernels: the largest power of two
@@ -2938,7 +2994,12 @@ extern "C"
     KERNEL_PRELUDE();
     if (!jac)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
-    hipLaunchKernelGGL(k_alpha_minus_jacobian, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, m->dev, n_cells, jac, alpha);
+    if (m->dev.n_species == 0)
+      return MICM_HIP_OK;
+    hipLaunchKernelGGL(k_alpha_minus_jacobian,
+                       dim3(static_cast<unsigned>((n_groups_of(n_cells) * static_cast<int64_t>(m->dev.n_species) * kGroup +
+                                                   kBlock - 1) / kBlock)),
+                       dim3(kBlock), 0, st, m->dev, n_cells, jac, alpha);
     HIP_TRY(hipGetLastError());
     return MICM_HIP_OK;
   }
@@ -2950,7 +3011,11 @@ extern "C"
     if (!jac || !lower || !upper)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
     const int tc = tile_cells(m, static_cast<size_t>(m->coop.nnz_alu));
-    if (tc > 0)
+    if (phases_with_tail(m, n_cells, tail_factor_lds(m->tail)))
+    {
+      HIP_TRY(lu_decompose_tail(m->dev, m->tail, n_cells, tiled_blocks(1, n_cells), jac, lower, upper, st));
+    }
+    else if (tc > 0)
     {
       const size_t lds = static_cast<size_t>(m->coop.nnz_alu) * tc * sizeof(double);
       const unsigned blocks = tiled_blocks(tc, n_cells);
@@ -2958,8 +3023,7 @@ extern "C"
       {
         case 16: LAUNCH_TILED(k_lu_decompose_tiled<16>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
         case 8: LAUNCH_TILED(k_lu_decompose_tiled<8>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
-        case 4: LAUNCH_TILED(k_lu_decompose_tiled<4>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
-        case 2: LAUNCH_TILED(k_lu_decompose_tiled<2>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
+        // (tiles of two and four cells are those of factors that the block takes)
         default: LAUNCH_TILED(k_lu_decompose_tiled<1>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
       }
     }
@@ -2978,7 +3042,11 @@ extern "C"
     if (!lower || !upper || !x)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
     const int tc = tile_cells(m, static_cast<size_t>(m->coop.nnz_alu) + 2 * static_cast<size_t>(m->dev.n_species));
-    if (tc > 0)
+    if (phases_with_tail(m, n_cells, tail_solve_lds(m->dev, m->tail)))
+    {
+      HIP_TRY(lu_solve_tail(m->dev, m->tail, n_cells, tiled_blocks(1, n_cells), lower, upper, x, st));
+    }
+    else if (tc > 0)
     {
       size_t lds = (static_cast<size_t>(m->coop.nnz_alu) + 2 * static_cast<size_t>(m->dev.n_species)) * tc *
                    sizeof(double);
@@ -3025,7 +3093,8 @@ extern "C"
     KERNEL_PRELUDE();
     if (!y || !ynew || !yerr || !atol || !error)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
-    hipLaunchKernelGGL(k_normalized_error, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, m->dev.n_species, n_cells, y,
+    hipLaunchKernelGGL(k_normalized_error, dim3(static_cast<unsigned>(n_groups_of(n_cells) * (kGroup / kErrorCells))),
+                       dim3(kBlock), 0, st, m->dev.n_species, n_cells, y,
                        ynew, yerr, atol, rtol, error);
     HIP_TRY(hipGetLastError());
     return MICM_HIP_OK;

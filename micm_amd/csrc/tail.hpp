@@ -18,7 +18,7 @@
 // right-hand sides and every difference of unlike values round to +0) -- unless u is
 // infinite or NaN.  Every result of the block is therefore checked to be finite, and a cell
 // with one that is not is done again with each product tested against the fill pattern
-// (tail_factor_masked, tail_masked), which is exact for every operand.
+// (the masked forms), which is exact for every operand.
 #pragma once
 
 #include "coop.hpp"
@@ -74,8 +74,9 @@ namespace micm_hip
   // go through LDS (two buffers, so one barrier a pivot); every four lanes divide one
   // column value each and pass the quotients on by DPP, and each thread updates its
   // elements below and right of the pivot.  Elements that are final already see a zero
-  // factor.
-  template<int PA>
+  // factor, which leaves them as they are but for the sign of a zero in L; that matters to no
+  // product, and with ZEROS (L is a result) they are kept by a select instead.
+  template<int PA, bool ZEROS>
   __device__ __forceinline__ void tail_pivots(double (&e)[4][4], int ti, int tj, double* buf)
   {
 #pragma unroll 1
@@ -124,7 +125,17 @@ namespace micm_hip
         const double la = a == PA ? l_pa : l[a];
 #pragma unroll
         for (int b = PA; b < 4; ++b)
-          e[a][b] -= la * (b == PA ? u_pa : u[b]);
+        {
+          if (ZEROS && b == PA)
+          {
+            const double v = e[a][b] - la * u[b];
+            e[a][b] = tj > kk ? v : e[a][b];
+          }
+          else
+          {
+            e[a][b] -= la * (b == PA ? u_pa : u[b]);
+          }
+        }
         if (tj == kk && (a > PA || ti > kk))
           e[a][PA] = l[a];
       }
@@ -134,11 +145,12 @@ namespace micm_hip
   // The block's own factorisation in place (A: the factor, its head and the block's sums
   // over the head's pivots final), 256 threads.  False (on every thread), the block left as
   // it is, when an element is not finite.  buf: kTailBuffer doubles; flags: one int per
-  // wave.  Ends with a barrier.
+  // wave.  ZEROS: tail_pivots.  Ends with a barrier.
   //
   // One pivot costs an LDS round trip with a barrier (140 clocks), a division (53) and ten
   // clocks for each of a thread's elements, whatever the fill; the level schedule of the
   // same rows takes two levels a pivot at 1,400 each.
+  template<bool ZEROS>
   __device__ inline bool tail_factor(const DevTail& t, double* A, double* buf, int* flags)
   {
     const int tid = threadIdx.x;
@@ -157,12 +169,12 @@ namespace micm_hip
           e[a][b] = base[kTailBlock * (stride * (a - p0) + (b - p0))];
       }
     if (p0 <= 0)
-      tail_pivots<0>(e, ti, tj, buf);
+      tail_pivots<0, ZEROS>(e, ti, tj, buf);
     if (p0 <= 1)
-      tail_pivots<1>(e, ti, tj, buf);
+      tail_pivots<1, ZEROS>(e, ti, tj, buf);
     if (p0 <= 2)
-      tail_pivots<2>(e, ti, tj, buf);
-    tail_pivots<3>(e, ti, tj, buf);
+      tail_pivots<2, ZEROS>(e, ti, tj, buf);
+    tail_pivots<3, ZEROS>(e, ti, tj, buf);
     bool finite = true;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -238,19 +250,31 @@ namespace micm_hip
     return RowsAhead{ row_record(r, 0), row_record(r, 1) };
   }
 
+  // What a level's tasks divide by: nothing, U[i][i], or L[i][i] (a lower factor whose diagonal
+  // is not 1, as the single-phase substitution takes it).
+  enum class Divide
+  {
+    kNone,
+    kUpper,
+    kLower
+  };
+
   // One level of sixteen tasks, one to a DPP row: lane k forms the products 16 g + k, the
-  // row subtracts them in order; DIV: and divides (by one where a task has no divisor).  A
+  // row subtracts them in order and divides (by one where a task has no divisor).  A
   // wavefront skips the groups that none of its tasks has (its lanes' words are all `pad`).
   // Every lane of a row writes the row's result: an exec mask around the write costs 70 of a
   // level's 570 clocks.
-  template<bool DIV>
-  __device__ __forceinline__ void tail_level(const RowRecord& rec, uint32_t pad, const double* A, double* x, double m1)
+  template<Divide DIV>
+  __device__ __forceinline__ void tail_level(const RowRecord& rec, uint32_t pad, const double* A, double* x, double m1,
+                                             const double* ld)
   {
     const uint32_t o = rec.head & 0xffffu, d = rec.head >> 16;
     const uint32_t w[4] = { rec.terms.x, rec.terms.y, rec.terms.z, rec.terms.w };
     double v = x[o], dv = 1.0;
-    if constexpr (DIV)
+    if constexpr (DIV == Divide::kUpper)
       dv = A[d < kUnitDivisor ? d : 0];
+    if constexpr (DIV == Divide::kLower)
+      dv = ld[d == kUnitDivisor ? o : 0];
     auto product = [&](int g) { return A[w[g] & 0xffffu] * x[w[g] >> 16]; };
     const double p0 = product(0);
     if (!__any(w[1] != pad))
@@ -271,9 +295,9 @@ namespace micm_hip
       v = ordered_sub16<0>(v, p2, m1);
       v = ordered_sub16<0>(v, p3, m1);
     }
-    if constexpr (DIV)
+    if constexpr (DIV != Divide::kNone)
     {
-      v = v / (d < kUnitDivisor ? dv : 1.0);
+      v = v / ((DIV == Divide::kUpper ? d < kUnitDivisor : d == kUnitDivisor) ? dv : 1.0);
       asm("" : "+v"(v));
     }
     x[o] = v;
@@ -404,27 +428,52 @@ namespace micm_hip
     return ok;
   }
 
-  // tail_forward (DIR 0) or tail_backward (1) with every product tested against the fill
-  // pattern, row by row (for values that are not finite; small code, not speed).
-  template<int DIR>
-  __device__ inline void tail_masked(const DevTail& t, const double* block, double* xt)
+  // tail_forward with every product tested against the fill pattern (for values that are not
+  // finite, or a right-hand side with -0; loops, about a third of the speed).  ld: divide by
+  // the rows' L[i][i] (null: they are 1).
+  __device__ inline void tail_forward_masked(const DevTail& t, const double* block, double* xt, const double* ld)
   {
-    const int d = t.size, stride = d + 1;
-    if ((threadIdx.x & (kWave - 1)) == 0)
+    const int lane = threadIdx.x & (kWave - 1);
+    const int d = t.size, r = lane < d ? lane : 0;
+    const double* row = block + r * (d + 1);
+    const uint64_t rm = t.row_mask[r];
+    double v = xt[r];
+#pragma unroll 1
+    for (int c = 0; c < d; ++c)
     {
-#pragma unroll 1
-      for (int q = 0; q < d; ++q)
+      double xc = readlane_f64(v, static_cast<uint32_t>(c));
+      if (ld)
       {
-        const int i = DIR == 0 ? q : d - 1 - q;
-        double v = xt[i];
-#pragma unroll 1
-        for (int j = DIR == 0 ? 0 : i + 1; j < (DIR == 0 ? i : d); ++j)
-          if ((t.row_mask[i] >> j) & 1u)
-            v -= block[i * stride + j] * xt[j];
-        xt[i] = DIR == 0 ? v : v / block[i * stride + i];
+        xc = xc / ld[c];
+        v = r == c ? xc : v;
       }
+      const double nv = v - row[c] * xc;
+      v = r > c && ((rm >> c) & 1u) ? nv : v;
     }
-    coop_sync<kWave>();
+    if (lane < d)
+      xt[lane] = v;
+  }
+
+  // tail_backward with every product tested against the fill pattern.
+  __device__ inline void tail_backward_masked(const DevTail& t, const double* block, double* xt, double m1)
+  {
+    const int l16 = threadIdx.x & 15;
+    const int d = t.size;
+#pragma unroll 1
+    for (int i = d - 1; i >= 0; --i)
+    {
+      const double* row = block + i * (d + 1);
+      const uint64_t rm = const_load(t.row_mask, i);
+      double v = xt[i];
+#pragma unroll 1
+      for (int j = l16; j < d; j += kTailBlock)
+      {
+        const double p = row[j] * xt[j];
+        v = ordered_sub16<0>(v, j > i && ((rm >> j) & 1u) ? p : 0.0, m1);
+      }
+      xt[i] = v / row[i];
+      coop_sync<kWave>();
+    }
   }
 
   // Both triangles of the block by one wavefront.
@@ -433,45 +482,49 @@ namespace micm_hip
                                                   double m1)
   {
     if (masked || !tail_forward<D>(block, xt))
-      tail_masked<0>(t, block, xt);
+      tail_forward_masked(t, block, xt, nullptr);
     coop_sync<kWave>();
     if (masked || !tail_backward<D>(block, xt, m1))
-      tail_masked<1>(t, block, xt);
+      tail_backward_masked(t, block, xt, m1);
+  }
+
+  // Levels [begin, end) of the rows' list, the record of level l + 2 read while level l runs.
+  // Three records rotate, unrolled by three so that none moves; level counts are padded to
+  // multiples of three, so that the next levels start with the same record.
+  template<Divide DIV>
+  __device__ __forceinline__ void tail_levels(const DevTail& t, int begin, int end, const double* A, double* x, double m1,
+                                              const double* ld, RowsAhead& ahead)
+  {
+    const DevRows& r = t.rows;
+    const uint32_t pad = static_cast<uint32_t>(t.nnz) | (static_cast<uint32_t>(t.first + t.size) << 16);
+    RowRecord spare;
+    auto step = [&](int l, const RowRecord& cur, RowRecord& next) {
+      next = row_record(r, l + 2);
+      if (l < end)
+      {
+        settle(cur.terms);
+        settle(uint4{ cur.head, 0u, 0u, 0u });
+        tail_level<DIV>(cur, pad, A, x, m1, ld);
+      }
+    };
+#pragma unroll 1
+    for (int l = begin; l < end; l += kRowPadding)
+    {
+      step(l, ahead.r0, spare);
+      step(l + 1, ahead.r1, ahead.r0);
+      step(l + 2, spare, ahead.r1);
+    }
   }
 
   // x <- U^-1 L^-1 x (x[n] = 0 behind it); masked: the factor holds values that are not
-  // finite.  The record of level l + 2 is read while level l runs; the levels before and
-  // after the block are one list that ends in its first two levels again, whose records the
-  // next solve starts with (`ahead`).  Three records rotate, unrolled by three so that none
-  // moves; both passes' level counts are padded to multiples of three, so that each pass and
-  // the next solve start with the same record.  Ends with a barrier.
+  // finite, or x holds a -0.  The levels before and after the block are one list that ends in
+  // its first two levels again, whose records the next solve starts with (`ahead`).  Ends with
+  // a barrier.
   __device__ inline void tail_solve(const DevTail& t, const double* A, double* x, bool masked, RowsAhead& ahead)
   {
     double m1 = -1.0;
     asm("" : "+v"(m1));
-    const DevRows& r = t.rows;
-    const uint32_t pad = static_cast<uint32_t>(t.nnz) | (static_cast<uint32_t>(t.first + t.size) << 16);
-    RowRecord spare;
-    auto levels = [&](auto div, int begin, int end) {
-      constexpr bool DIV = decltype(div)::value;
-      auto step = [&](int l, const RowRecord& cur, RowRecord& next) {
-        next = row_record(r, l + 2);
-        if (l < end)
-        {
-          settle(cur.terms);
-          settle(uint4{ cur.head, 0u, 0u, 0u });
-          tail_level<DIV>(cur, pad, A, x, m1);
-        }
-      };
-#pragma unroll 1
-      for (int l = begin; l < end; l += kRowPadding)
-      {
-        step(l, ahead.r0, spare);
-        step(l + 1, ahead.r1, ahead.r0);
-        step(l + 2, spare, ahead.r1);
-      }
-    };
-    levels(std::false_type{}, 0, t.fwd_levels);
+    tail_levels<Divide::kNone>(t, 0, t.fwd_levels, A, x, m1, nullptr, ahead);
     if (threadIdx.x < kWave)
     {
       const double* b = A + t.head;
@@ -485,6 +538,23 @@ namespace micm_hip
       }
     }
     lds_barrier<kTailThreads>();
-    levels(std::true_type{}, t.fwd_padded, t.bwd_end);
+    tail_levels<Divide::kUpper>(t, t.fwd_padded, t.bwd_end, A, x, m1, nullptr, ahead);
+  }
+
+  // The same for a lower factor with the diagonal ld (rows without terms already divided).
+  __device__ inline void tail_solve_lower_diagonal(const DevTail& t, const double* A, double* x, const double* ld,
+                                                   RowsAhead& ahead)
+  {
+    double m1 = -1.0;
+    asm("" : "+v"(m1));
+    tail_levels<Divide::kLower>(t, 0, t.fwd_levels, A, x, m1, ld, ahead);
+    if (threadIdx.x < kWave)
+    {
+      tail_forward_masked(t, A + t.head, x + t.first, ld + t.first);
+      coop_sync<kWave>();
+      tail_backward_masked(t, A + t.head, x + t.first, m1);
+    }
+    lds_barrier<kTailThreads>();
+    tail_levels<Divide::kUpper>(t, t.fwd_padded, t.bwd_end, A, x, m1, nullptr, ahead);
   }
 }  // namespace micm_hip
