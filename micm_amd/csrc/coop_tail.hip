@@ -9,6 +9,13 @@ namespace micm_hip
 {
 namespace
 {
+  // a value that all lanes hold, as one in scalar registers
+  __device__ __forceinline__ double uniform(double v)
+  {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+  }
+
   // LDS holds what other threads read: the factor (head, block, zero), y, one vector x (stage
   // inputs, right-hand sides and solutions, x[n] = 0) and a scratch area shared in time by
   // the reaction rates, the Jacobian's partial products, the block's pivots and the error
@@ -16,15 +23,14 @@ namespace
   // in registers; rate constants are read from a per-workgroup copy in global memory.
   //
   // Bound by the dependency chain of one attempt.  An attempt of the slowest cell, two waves
-  // per SIMD, against the level-scheduled compact layout it replaced: 210/560 366 -> 131 us,
-  // 60/200 110 -> 46 us, TS1 190 -> 71 us.
+  // per SIMD, against the level-scheduled compact layout it replaced: 210/560 366 -> 130 us,
+  // 60/200 110 -> 45 us, TS1 190 -> 70 us.
   template<int MINW, bool RECORD>
   __global__ void __launch_bounds__(kTailThreads, MINW)
       k_coop_tail(DevMech m, DevCoop c, DevTail t, DevParams p, int64_t n_fixed, const int32_t* __restrict__ list,
                   const int* list_count, int* next, const CellControl* resume, double* __restrict__ y_state,
-                  double* __restrict__ k_state, const double* __restrict__ atol, int32_t* status_out,
-                  int64_t* stats_out, double* final_time_out, const double* __restrict__ cond_state,
-                  const double* __restrict__ custom_state, double* __restrict__ k_wg, Tape tape)
+                  const double* __restrict__ k_state, const double* __restrict__ atol, int32_t* status_out,
+                  int64_t* stats_out, double* final_time_out, double* __restrict__ k_wg, Tape tape)
   {
     constexpr int NT = kTailThreads;
     extern __shared__ double lds[];
@@ -53,7 +59,7 @@ namespace
       if (tid == 0)
         s_idx = atomicAdd(next, 1);
       coop_sync<NT>();
-      const int64_t idx = s_idx;
+      const int64_t idx = __builtin_amdgcn_readfirstlane(s_idx);
       coop_sync<NT>();
       if (idx >= count)
         return;
@@ -62,29 +68,13 @@ namespace
       const int cl = cell % kGroup;
       {
         Lane ys = lane_view(y_state, g, n, cl);
-        Lane ks = lane_view(k_state, g, m.n_reactions, cl);
+        Lane ks = lane_view(const_cast<double*>(k_state), g, m.n_reactions, cl);
         if (mine)
           L.y[tid] = ys[tid];
         if (tid == 0)
           x[n] = 0.0;
-        if (cond_state)
-        {
-          // UpdateStateParameters fused into the launch
-          Lane cd = lane_view(const_cast<double*>(cond_state), g, 3, cl);
-          Lane cu = lane_view(const_cast<double*>(custom_state), g, m.n_custom, cl);
-          const double T = cd[0], P = cd[1], rho = cd[2];
-          for (int r = tid; r < m.n_reactions; r += NT)
-          {
-            const double kr = rate_constant(m, r, T, P, rho, cu);
-            L.k[r] = kr;
-            ks[r] = kr;
-          }
-        }
-        else
-        {
-          for (int r = tid; r < m.n_reactions; r += NT)
-            L.k[r] = ks[r];
-        }
+        for (int r = tid; r < m.n_reactions; r += NT)
+          L.k[r] = ks[r];
       }
       CellControl cc;
       if (resume)
@@ -138,7 +128,7 @@ namespace
         }
         coop_sync<NT>();
         coop_levels_piped<NT, true>(t.lu, t.lu.terms, L.alu, L.alu, L.alu);
-        const bool masked = !tail_factor<false>(t, L.alu, L.scratch, s_flags);
+        const bool masked = __builtin_amdgcn_readfirstlane(!tail_factor<false>(t, L.alu, L.scratch, s_flags));
         if (masked)
           tail_factor_masked(t, L.alu);
         cc.stats[MICM_HIP_STAT_DECOMPOSITIONS] += 1;
@@ -205,6 +195,7 @@ namespace
             q = qn;
           }
         }
+        acc = uniform(acc);
         const double error = smax(sqrt(acc / static_cast<double>(n > 0 ? n : 1)), 1.0e-10);
         const double h_used = cc.H;
         if (control_update(p, cc, error))
@@ -394,7 +385,7 @@ namespace
       return e;
     hipLaunchKernelGGL((k_coop_tail<MINW, RECORD>), dim3(blocks), dim3(kTailThreads), lds, stream, a.m, a.c, a.t, a.p,
                        a.n_fixed, a.list, a.list_count, a.next, a.resume, a.y, a.k, a.atol, a.status, a.stats,
-                       a.final_time, a.cond, a.custom, a.k_rows, a.tape);
+                       a.final_time, a.k_rows, a.tape);
     return hipGetLastError();
   }
 }  // namespace

@@ -39,14 +39,14 @@ namespace micm_hip
     const int* list_count;
     int* next;  // queue counter, zeroed before the launch
     const CellControl* resume;
-    double *y, *k;
+    double* y;
+    const double* k;
     const double* atol;
     int32_t* status;
     int64_t* stats;
     double* final_time;
-    const double *cond, *custom;  // null: the rate constants are the state's
-    double* k_rows;               // gridDim.x rows of n_reactions
-    Tape tape;                    // records null: not recorded
+    double* k_rows;  // gridDim.x rows of n_reactions
+    Tape tape;       // records null: not recorded
   };
 
   // Workgroups per CU of the build for min_waves waves per SIMD (3 or 2), 0 where it does not fit.

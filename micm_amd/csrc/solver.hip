@@ -2567,9 +2567,15 @@ namespace
     const CoopTailArgs a{ m->dev,          m->coop,  m->tail,   p,        n_fixed,
                           list,            count,    ext ? s->ext_next : s->coop_next,
                           resume,          s->y,     s->k,      s->atol,  s->status,
-                          s->stats,        s->final_time,       update_rates ? s->cond : nullptr,
-                          update_rates ? s->custom : nullptr,   ext ? s->ext_k : s->coop_k,
-                          s->recording };
+                          s->stats,        s->final_time,       ext ? s->ext_k : s->coop_k, s->recording };
+    // The rate constants from a launch of their own: held ready in the Solve's kernel, the rate
+    // laws' constants and temporaries cost it 140 spilled registers and 30 KB of code.
+    if (update_rates)
+    {
+      hipLaunchKernelGGL(k_rate_constants, rate_grid(s->n_cells, m->dev.n_reactions), dim3(kBlock), 0, st, m->dev,
+                         s->n_cells, s->cond, s->custom, s->k);
+      HIP_TRY(hipGetLastError());
+    }
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, a.next);
     HIP_TRY(coop_tail_launch(plan.min_waves, static_cast<unsigned>(blocks), plan.lds, st, a));
     return MICM_HIP_OK;
