@@ -23,8 +23,8 @@ namespace
   // in registers; rate constants are read from a per-workgroup copy in global memory.
   //
   // Bound by the dependency chain of one attempt.  An attempt of the slowest cell, two waves
-  // per SIMD, against the level-scheduled compact layout it replaced: 210/560 366 -> 130 us,
-  // 60/200 110 -> 45 us, TS1 190 -> 70 us.
+  // per SIMD, against the level-scheduled compact layout it replaced: 210/560 366 -> 128 us,
+  // 60/200 110 -> 45 us, TS1 190 -> 69 us.
   template<int MINW, bool RECORD>
   __global__ void __launch_bounds__(kTailThreads, MINW)
       k_coop_tail(DevMech m, DevCoop c, DevTail t, DevParams p, int64_t n_fixed, const int32_t* __restrict__ list,

@@ -30,6 +30,14 @@ namespace micm_hip
 {
   static_assert(kTailBuffer == 4 * kTailMax && kTailBlock == 16, "as coop_tail.hpp has them");
 
+  // What depends on v is formed here, each time: kept across a Solve's loops, the straight-line
+  // code's lane comparisons and addresses spill 46 vector and 350 scalar registers of the
+  // three-wave build (an attempt: 60/200 46.5 -> 44.5 us, 20/50 27.5 -> 25.3, 210/560 130 -> 127.6).
+  __device__ __forceinline__ void here(int& v)
+  {
+    asm volatile("" : "+v"(v));
+  }
+
   // v - p[K0] - ... - p[15], subtracted in that order, p[k] being lane k's p of the reader's
   // DPP row of sixteen lanes.  One instruction a product: the multiply by m1 = -1 is exact,
   // so the fused form rounds once, as the subtraction does.  5.4 clocks a product on
@@ -153,7 +161,8 @@ namespace micm_hip
   template<bool ZEROS>
   __device__ inline bool tail_factor(const DevTail& t, double* A, double* buf, int* flags)
   {
-    const int tid = threadIdx.x;
+    int tid = threadIdx.x;
+    here(tid);
     const int ti = tid >> 4, tj = tid & 15;
     const int p0 = 4 - t.size / kTailBlock;
     const int stride = t.size + 1;
@@ -316,7 +325,8 @@ namespace micm_hip
                                             double m1)
   {
     constexpr int Q = D / kTailBlock, S = D + 1;
-    const int l16 = threadIdx.x & 15;
+    int l16 = threadIdx.x & 15;
+    here(l16);
     const double* lane = block + l16;
     double u[Q], diag, z;
     constexpr int last = kTailBlock * G + kTailBlock - 1;
@@ -367,7 +377,8 @@ namespace micm_hip
   {
     constexpr int S = D + 1;
     const int lane = threadIdx.x & (kWave - 1);
-    const int r = lane < D ? lane : 0;  // lanes past the block hold row 0, which no column changes
+    int r = lane < D ? lane : 0;  // lanes past the block hold row 0, which no column changes
+    here(r);
     double v = xt[r];
     const double* row = block + r * S;
     double a[8];
