@@ -28,7 +28,8 @@
 // One workgroup integrates one cell: each record is replayed from its checkpoint (the
 // Jacobian, the factorisation and the stage vectors are recomputed with the cooperative
 // form's level schedules, so the stage vectors are those of the recorded step), then the
-// stages are reversed.  Nothing per step is stored but the checkpoint.
+// stages are reversed.  Nothing per step is stored but the checkpoint.  k_adjoint below is for
+// mechanisms outside the range of adjoint_tail.hip's kernel, which has the factor's dense block.
 #pragma once
 
 #include "coop.hpp"

@@ -253,9 +253,10 @@ namespace micm_hip
                : 0.0;
   }
 
-  // L.jac = -J(y); with TO_ALU the elements go straight to their factor positions
-  template<int NT, bool TO_ALU = false>
-  __device__ inline void coop_jacobian(const DevMech& m, const DevCoop& c, const CoopLds& L)
+  // store(t, d_t(yv), term_pack[t]) for every Jacobian term t
+  template<int NT, class Store>
+  __device__ __forceinline__ void coop_term_products(const DevMech& m, const DevCoop& c, const CoopLds& L, const double* yv,
+                                                     Store store)
   {
     const int tid = threadIdx.x;
     const int nt = c.n_terms;
@@ -273,8 +274,8 @@ namespace micm_hip
       for (int j = 0; j < 4; ++j)
       {
         kk[j] = L.k[pk[j] & 0xffffu];
-        y0[j] = L.y[(pk[j] >> 16) & 0xffffu];
-        y1[j] = L.y[(pk[j] >> 32) & 0xffffu];
+        y0[j] = yv[(pk[j] >> 16) & 0xffffu];
+        y1[j] = yv[(pk[j] >> 32) & 0xffffu];
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -286,16 +287,24 @@ namespace micm_hip
           if ((pk[j] >> 48) == 0xffffu)
           {
             for (int i = m.term_dep_offsets[t]; i < m.term_dep_offsets[t + 1]; ++i)
-              d *= L.y[m.term_dep_ids[i]];
+              d *= yv[m.term_dep_ids[i]];
           }
           else
           {
             d = packed_product(d, pk[j], y0[j], y1[j], 0.0);
           }
-          L.jterm[t] = d;
+          store(t, d, pk[j]);
         }
       }
     }
+  }
+
+  // L.jac = -J(y); with TO_ALU the elements go straight to their factor positions
+  template<int NT, bool TO_ALU = false>
+  __device__ inline void coop_jacobian(const DevMech& m, const DevCoop& c, const CoopLds& L)
+  {
+    const int tid = threadIdx.x;
+    coop_term_products<NT>(m, c, L, L.y, [&](int t, double d, uint64_t) { L.jterm[t] = d; });
     coop_sync<NT>();
     for (int e = tid; e < m.nnz_jac; e += NT)
     {

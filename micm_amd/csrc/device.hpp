@@ -110,6 +110,9 @@ namespace micm_hip
     // substitution's (up to bwd_end, padded to rows.n_levels), the first two levels again
     DevRows rows;
     int32_t fwd_levels, fwd_padded, bwd_end;
+    // the same of the transposed substitutions
+    DevRows t_rows;
+    int32_t t_fwd_levels, t_fwd_padded, t_bwd_end;
   };
 
   // Tables of the cooperative (one workgroup per cell) form; see MechanismTables.

@@ -1039,6 +1039,34 @@ namespace micm_hip
         const std::vector<int32_t> capped = cap_levels(tasks, order, 256);
         tail.lu = pack_levels(tasks, &capped, zero * 0x10001u);
       }
+      // A forward and a back substitution's levels as one list (TailTables::rows).
+      auto join_rows = [&](RowLevels rows, const RowLevels& back, int32_t& fwd_levels, int32_t& fwd_padded,
+                           int32_t& bwd_end) {
+        // empty levels up to a multiple of kRowPadding (at least `least` in all, for the read
+        // ahead)
+        auto pad_levels = [&](int32_t least) {
+          while (rows.n_levels() % kRowPadding != 0 || rows.n_levels() < least)
+          {
+            rows.heads.insert(rows.heads.end(), kRowSlots, zero_x | (kNoDivisor << 16));
+            rows.terms.insert(rows.terms.end(), kRowSlots * kRowTerms, zero | (zero_x << 16));
+            ++rows.n_levels_;
+          }
+          return rows.n_levels();
+        };
+        fwd_levels = rows.n_levels();
+        fwd_padded = pad_levels(0);
+        rows.heads.insert(rows.heads.end(), back.heads.begin(), back.heads.end());
+        rows.terms.insert(rows.terms.end(), back.terms.begin(), back.terms.end());
+        rows.n_levels_ += back.n_levels_;
+        bwd_end = rows.n_levels();
+        pad_levels(kRowPadding);
+        // the next solve's first records
+        for (int32_t k = 0; k < 2 * kRowSlots; ++k)
+          rows.heads.push_back(rows.heads[static_cast<size_t>(k)]);
+        for (int32_t k = 0; k < 2 * kRowSlots * kRowTerms; ++k)
+          rows.terms.push_back(rows.terms[static_cast<size_t>(k)]);
+        return rows;
+      };
       // substitutions: rows and row parts that read x before the block (forward) and the
       // rows before the block (back)
       {
@@ -1054,20 +1082,7 @@ namespace micm_hip
           if (!r.terms.empty())
             rows.push_back(std::move(r));
         }
-        tail.rows = row_levels(rows, n, zero, zero_x);
-        // empty levels up to a multiple of kRowPadding (at least that many in all, for the
-        // read ahead)
-        auto pad_levels = [&](int32_t least) {
-          while (tail.rows.n_levels() % kRowPadding != 0 || tail.rows.n_levels() < least)
-          {
-            tail.rows.heads.insert(tail.rows.heads.end(), kRowSlots, zero_x | (kNoDivisor << 16));
-            tail.rows.terms.insert(tail.rows.terms.end(), kRowSlots * kRowTerms, zero | (zero_x << 16));
-            ++tail.rows.n_levels_;
-          }
-          return tail.rows.n_levels();
-        };
-        tail.fwd_levels = tail.rows.n_levels();
-        tail.fwd_padded = pad_levels(0);
+        const RowLevels forward = row_levels(rows, n, zero, zero_x);
         rows.clear();
         for (int32_t i = first - 1; i >= 0; --i)
         {
@@ -1079,17 +1094,36 @@ namespace micm_hip
                               (static_cast<uint32_t>(t.bwd_col[q]) << 16));
           rows.push_back(std::move(r));
         }
-        const RowLevels back = row_levels(rows, n, zero, zero_x);
-        tail.rows.heads.insert(tail.rows.heads.end(), back.heads.begin(), back.heads.end());
-        tail.rows.terms.insert(tail.rows.terms.end(), back.terms.begin(), back.terms.end());
-        tail.rows.n_levels_ += back.n_levels_;
-        tail.bwd_end = tail.rows.n_levels();
-        pad_levels(kRowPadding);
-        // the next solve's first records
-        for (int32_t k = 0; k < 2 * kRowSlots; ++k)
-          tail.rows.heads.push_back(tail.rows.heads[static_cast<size_t>(k)]);
-        for (int32_t k = 0; k < 2 * kRowSlots * kRowTerms; ++k)
-          tail.rows.terms.push_back(tail.rows.terms[static_cast<size_t>(k)]);
+        tail.rows = join_rows(forward, row_levels(rows, n, zero, zero_x), tail.fwd_levels, tail.fwd_padded, tail.bwd_end);
+      }
+      // the transposed ones: the columns of U and of the strict lower L as rows, ascending
+      {
+        std::vector<SubstitutionRow> rows(static_cast<size_t>(n)), lt(static_cast<size_t>(n));
+        for (int32_t i = 0; i < n; ++i)
+        {
+          rows[static_cast<size_t>(i)].out = lt[static_cast<size_t>(i)].out = static_cast<uint32_t>(i);
+          if (i < first)
+            rows[static_cast<size_t>(i)].diag = static_cast<uint32_t>(pos[t.alu_diag[i]]);
+        }
+        for (int32_t j = 0; j < n; ++j)
+        {
+          const uint32_t x = static_cast<uint32_t>(j) << 16;
+          for (int32_t p = t.upper_row_ptr[j]; j < first && p < t.upper_row_ptr[j + 1]; ++p)
+            if (t.upper_col[p] > j)
+              rows[static_cast<size_t>(t.upper_col[p])].terms.push_back(static_cast<uint32_t>(pos[t.alu_upper[p]]) | x);
+          for (int32_t p = t.lower_row_ptr[j]; p < t.lower_row_ptr[j + 1]; ++p)
+            if (t.lower_col[p] < j && t.lower_col[p] < first)
+              lt[static_cast<size_t>(t.lower_col[p])].terms.push_back(static_cast<uint32_t>(pos[t.alu_lower[p]]) | x);
+        }
+        std::vector<SubstitutionRow> back;
+        for (int32_t i = first - 1; i >= 0; --i)
+          if (!lt[static_cast<size_t>(i)].terms.empty())
+            back.push_back(std::move(lt[static_cast<size_t>(i)]));
+        rows.erase(std::remove_if(rows.begin(), rows.end(),
+                                  [](const SubstitutionRow& r) { return r.terms.empty() && r.diag == kNoDivisor; }),
+                   rows.end());
+        tail.t_rows = join_rows(row_levels(rows, n, zero, zero_x), row_levels(back, n, zero, zero_x), tail.t_fwd_levels,
+                                tail.t_fwd_padded, tail.t_bwd_end);
       }
     }
 
@@ -1180,6 +1214,56 @@ namespace micm_hip
         }
         t.hes_offsets.push_back(static_cast<int32_t>(t.hes_term.size()));
       }
+      // the same lists for batched gathers, with eight padding entries
+      PackedAdjoint& a = t.packed_adjoint;
+      a = PackedAdjoint{};
+      a.weight_offsets.assign(1, 0);
+      for (int32_t r = 0; r < R; ++r)
+      {
+        for (int32_t i = t.product_offsets[r]; i < t.product_offsets[r + 1]; ++i)
+        {
+          a.weight_species.push_back(t.product_ids[i]);
+          a.weight_coef.push_back(t.yields[i]);
+        }
+        for (int32_t i = t.reactant_offsets[r]; i < t.reactant_offsets[r + 1]; ++i)
+        {
+          a.weight_species.push_back(t.reactant_ids[i]);
+          a.weight_coef.push_back(-1.0);
+        }
+        a.weight_offsets.push_back(static_cast<int32_t>(a.weight_species.size()));
+      }
+      a.rxn_terms = t.rxn_terms;
+      for (int32_t q : t.rxn_terms)
+        a.rxn_indep.push_back(t.term_indep[q]);
+      a.indep_terms = t.indep_terms;
+      bool fits = R < 0xffff && n < 0xffff;
+      for (size_t e = 0; e < t.hes_term.size(); ++e)
+      {
+        const int32_t q = t.hes_term[e];
+        uint64_t pack = static_cast<uint64_t>(t.term_process[q]) | (static_cast<uint64_t>(t.term_indep[q]) << 16);
+        int others = 0;
+        for (int32_t i = t.term_dep_offsets[q]; i < t.term_dep_offsets[q + 1]; ++i)
+        {
+          if (i - t.term_dep_offsets[q] == t.hes_slot[e])
+            continue;
+          if (others < 2)
+            pack |= static_cast<uint64_t>(t.term_dep_ids[i]) << (32 + 16 * others);
+          ++others;
+        }
+        fits = fits && others <= 2;
+        for (; others < 2; ++others)
+          pack |= uint64_t(0xffff) << (32 + 16 * others);
+        a.second.push_back(pack);
+      }
+      for (int i = 0; i < 8; ++i)
+      {
+        a.weight_species.push_back(0);
+        a.weight_coef.push_back(0.0);
+        a.rxn_terms.push_back(0);
+        a.rxn_indep.push_back(0);
+        a.indep_terms.push_back(0);
+      }
+      a.ok = fits;
     }
   }  // namespace
 

@@ -128,9 +128,27 @@ namespace micm_hip
     // of kRowPadding (tail_solve's unrolling)
     RowLevels rows;
     int32_t fwd_levels = 0, fwd_padded = 0, bwd_end = 0;
+    // the same of the transposed substitutions, U^T (with its divisions) and then L^T
+    RowLevels t_rows;
+    int32_t t_fwd_levels = 0, t_fwd_padded = 0, t_bwd_end = 0;
   };
   constexpr int kTailBlock = 16;
   constexpr int kTailMax = 64;
+
+  // The adjoint's lists as its kernel with the dense block gathers them: every list ends in
+  // eight padding entries.
+  struct PackedAdjoint
+  {
+    bool ok = false;  // false: positions past 16 bits, or a reaction of more than four reactants
+    // per reaction: its products with their yields, then its reactants with -1
+    std::vector<int32_t> weight_offsets, weight_species;
+    std::vector<double> weight_coef;
+    std::vector<int32_t> rxn_terms, rxn_indep;  // by rxn_term_offsets: the term, its independent species
+    std::vector<int32_t> indep_terms;
+    // second derivatives in hes_offsets' order: process | independent species << 16 | the
+    // term's other reactants << 32, << 48 (0xffff: none)
+    std::vector<uint64_t> second;
+  };
 
   // Rate parameters as consumed by the device (per sorted reaction, stride
   // MICM_HIP_RATE_PARAM_STRIDE).  Derived values live in spare slots:
@@ -229,6 +247,7 @@ namespace micm_hip
     // second derivative: entry (term t, dependent slot a) differentiates d_t by the species
     // in slot a; grouped by that species
     std::vector<int32_t> hes_offsets, hes_term, hes_slot;
+    PackedAdjoint packed_adjoint;
 
     int64_t nnz_alu() const { return (int64_t)alu_col.size(); }
     int64_t nnz_jacobian() const { return (int64_t)jac_col.size(); }

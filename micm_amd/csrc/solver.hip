@@ -17,6 +17,7 @@
 //   COOPERATIVE -- per-cell step size; one workgroup per cell (coop.hpp), cells from
 //                 a work queue, in the previous Solve's cost order once there was one.
 #include "adjoint.hpp"
+#include "adjoint_tail.hpp"
 #include "coop_tail.hpp"
 #include "coop.hpp"
 #include "device.hpp"
@@ -1725,6 +1726,7 @@ struct micm_hip_mechanism
   DevLevels lu_capped[kNumLuBlockings * kNumLuCaps] = {};
   DevTail tail{};
   DevAdjoint adj{};
+  DevAdjointLists adj_lists{};
   void* blob = nullptr;  // one device allocation for every table
   int device = 0;
 };
@@ -1864,7 +1866,14 @@ namespace
   {
     return padded_bytes(t.jac_pos) + padded_bytes(t.diag_pos) + padded_bytes(t.lower_pos) +
            padded_bytes(t.upper_pos) + padded_bytes(t.row_mask) + level_bytes(t.lu) +
-           padded_bytes(t.rows.heads) + padded_bytes(t.rows.terms);
+           padded_bytes(t.rows.heads) + padded_bytes(t.rows.terms) + padded_bytes(t.t_rows.heads) +
+           padded_bytes(t.t_rows.terms);
+  }
+
+  size_t packed_adjoint_bytes(const PackedAdjoint& a)
+  {
+    return padded_bytes(a.weight_offsets) + padded_bytes(a.weight_species) + padded_bytes(a.weight_coef) +
+           padded_bytes(a.rxn_terms) + padded_bytes(a.rxn_indep) + padded_bytes(a.indep_terms) + padded_bytes(a.second);
   }
 
   size_t blocked_level_bytes(const MechanismTables& t)
@@ -2062,7 +2071,7 @@ namespace
              padded_bytes(t.jel_coef) + padded_bytes(t.jel_pack) + level_bytes(t.lv_ut) + level_bytes(t.lv_lt) +
              padded_bytes(t.term_indep) + padded_bytes(t.rxn_term_offsets) + padded_bytes(t.rxn_terms) +
              padded_bytes(t.indep_term_offsets) + padded_bytes(t.indep_terms) + padded_bytes(t.hes_offsets) +
-             padded_bytes(t.hes_term) + padded_bytes(t.hes_slot) + 256;
+             padded_bytes(t.hes_term) + padded_bytes(t.hes_slot) + packed_adjoint_bytes(t.packed_adjoint) + 256;
     HIP_TRY(hipMalloc(&m->blob, bytes));
     std::vector<char> staging;
     size_t off = 0;
@@ -2159,6 +2168,10 @@ namespace
       tl.fwd_levels = t.tail.fwd_levels;
       tl.fwd_padded = t.tail.fwd_padded;
       tl.bwd_end = t.tail.bwd_end;
+      upload_rows(m->blob, off, t.tail.t_rows, tl.t_rows, staging);
+      tl.t_fwd_levels = t.tail.t_fwd_levels;
+      tl.t_fwd_padded = t.tail.t_fwd_padded;
+      tl.t_bwd_end = t.tail.t_bwd_end;
     }
     DevAdjoint& a = m->adj;
     upload_levels(m->blob, off, t.lv_ut, a.ut, staging);
@@ -2171,6 +2184,19 @@ namespace
     upload(m->blob, off, t.hes_offsets, a.hes_offsets, staging);
     upload(m->blob, off, t.hes_term, a.hes_term, staging);
     upload(m->blob, off, t.hes_slot, a.hes_slot, staging);
+    const PackedAdjoint& pa = t.packed_adjoint;
+    DevAdjointLists& al = m->adj_lists;
+    upload(m->blob, off, pa.weight_offsets, al.weight_offsets, staging);
+    upload(m->blob, off, pa.weight_species, al.weight_species, staging);
+    upload(m->blob, off, pa.weight_coef, al.weight_coef, staging);
+    al.rxn_offsets = a.rxn_term_offsets;
+    upload(m->blob, off, pa.rxn_terms, al.rxn_terms, staging);
+    upload(m->blob, off, pa.rxn_indep, al.rxn_indep, staging);
+    al.indep_offsets = a.indep_term_offsets;
+    upload(m->blob, off, pa.indep_terms, al.indep_terms, staging);
+    al.second_offsets = a.hes_offsets;
+    upload(m->blob, off, pa.second, al.second, staging);
+    al.n_second = pa.ok ? static_cast<int32_t>(pa.second.size()) : -1;
     if (off > bytes)
       return fail(MICM_HIP_ERR_DEVICE, "internal table sizing error");
     HIP_TRY(hipMemcpy(m->blob, staging.data(), off, hipMemcpyHostToDevice));
@@ -3665,17 +3691,34 @@ extern "C"
       return fail(MICM_HIP_ERR_UNSUPPORTED, "the adjoint's per-cell working set (" + std::to_string(lds) +
                                                 " bytes) does not fit one workgroup's LDS");
     const DevParams p = make_params(*params, 1.0, s->rtol);
-    constexpr int kAdjThreads = 256;
-    const void* fn = reinterpret_cast<const void*>(k_adjoint<kAdjThreads>);
-    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    const Tape tp{ tape->records, tape->counts, tape->max_records };
     int dev = 0, cus = 0, per_cu = 0;
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const auto grid = [&](int resident) {
+      return static_cast<unsigned>(std::max<int64_t>(
+          1, std::min<int64_t>(s->n_cells, static_cast<int64_t>(cus) * std::max(resident, 1) * 4)));
+    };
+    // with the dense block wherever it takes the mechanism (16 to 256 species, reactions of up
+    // to four reactants, the working set in LDS): 20/50 to 210/560 in a half to a fifth of
+    // k_adjoint's time (adjoint_tail.hip)
+    if (m->tail.size > 0 && d.n_species <= kTailThreads && m->adj_lists.n_second >= 0)
+    {
+      const size_t tail_lds = adjoint_tail_lds(d, c, m->tail, m->adj_lists, static_cast<int>(params->stages));
+      const int resident = tail_lds <= lds_limit() ? adjoint_tail_occupancy(tail_lds) : 0;
+      if (resident > 0)
+      {
+        HIP_TRY(adjoint_tail(d, c, m->tail, m->adj_lists, p, s->n_cells, grid(resident), tail_lds, s->k, tp, seed,
+                             grad_variables, grad_log_rate_constants, s->stream));
+        HIP_TRY(hipStreamSynchronize(s->stream));
+        return MICM_HIP_OK;
+      }
+    }
+    constexpr int kAdjThreads = 256;
+    const void* fn = reinterpret_cast<const void*>(k_adjoint<kAdjThreads>);
+    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_adjoint<kAdjThreads>, kAdjThreads, lds));
-    const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>(s->n_cells, static_cast<int64_t>(cus) *
-                                                                                   std::max(per_cu, 1) * 4));
-    const Tape tp{ tape->records, tape->counts, tape->max_records };
-    hipLaunchKernelGGL(k_adjoint<kAdjThreads>, dim3(static_cast<unsigned>(blocks)), dim3(kAdjThreads), lds, s->stream,
+    hipLaunchKernelGGL(k_adjoint<kAdjThreads>, dim3(grid(per_cu)), dim3(kAdjThreads), lds, s->stream,
                        d, c, m->adj, p, s->n_cells, s->k, tp, seed, grad_variables, grad_log_rate_constants);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));

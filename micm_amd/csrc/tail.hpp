@@ -320,20 +320,24 @@ namespace micm_hip
   // one wavefront issues an instruction every five clocks, so a row costs its products (5.4
   // clocks each) and its instructions: 9.6 us for both triangles of 64 rows, 3.6 us of 32
   // (13.6 and 5.7 us with the rows in a loop and their addresses formed in it).
-  template<int D, int G>
+  //
+  // TRANSPOSED: the rows of L^T, the block's columns below its diagonal, without divisions.
+  template<int D, int G, bool TRANSPOSED>
   __device__ __forceinline__ void tail_back(double (&xg)[D / kTailBlock], const double* block, const double* zs,
                                             double m1)
   {
     constexpr int Q = D / kTailBlock, S = D + 1;
     int l16 = threadIdx.x & 15;
     here(l16);
-    const double* lane = block + l16;
-    double u[Q], diag, z;
+    constexpr int row = TRANSPOSED ? 1 : S, column = TRANSPOSED ? S : 1;
+    const double* lane = block + l16 * column;
+    double u[Q], diag = 1.0, z;
     constexpr int last = kTailBlock * G + kTailBlock - 1;
 #pragma unroll
     for (int g = G; g < Q; ++g)
-      u[g] = lane[last * S + kTailBlock * g];
-    diag = block[last * S + last];
+      u[g] = lane[last * row + kTailBlock * g * column];
+    if constexpr (!TRANSPOSED)
+      diag = block[last * S + last];
     z = zs[last];
 #pragma unroll
     for (int rr = kTailBlock - 1; rr >= 0; --rr)
@@ -348,8 +352,9 @@ namespace micm_hip
       {
 #pragma unroll
         for (int g = G; g < Q; ++g)
-          u[g] = lane[(i - 1) * S + kTailBlock * g];
-        diag = block[(i - 1) * S + i - 1];
+          u[g] = lane[(i - 1) * row + kTailBlock * g * column];
+        if constexpr (!TRANSPOSED)
+          diag = block[(i - 1) * S + i - 1];
         z = zs[i - 1];
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -364,8 +369,11 @@ namespace micm_hip
 #pragma unroll
       for (int g = G + 1; g < Q; ++g)
         v = ordered_sub16<0>(v, p[g], m1);
-      v = v / d;
-      asm("" : "+v"(v));  // on every lane: no branch around the division
+      if constexpr (!TRANSPOSED)
+      {
+        v = v / d;
+        asm("" : "+v"(v));  // on every lane: no branch around the division
+      }
       xg[G] = l16 == rr ? v : xg[G];
     }
   }
@@ -409,8 +417,61 @@ namespace micm_hip
     return ok;
   }
 
-  // The block's back rows by one wavefront, as tail_forward.
+  // tail_forward with the block's U^T, lane = column: a column's result is divided by its
+  // U[c][c] before the later ones subtract its products.  Every lane divides, so a column
+  // costs a division and a broadcast (about 100 clocks) and a row of the block one
+  // conflict-free read.
   template<int D>
+  __device__ __forceinline__ bool tail_forward_transposed(const double* block, double* xt)
+  {
+    constexpr int S = D + 1;
+    const int lane = threadIdx.x & (kWave - 1);
+    int r = lane < D ? lane : 0;
+    here(r);
+    double v = xt[r];
+    double u[4], d[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+    {
+      u[q] = block[q * S + r];
+      d[q] = block[q * S + q];
+    }
+#pragma unroll
+    for (int c0 = 0; c0 < D; c0 += 4)
+    {
+      double un[4], dn[4];
+      if (c0 + 4 < D)
+      {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+          un[q] = block[(c0 + 4 + q) * S + r];
+          dn[q] = block[(c0 + 4 + q) * (S + 1)];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+      {
+        double z = readlane_f64(v, static_cast<uint32_t>(c0 + q)) / d[q];
+        asm("" : "+v"(z));
+        const double nv = v - u[q] * z;
+        v = r > c0 + q ? nv : (r == c0 + q ? z : v);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+      {
+        u[q] = un[q];
+        d[q] = dn[q];
+      }
+    }
+    const bool ok = __ballot(!__builtin_isfinite(v)) == 0;
+    if (ok && lane < D)
+      xt[lane] = v;
+    return ok;
+  }
+
+  // The block's back rows by one wavefront, as tail_forward.
+  template<int D, bool TRANSPOSED = false>
   __device__ __forceinline__ bool tail_backward(const double* block, double* xt, double m1)
   {
     constexpr int Q = D / kTailBlock;
@@ -419,12 +480,12 @@ namespace micm_hip
     for (int g = 0; g < Q; ++g)
       xg[g] = 0.0;
     if constexpr (Q > 3)
-      tail_back<D, 3>(xg, block, xt, m1);
+      tail_back<D, 3, TRANSPOSED>(xg, block, xt, m1);
     if constexpr (Q > 2)
-      tail_back<D, 2>(xg, block, xt, m1);
+      tail_back<D, 2, TRANSPOSED>(xg, block, xt, m1);
     if constexpr (Q > 1)
-      tail_back<D, 1>(xg, block, xt, m1);
-    tail_back<D, 0>(xg, block, xt, m1);
+      tail_back<D, 1, TRANSPOSED>(xg, block, xt, m1);
+    tail_back<D, 0, TRANSPOSED>(xg, block, xt, m1);
     bool finite = true;
 #pragma unroll
     for (int g = 0; g < Q; ++g)
@@ -487,6 +548,42 @@ namespace micm_hip
     }
   }
 
+  // Both transposed triangles of the block with every product tested against the fill pattern.
+  __device__ inline void tail_transposed_masked(const DevTail& t, const double* block, double* xt, bool forward,
+                                                double m1)
+  {
+    const int lane = threadIdx.x & (kWave - 1), l16 = threadIdx.x & 15;
+    const int d = t.size, r = lane < d ? lane : 0;
+    if (forward)
+    {
+      double v = xt[r];
+#pragma unroll 1
+      for (int c = 0; c < d; ++c)
+      {
+        double z = readlane_f64(v, static_cast<uint32_t>(c)) / block[c * (d + 1) + c];
+        asm("" : "+v"(z));
+        const double nv = v - block[c * (d + 1) + r] * z;
+        v = r == c ? z : r > c && ((const_load(t.row_mask, c) >> r) & 1u) ? nv : v;
+      }
+      if (lane < d)
+        xt[lane] = v;
+      return;
+    }
+#pragma unroll 1
+    for (int i = d - 1; i >= 0; --i)
+    {
+      double v = xt[i];
+#pragma unroll 1
+      for (int j = l16; j < d; j += kTailBlock)
+      {
+        const double p = block[j * (d + 1) + i] * xt[j];
+        v = ordered_sub16<0>(v, j > i && ((t.row_mask[j] >> i) & 1u) ? p : 0.0, m1);
+      }
+      xt[i] = v;
+      coop_sync<kWave>();
+    }
+  }
+
   // Both triangles of the block by one wavefront.
   template<int D>
   __device__ __forceinline__ void tail_substitute(const DevTail& t, const double* block, double* xt, bool masked,
@@ -499,14 +596,25 @@ namespace micm_hip
       tail_backward_masked(t, block, xt, m1);
   }
 
+  // Both transposed triangles, U^T and then L^T.
+  template<int D>
+  __device__ __forceinline__ void tail_substitute_transposed(const DevTail& t, const double* block, double* xt,
+                                                             bool masked, double m1)
+  {
+    if (masked || !tail_forward_transposed<D>(block, xt))
+      tail_transposed_masked(t, block, xt, true, m1);
+    coop_sync<kWave>();
+    if (masked || !tail_backward<D, true>(block, xt, m1))
+      tail_transposed_masked(t, block, xt, false, m1);
+  }
+
   // Levels [begin, end) of the rows' list, the record of level l + 2 read while level l runs.
   // Three records rotate, unrolled by three so that none moves; level counts are padded to
   // multiples of three, so that the next levels start with the same record.
   template<Divide DIV>
-  __device__ __forceinline__ void tail_levels(const DevTail& t, int begin, int end, const double* A, double* x, double m1,
-                                              const double* ld, RowsAhead& ahead)
+  __device__ __forceinline__ void tail_levels(const DevTail& t, const DevRows& r, int begin, int end, const double* A, double* x,
+                                              double m1, const double* ld, RowsAhead& ahead)
   {
-    const DevRows& r = t.rows;
     const uint32_t pad = static_cast<uint32_t>(t.nnz) | (static_cast<uint32_t>(t.first + t.size) << 16);
     RowRecord spare;
     auto step = [&](int l, const RowRecord& cur, RowRecord& next) {
@@ -535,7 +643,7 @@ namespace micm_hip
   {
     double m1 = -1.0;
     asm("" : "+v"(m1));
-    tail_levels<Divide::kNone>(t, 0, t.fwd_levels, A, x, m1, nullptr, ahead);
+    tail_levels<Divide::kNone>(t, t.rows, 0, t.fwd_levels, A, x, m1, nullptr, ahead);
     if (threadIdx.x < kWave)
     {
       const double* b = A + t.head;
@@ -549,7 +657,29 @@ namespace micm_hip
       }
     }
     lds_barrier<kTailThreads>();
-    tail_levels<Divide::kUpper>(t, t.fwd_padded, t.bwd_end, A, x, m1, nullptr, ahead);
+    tail_levels<Divide::kUpper>(t, t.rows, t.fwd_padded, t.bwd_end, A, x, m1, nullptr, ahead);
+  }
+
+  // The same with the transposed factors: U^T, then L^T; x[n] = 0, `ahead` of t.t_rows.
+  __device__ inline void tail_solve_transposed(const DevTail& t, const double* A, double* x, bool masked, RowsAhead& ahead)
+  {
+    double m1 = -1.0;
+    asm("" : "+v"(m1));
+    tail_levels<Divide::kUpper>(t, t.t_rows, 0, t.t_fwd_levels, A, x, m1, nullptr, ahead);
+    if (threadIdx.x < kWave)
+    {
+      const double* b = A + t.head;
+      double* xt = x + t.first;
+      switch (t.size)
+      {
+        case 16: tail_substitute_transposed<16>(t, b, xt, masked, m1); break;
+        case 32: tail_substitute_transposed<32>(t, b, xt, masked, m1); break;
+        case 48: tail_substitute_transposed<48>(t, b, xt, masked, m1); break;
+        default: tail_substitute_transposed<64>(t, b, xt, masked, m1); break;
+      }
+    }
+    lds_barrier<kTailThreads>();
+    tail_levels<Divide::kNone>(t, t.t_rows, t.t_fwd_padded, t.t_bwd_end, A, x, m1, nullptr, ahead);
   }
 
   // The same for a lower factor with the diagonal ld (rows without terms already divided).
@@ -558,7 +688,7 @@ namespace micm_hip
   {
     double m1 = -1.0;
     asm("" : "+v"(m1));
-    tail_levels<Divide::kLower>(t, 0, t.fwd_levels, A, x, m1, ld, ahead);
+    tail_levels<Divide::kLower>(t, t.rows, 0, t.fwd_levels, A, x, m1, ld, ahead);
     if (threadIdx.x < kWave)
     {
       tail_forward_masked(t, A + t.head, x + t.first, ld + t.first);
@@ -566,6 +696,6 @@ namespace micm_hip
       tail_backward_masked(t, A + t.head, x + t.first, m1);
     }
     lds_barrier<kTailThreads>();
-    tail_levels<Divide::kUpper>(t, t.fwd_padded, t.bwd_end, A, x, m1, nullptr, ahead);
+    tail_levels<Divide::kUpper>(t, t.rows, t.fwd_padded, t.bwd_end, A, x, m1, nullptr, ahead);
   }
 }  // namespace micm_hip
