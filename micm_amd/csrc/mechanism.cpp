@@ -1127,6 +1127,41 @@ namespace micm_hip
       }
     }
 
+    void build_tiny_tables(MechanismTables& t)
+    {
+      TinyTables& tiny = t.tiny;
+      tiny = TinyTables{};
+      const int32_t n = static_cast<int32_t>(t.n_species);
+      if (n > kTinySpecies || !t.coop_levels_ok)
+        return;
+      for (uint64_t v : t.rxn_pack)
+        if ((v >> 48) == 0xffffu)
+          return;
+      for (uint64_t v : t.term_pack)
+        if ((v >> 48) == 0xffffu)
+          return;
+      auto add = [](std::vector<TinyEntry>& list, const std::vector<int32_t>& from, const std::vector<double>& coef, int32_t b,
+                    int32_t e, int32_t to, int32_t spare) {
+        for (int32_t q = b; q < e; ++q)
+          list.push_back(TinyEntry{ static_cast<uint32_t>(from[q]), static_cast<uint32_t>(q + 1 < e ? spare : to), coef[q] });
+      };
+      auto pad = [](std::vector<TinyEntry>& list, int32_t spare) {
+        while (list.size() % kTinyBatch != 0)
+          list.push_back(TinyEntry{ 0, static_cast<uint32_t>(spare), 0.0 });
+      };
+      for (int32_t i = 0; i < n; ++i)
+      {
+        add(tiny.forcing, t.spec_rxn, t.spec_coef, t.spec_offsets[i], t.spec_offsets[i + 1], i, n);
+        for (int32_t p = t.jac_row_ptr[i]; p < t.jac_row_ptr[i + 1]; ++p)
+          add(tiny.jacobian, t.jel_term, t.jel_coef, t.jel_offsets[p], t.jel_offsets[p + 1], n * i + t.jac_col[p], n * n);
+        for (int32_t p = t.alu_row_ptr[i]; p < t.alu_row_ptr[i + 1]; ++p)
+          tiny.pattern |= uint64_t(1) << (kTinySpecies * i + t.alu_col[p]);
+      }
+      pad(tiny.forcing, n);
+      pad(tiny.jacobian, n * n);
+      tiny.ok = true;
+    }
+
     // Tables of the discrete adjoint.  The transposed substitutions have no counterpart in
     // the reference; their sums run in ascending column order.
     void build_adjoint_tables(MechanismTables& t)
@@ -1583,6 +1618,7 @@ namespace micm_hip
     build_cooperative_schedule(t);
     build_tail_tables(t);
     build_adjoint_tables(t);
+    build_tiny_tables(t);
     for (size_t i = 0; i < t.lu_term_l.size(); ++i)
     {
       t.lu_term_pairs.push_back(t.lu_term_l[i]);

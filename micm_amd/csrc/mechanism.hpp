@@ -150,6 +150,25 @@ namespace micm_hip
     std::vector<uint64_t> second;
   };
 
+  // Gathers of a mechanism of at most kTinySpecies species as lists that one lane walks for its
+  // own cell: an entry adds coef * source[from] to a running sum and stores it at `to`; the sum
+  // starts from zero again after an entry whose `to` is not the spare place (after the last of
+  // the destination), which entries before the end of a sum name.
+  constexpr int kTinySpecies = 8;
+  constexpr int kTinyBatch = 4;  // lists are padded to a multiple
+  struct TinyEntry
+  {
+    uint32_t from, to;
+    double coef;
+  };
+  struct TinyTables
+  {
+    bool ok = false;
+    uint64_t pattern = 0;  // bit kTinySpecies i + j: element (i, j) of the in-place factor
+    std::vector<TinyEntry> forcing;   // rates into species
+    std::vector<TinyEntry> jacobian;  // Jacobian terms into elements, n_species i + j
+  };
+
   // Rate parameters as consumed by the device (per sorted reaction, stride
   // MICM_HIP_RATE_PARAM_STRIDE).  Derived values live in spare slots:
   //   BRANCHED  slot 5 = k0, slot 6 = z   (reaction_rate_store.hpp:286-293)
@@ -248,6 +267,7 @@ namespace micm_hip
     // in slot a; grouped by that species
     std::vector<int32_t> hes_offsets, hes_term, hes_slot;
     PackedAdjoint packed_adjoint;
+    TinyTables tiny;
 
     int64_t nnz_alu() const { return (int64_t)alu_col.size(); }
     int64_t nnz_jacobian() const { return (int64_t)jac_col.size(); }

@@ -18,6 +18,7 @@
 //                 a work queue, in the previous Solve's cost order once there was one.
 #include "adjoint.hpp"
 #include "adjoint_tail.hpp"
+#include "tiny.hpp"
 #include "coop_tail.hpp"
 #include "coop.hpp"
 #include "device.hpp"
@@ -1727,6 +1728,7 @@ struct micm_hip_mechanism
   DevTail tail{};
   DevAdjoint adj{};
   DevAdjointLists adj_lists{};
+  DevTiny tiny{ nullptr, nullptr, -1, 0, 0 };
   void* blob = nullptr;  // one device allocation for every table
   int device = 0;
 };
@@ -2071,7 +2073,8 @@ namespace
              padded_bytes(t.jel_coef) + padded_bytes(t.jel_pack) + level_bytes(t.lv_ut) + level_bytes(t.lv_lt) +
              padded_bytes(t.term_indep) + padded_bytes(t.rxn_term_offsets) + padded_bytes(t.rxn_terms) +
              padded_bytes(t.indep_term_offsets) + padded_bytes(t.indep_terms) + padded_bytes(t.hes_offsets) +
-             padded_bytes(t.hes_term) + padded_bytes(t.hes_slot) + packed_adjoint_bytes(t.packed_adjoint) + 256;
+             padded_bytes(t.hes_term) + padded_bytes(t.hes_slot) + packed_adjoint_bytes(t.packed_adjoint) +
+             padded_bytes(t.tiny.forcing) + padded_bytes(t.tiny.jacobian) + 256;
     HIP_TRY(hipMalloc(&m->blob, bytes));
     std::vector<char> staging;
     size_t off = 0;
@@ -2197,6 +2200,14 @@ namespace
     al.second_offsets = a.hes_offsets;
     upload(m->blob, off, pa.second, al.second, staging);
     al.n_second = pa.ok ? static_cast<int32_t>(pa.second.size()) : -1;
+    m->tiny = DevTiny{ nullptr, nullptr, -1, 0, t.tiny.pattern };
+    if (t.tiny.ok)
+    {
+      upload(m->blob, off, t.tiny.forcing, m->tiny.forcing, staging);
+      upload(m->blob, off, t.tiny.jacobian, m->tiny.jacobian, staging);
+      m->tiny.n_forcing = static_cast<int32_t>(t.tiny.forcing.size());
+      m->tiny.n_jacobian = static_cast<int32_t>(t.tiny.jacobian.size());
+    }
     if (off > bytes)
       return fail(MICM_HIP_ERR_DEVICE, "internal table sizing error");
     HIP_TRY(hipMemcpy(m->blob, staging.data(), off, hipMemcpyHostToDevice));
@@ -2576,6 +2587,34 @@ namespace
     }
   }
 
+  int launch_rate_constants(micm_hip_state* s, hipStream_t st)
+  {
+    const DevMech& d = s->mech->dev;
+    hipLaunchKernelGGL(k_rate_constants, rate_grid(s->n_cells, d.n_reactions), dim3(kBlock), 0, st, d, s->n_cells, s->cond,
+                       s->custom, s->k);
+    HIP_TRY(hipGetLastError());
+    return MICM_HIP_OK;
+  }
+
+  // LDS of the one-lane-per-cell kernel where a Solve's cells take it, else 0: at most eight
+  // species, the library's choice of layout (stage < 0; the threads per cell have nothing to do
+  // in a mechanism of this size), no recording.
+  // README system, whole Solves with their transfers, against a workgroup per cell: 1 cell 254 ->
+  // 177 us, 1,000 cells 331 -> 213, 10,000 cells 1,147 -> 200, 100,000 cells 9.9 -> 0.62 ms; against
+  // the persistent form 446 -> 176 us, 753 -> 200 us (10,000), 3.4 -> 0.62 ms (100,000).
+  size_t tiny_solve_lds(const micm_hip_state* s, int stages)
+  {
+    return s->coop_stage < 0 && !s->recording.records ? tiny_lds(s->mech->dev, s->mech->coop, s->mech->tiny, stages)
+                                                   : 0;
+  }
+
+  TinyArgs tiny_args(micm_hip_state* s, const DevParams& p)
+  {
+    const micm_hip_mechanism* m = s->mech;
+    return TinyArgs{ m->dev, m->coop, m->tiny,   p,         s->n_cells, nullptr,      nullptr,
+                     nullptr, s->y,   s->k,      s->atol,   s->status,  s->stats,     s->final_time };
+  }
+
   int launch_coop_tail(micm_hip_state* s, const DevParams& p, const CoopPlan& plan, const int32_t* list,
                        const int* count, int64_t n_fixed, const CellControl* resume, bool update_rates, hipStream_t st)
   {
@@ -2597,11 +2636,8 @@ namespace
     // The rate constants from a launch of their own: held ready in the Solve's kernel, the rate
     // laws' constants and temporaries cost it 140 spilled registers and 30 KB of code.
     if (update_rates)
-    {
-      hipLaunchKernelGGL(k_rate_constants, rate_grid(s->n_cells, m->dev.n_reactions), dim3(kBlock), 0, st, m->dev,
-                         s->n_cells, s->cond, s->custom, s->k);
-      HIP_TRY(hipGetLastError());
-    }
+      if (int rc = launch_rate_constants(s, st))
+        return rc;
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, a.next);
     HIP_TRY(coop_tail_launch(plan.min_waves, static_cast<unsigned>(blocks), plan.lds, st, a));
     return MICM_HIP_OK;
@@ -2610,6 +2646,19 @@ namespace
   int launch_coop(micm_hip_state* s, const DevParams& p, const int32_t* list, const int* count, int64_t n_fixed,
                   const CellControl* resume, bool update_rates, hipStream_t st)
   {
+    if (const size_t lds = tiny_solve_lds(s, p.stages))
+    {
+      if (update_rates)
+        if (int rc = launch_rate_constants(s, st))
+          return rc;
+      TinyArgs a = tiny_args(s, p);
+      a.n_cells = list ? s->n_cells : n_fixed;
+      a.list = list;
+      a.list_count = count;
+      a.resume = resume;
+      HIP_TRY(tiny_solve(a, lds, st));
+      return MICM_HIP_OK;
+    }
     const CoopPlan plan = plan_coop(s->mech, p.stages, s->coop_stage, s->coop_threads, s->lu_blocking);
     if (plan.lds == 0)
       return fail(MICM_HIP_ERR_UNSUPPORTED, "the cooperative form does not fit this mechanism in LDS");
@@ -2647,15 +2696,17 @@ namespace
   // factors in numbers that fill the chip's lanes (64 lanes x 4 SIMDs x 256 CUs).  60/200:
   // 20,011 cells 55 ms against 195 (hand-off after 16 steps) and 351 (48), 120,000 cells 250
   // against 370 and 519; 210/560, 20,000 cells 394 against 1,424; 20/50: 10,000 cells 28
-  // against 41, 200,000 cells 97 against 67 ms.
+  // against 41, 200,000 cells 97 against 67 ms.  With one cell per lane (tiny_solve_lds) always.
   constexpr int64_t kPerLaneFactor = 300;
   constexpr int64_t kPerLaneCells = 65536;
   constexpr int64_t kHandoffBlock = 16, kHandoffLevels = 48;  // default hand-off steps
 
-  bool hands_off_at_once(const micm_hip_state* s, const CoopPlan& plan)
+  bool hands_off_at_once(const micm_hip_state* s, const CoopPlan& plan, int stages)
   {
-    return s->handoff_steps < 0 && plan.tail &&
-           (s->mech->coop.nnz_alu > kPerLaneFactor || s->n_cells < kPerLaneCells);
+    if (s->handoff_steps >= 0)
+      return false;
+    return tiny_solve_lds(s, stages) > 0 ||
+           (plan.tail && (s->mech->coop.nnz_alu > kPerLaneFactor || s->n_cells < kPerLaneCells));
   }
 
   int prepare_solve(micm_hip_state* s, int32_t form, int stages)
@@ -2663,7 +2714,7 @@ namespace
     if (form == MICM_HIP_SOLVE_COOPERATIVE || form == MICM_HIP_SOLVE_PERSISTENT)
     {
       const CoopPlan plan = plan_coop(s->mech, stages, s->coop_stage, s->coop_threads, s->lu_blocking);
-      if (form == MICM_HIP_SOLVE_PERSISTENT && hands_off_at_once(s, plan))
+      if (form == MICM_HIP_SOLVE_PERSISTENT && hands_off_at_once(s, plan, stages))
         form = MICM_HIP_SOLVE_COOPERATIVE;
       if (plan.compact)
       {
@@ -2728,6 +2779,9 @@ namespace
   // first, once there was one), then the order for the next.
   int enqueue_solve(micm_hip_state* s, const DevParams& p, int32_t form, bool update_rates, hipStream_t st)
   {
+    // one cell per lane: as the cells stand, no order
+    if (tiny_solve_lds(s, p.stages) > 0 && (form == MICM_HIP_SOLVE_COOPERATIVE || s->handoff_steps < 0))
+      return launch_coop(s, p, nullptr, nullptr, s->n_cells, nullptr, update_rates, st);
     if (int rc = enqueue_solve_cells(s, p, form, update_rates, st))
       return rc;
     return enqueue_order(s, st);
@@ -2738,7 +2792,7 @@ namespace
     const micm_hip_mechanism* m = s->mech;
     const DevMech& d = m->dev;
     const CoopPlan plan = plan_coop(m, p.stages, s->coop_stage, s->coop_threads, s->lu_blocking);
-    if (form == MICM_HIP_SOLVE_COOPERATIVE || hands_off_at_once(s, plan))
+    if (form == MICM_HIP_SOLVE_COOPERATIVE || hands_off_at_once(s, plan, p.stages))
       return s->has_order ? launch_coop(s, p, s->order, s->order_bins + kOrderBins, 0, nullptr, update_rates, st)
                           : launch_coop(s, p, nullptr, nullptr, s->n_cells, nullptr, update_rates, st);
     int64_t blocks = 0;
@@ -3399,6 +3453,16 @@ extern "C"
       }
       const bool lockstep = form == MICM_HIP_SOLVE_LOCKSTEP;
       p.error_group = s->lockstep_group;
+      // a wavefront of cells of a mechanism of at most eight species: one lane per cell
+      // (README system through the facade: 1 cell 495 -> 242 us, 64 cells 493 -> 292; the loop in
+      // one workgroup takes its values and tables from global memory)
+      if (lockstep && s->n_cells <= kGroup)
+        if (const size_t lds = tiny_lds(d, m->coop, m->tiny, p.stages))
+        {
+          HIP_TRY(tiny_lockstep(tiny_args(s, p), lds, st));
+          HIP_TRY(hipStreamSynchronize(st));
+          return MICM_HIP_OK;
+        }
       Work w = state_work(s);
       hipLaunchKernelGGL(k_plain_init, dim3(grid), dim3(kBlock), 0, st, p, s->n_cells, s->ctl);
       HIP_TRY(hipGetLastError());
