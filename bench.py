@@ -262,7 +262,16 @@ def kernel_rooflines(mech, state, stream, n_cells, repeats=5):
     return out
 
 
-def measured_traffic(workload_name, n_cells, threads, stage):
+def solve_kernel(threads, stage, n_species):
+    """The cooperative form's kernel for a requested shape."""
+    if stage < 0 and n_species <= 8:
+        return "k_tiny"
+    if 16 <= n_species <= 256 and ((threads == 256 and (stage < 0 or stage >= 4)) or (threads == 0 and stage < 0)):
+        return "k_coop_tail"
+    return f"k_coop<{threads}>"
+
+
+def measured_traffic(workload_name, n_cells, threads, stage, n_species):
     """HBM bytes per Solve launch from a committed rocprofv3 PMC summary
     (profiles/*_hbm_traffic.md, FETCH_SIZE and WRITE_SIZE runs scaled by the same
     counters on a 1 GiB copy) when one covers this workload, cell count and
@@ -274,7 +283,7 @@ def measured_traffic(workload_name, n_cells, threads, stage):
         for block in text.split("```json")[1:]:
             rec = json.loads(block.split("```")[0])
             if (rec.get("workload"), rec.get("cells"), rec.get("kernel"), rec.get("stage")) == \
-                    (workload_name, n_cells, f"k_coop<{threads}>", stage):
+                    (workload_name, n_cells, solve_kernel(threads, stage, n_species), stage):
                 return rec["traffic_bytes"], os.path.relpath(path, ROOT)
     return None, None
 
@@ -480,7 +489,8 @@ def main():
     achieved = bytes_per_step / (kernel_ms * 1e-3) / 1e9
     flops_per_step = algorithmic_flops(flops_per_invocation(desc, mech), stats)
     tflops = flops_per_step / (kernel_ms * 1e-3) / 1e12
-    traffic, traffic_source = (measured_traffic(args.workload, n_cells, coop_threads, coop_stage) if coop_threads
+    traffic, traffic_source = (measured_traffic(args.workload, n_cells, coop_threads, coop_stage,
+                                                       mech.n_species) if coop_threads
                                else (None, None))
     conv = status == 2
     result = {
@@ -508,9 +518,9 @@ def main():
                      "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
                      "traffic_source": traffic_source,
                      "traffic_gbs": round(traffic / (kernel_ms * 1e-3) / 1e9, 2) if traffic else None,
-                     "limiter": ("latency: the factorisation's and substitutions' level schedules, a few dependent "
-                                 "LDS round trips per level, as many cells per CU as LDS holds" if coop_threads else
-                                 "latency and HBM: one cell per lane over the grouped arrays"),
+                     "limiter": ("latency: the dependency chains of the factorisation and the substitutions (dense "
+                                 "block, level schedules), as many cells per CU as LDS holds" if coop_threads else
+                                 "latency: one cell per lane, or one workgroup per cell"),
                      "kernel": "the Solve launch (one persistent or cooperative kernel per step); algorithmic bytes "
                                f"per step {bytes_per_step} summed over the attempts the cells took; `achieved` "
                                "prices them as per-kernel HBM streams, `traffic_gbs` is what the fused kernel "

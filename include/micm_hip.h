@@ -104,11 +104,12 @@ extern "C" {
 #define MICM_HIP_SOLVE_PLAIN 1      /* per-cell step size, one launch per phase of an attempt */
 #define MICM_HIP_SOLVE_PERSISTENT 2 /* per-cell step size, persistent work-queue kernel; cells that
                                        reach the hand-off step count continue in the cooperative form */
-#define MICM_HIP_SOLVE_COOPERATIVE 3 /* per-cell step size, one wavefront per cell, working set in LDS */
-/* OR-ed into the form: UpdateStateParameters fused into the Solve launch -- each
- * cell's rate constants are computed from its conditions and custom parameters as
- * the cell is loaded (and stored in the state), instead of by a separate
- * micm_hip_update_state_parameters call.  Same results. */
+#define MICM_HIP_SOLVE_COOPERATIVE 3 /* per-cell step size, one workgroup per cell, working set in LDS
+                                        (one lane per cell for mechanisms of at most eight species) */
+/* OR-ed into the form: UpdateStateParameters with the Solve -- each cell's rate
+ * constants are computed from its conditions and custom parameters (and stored in
+ * the state), instead of by a separate micm_hip_update_state_parameters call.  Same
+ * results. */
 #define MICM_HIP_SOLVE_UPDATE_RATES 0x100
 
 /* Flat mechanism description.  Species are the phase's non-parameterized
@@ -312,9 +313,10 @@ int micm_hip_state_set_handoff(micm_hip_state* state, int64_t steps);
  * needs more than 64 threads and at least one thread per species, else ignored).  With 256
  * threads and 16 to 256 species the compact layout is the kernel that takes the factor's last
  * rows as a dense block, which the library's choice of staging (-1) also picks for 256 threads or
- * its own choice of threads; 5 / 6 / 7: that kernel built for three waves per SIMD (168 registers) / two (256) / two, 4 leaving the choice
- * to the occupancy.  A tuning
- * knob in the role of the vector length L of the reference's GPU policies
+ * its own choice of threads; 5 / 6 / 7: that kernel built for three waves per SIMD (168
+ * registers) / two (256) / two, 4 leaving the choice to the occupancy.  With the library's choice
+ * of staging (-1), mechanisms of at most eight species run one cell per lane whatever the threads
+ * (recorded Solves excepted).  A tuning knob in the role of the vector length L of the reference's GPU policies
  * (cuda_solver_builder.hpp:24-38); results do not depend on it. */
 int micm_hip_state_set_cooperative_shape(micm_hip_state* state, int32_t threads, int32_t stage);
 /* Blocking of the cooperative form's LU level schedule: the shortest run of products an
