@@ -19,7 +19,9 @@
 #include "tail.hpp"
 #define MICM_HOST_DEVICE __host__ __device__
 #else
-#define MICM_HOST_DEVICE  // the arithmetic alone, for the host
+// the arithmetic alone, for the host; with MICM_WORKGROUP_ON_HOST the workgroup's sum too, over
+// the includer's own wavefront and barrier operations
+#define MICM_HOST_DEVICE
 #endif
 
 namespace micm_hip
@@ -115,7 +117,7 @@ namespace micm_hip
                      double_from_bits((2 * 1023 + 52 - e) << 52), double_from_bits((e - 52) << 52) };
   }
 
-#if defined(__HIPCC__)
+#if defined(__HIPCC__) || defined(MICM_WORKGROUP_ON_HOST)
   constexpr int kSumChain = 2048;  // leading terms added as one chain
 
   template<int NT>
@@ -222,7 +224,10 @@ namespace micm_hip
           for (int w = 0; w < W; ++w)
             first = s.first[w] < first ? s.first[w] : first;
           if (first == NT)
+          {
+            lds_barrier<NT>();  // s.first is read before the next tile writes it
             break;
+          }
           if (tid == first)
           {
 #pragma unroll
@@ -240,6 +245,7 @@ namespace micm_hip
         {
           // wavefront after wavefront, lane after lane
           load_ordered(base, v);
+          lds_barrier<NT>();  // the chain's s.acc is read before the first wavefront writes it
           for (int w = 0; w < W; ++w)
           {
             if (wave == w)
