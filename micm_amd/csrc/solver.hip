@@ -22,6 +22,7 @@
 #include "coop_tail.hpp"
 #include "coop.hpp"
 #include "device.hpp"
+#include "launch_rules.hpp"
 #include "mechanism.hpp"
 #include "ordered_sum.hpp"
 #include "path.hpp"
@@ -2284,20 +2285,16 @@ namespace
     return static_cast<size_t>(std::max(max_lds, optin)) - 64;  // static __shared__ of the kernel
   }
 
-  // Cells per workgroup of the tiled LU / substitution kernels: the largest power of
-  // two up to 16 whose tile of `doubles_per_cell` leaves room for two workgroups per CU
-  // (two independent workgroups hide each other's level latency: 210/560 LU 1.4x,
-  // 60/200 2.1x against one workgroup of twice the cells), else one cell if it fits;
-  // 0 when the level schedules are unavailable or one cell does not fit.
+  // tile_cells / lu_tile_cells (launch_rules.hpp) of a mechanism, 0 also where the level
+  // schedules are unavailable.
   int tile_cells(const micm_hip_mechanism* m, size_t doubles_per_cell)
   {
-    if (!m->t.coop_levels_ok)
-      return 0;
-    const size_t limit = lds_limit();
-    for (int tc = 16; tc >= 1; tc /= 2)
-      if (2 * doubles_per_cell * tc * sizeof(double) <= limit)
-        return tc;
-    return doubles_per_cell * sizeof(double) <= limit ? 1 : 0;
+    return m->t.coop_levels_ok ? micm_hip::tile_cells(doubles_per_cell, lds_limit()) : 0;
+  }
+
+  int lu_tile_cells(const micm_hip_mechanism* m)
+  {
+    return m->t.coop_levels_ok ? micm_hip::lu_tile_cells(static_cast<size_t>(m->coop.nnz_alu), lds_limit()) : 0;
   }
 
   // Whether the single-phase LU and substitution take the kernels with the factor's dense block
@@ -3112,7 +3109,7 @@ extern "C"
     KERNEL_PRELUDE();
     if (!jac || !lower || !upper)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
-    const int tc = tile_cells(m, static_cast<size_t>(m->coop.nnz_alu));
+    const int tc = lu_tile_cells(m);
     if (phases_with_tail(m, n_cells, tail_factor_lds(m->tail)))
     {
       HIP_TRY(lu_decompose_tail(m->dev, m->tail, n_cells, tiled_blocks(1, n_cells), jac, lower, upper, st));
@@ -3125,7 +3122,6 @@ extern "C"
       {
         case 16: LAUNCH_TILED(k_lu_decompose_tiled<16>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
         case 8: LAUNCH_TILED(k_lu_decompose_tiled<8>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
-        // (tiles of two and four cells are those of factors that the block takes)
         default: LAUNCH_TILED(k_lu_decompose_tiled<1>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
       }
     }

@@ -1,0 +1,35 @@
+"""Sizes of launches (micm_amd/csrc/launch_rules.hpp) over the ranges they are asked for."""
+import ctypes
+import os
+import re
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOLVER = os.path.join(ROOT, "micm_amd", "csrc", "solver.hip")
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("rules") / "librules.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", os.path.join(ROOT, "tests", "launch_rules_harness.cpp"),
+                    "-o", out], check=True)
+    lib = ctypes.CDLL(out)
+    for name in ("tile_cells_host", "tile_cells_host"):
+        getattr(lib, name).argtypes = [ctypes.c_int64, ctypes.c_int64]
+    return lib
+
+
+@pytest.mark.parametrize("kernel,rule", [("k_lu_decompose_tiled", "lu_tile_cells_host"),
+                                         ("k_lu_solve_tiled", "tile_cells_host")])
+@pytest.mark.parametrize("limit", [64 * 1024 - 64, 160 * 1024 - 64])
+def test_a_tile_has_a_kernel_of_its_size(lib, kernel, rule, limit):
+    """The grid is sized for the tile that the rule gives, so the launch needs a kernel built for
+    exactly that tile: with a smaller one, cells past its first would be left out."""
+    built = {int(tc) for tc in re.findall(rf"LAUNCH_TILED\({kernel}<(\d+)>", open(SOLVER).read())}
+    for doubles in range(1, 22000):
+        tc = getattr(lib, rule)(doubles, limit)
+        assert tc == 0 or tc in built, (doubles, tc)
+        assert (tc == 0) == (doubles * 8 > limit), (doubles, tc)
+        assert tc <= 1 or 2 * doubles * tc * 8 <= limit, (doubles, tc)
