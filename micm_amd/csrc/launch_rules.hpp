@@ -1,7 +1,9 @@
 // launch_rules.hpp -- sizes of launches and workspaces as plain functions of their arguments.
 #pragma once
 
+#include <algorithm>
 #include <cstddef>
+#include <cstdint>
 
 namespace micm_hip
 {
@@ -28,6 +30,27 @@ namespace micm_hip
     for (int tc : kLuTiles)
       if (tc <= most)
         return tc;
+    return 0;
+  }
+
+  // A launch takes fewer than 2^32 threads; of more, HIP runs the number modulo 2^32 and reports
+  // nothing.  Cells are therefore launched in slices of at most kMostThreads threads, whole
+  // groups of 64 cells for each of the eight XCDs.
+  constexpr int64_t kMostThreads = int64_t(1) << 31;
+  constexpr int64_t kSliceCells = 512;
+  constexpr int64_t slice_cells(int64_t threads_per_cell)
+  {
+    return std::max(kMostThreads / std::max<int64_t>(threads_per_cell, 1) / kSliceCells, int64_t(1)) * kSliceCells;
+  }
+
+  // launch(first cell, cells) over n_cells cells in slices, until one returns other than 0.
+  template<class Launch>
+  int for_slices(int64_t n_cells, int64_t threads_per_cell, const Launch& launch)
+  {
+    const int64_t most = slice_cells(threads_per_cell);
+    for (int64_t first = 0; first < n_cells; first += most)
+      if (const int rc = launch(first, std::min(most, n_cells - first)))
+        return rc;
     return 0;
   }
 }  // namespace micm_hip

@@ -2333,6 +2333,8 @@ namespace
     return 2 * gather_tile_bytes(m, 2) <= limit ? 2 : 0;
   }
 
+  static_assert(kSliceCells == kXcds * kGroup && MICM_HIP_OK == 0, "as launch_rules.hpp has them");
+
   inline unsigned tiled_blocks(int tc, int64_t n_cells)
   {
     return static_cast<unsigned>((n_groups_of(n_cells) + kXcds - 1) / kXcds * kXcds * (kGroup / tc));
@@ -2758,20 +2760,25 @@ namespace
   // on `st` without waiting; prepare_solve must have run.
   // The processing order of the next Solve from this Solve's per-cell attempt counts.
   // -J of the cells marked kJacobianDue, formed from zero by the LDS-tiled gather
-  int launch_jacobian_due(const micm_hip_mechanism* m, int64_t n_cells, const double* k, const double* y, double* jac,
+  int launch_jacobian_due(const micm_hip_mechanism* m, int64_t all_cells, const double* k, const double* y, double* jac,
                           const CellControl* ctl, hipStream_t st)
   {
     const int tc = gather_tile_cells(m);
     const size_t lds = gather_tile_bytes(m, tc);
-    switch (tc)
-    {
-      case 16: LAUNCH_GATHER(k_jacobian_due_tiled, 16, lds, st, m->dev, m->coop, n_cells, k, y, jac, ctl); break;
-      case 8: LAUNCH_GATHER(k_jacobian_due_tiled, 8, lds, st, m->dev, m->coop, n_cells, k, y, jac, ctl); break;
-      case 4: LAUNCH_GATHER(k_jacobian_due_tiled, 4, lds, st, m->dev, m->coop, n_cells, k, y, jac, ctl); break;
-      default: LAUNCH_GATHER(k_jacobian_due_tiled, 2, lds, st, m->dev, m->coop, n_cells, k, y, jac, ctl); break;
-    }
-    HIP_TRY(hipGetLastError());
-    return MICM_HIP_OK;
+    const DevMech& d = m->dev;
+    return for_slices(all_cells, kGatherThreads / std::max(tc, 1), [&](int64_t c0, int64_t n_cells) -> int {
+      const double *ks = k + c0 * d.n_reactions, *ys = y + c0 * d.n_species;
+      double* js = jac + c0 * d.nnz_jac;
+      switch (tc)
+      {
+        case 16: LAUNCH_GATHER(k_jacobian_due_tiled, 16, lds, st, d, m->coop, n_cells, ks, ys, js, ctl + c0); break;
+        case 8: LAUNCH_GATHER(k_jacobian_due_tiled, 8, lds, st, d, m->coop, n_cells, ks, ys, js, ctl + c0); break;
+        case 4: LAUNCH_GATHER(k_jacobian_due_tiled, 4, lds, st, d, m->coop, n_cells, ks, ys, js, ctl + c0); break;
+        default: LAUNCH_GATHER(k_jacobian_due_tiled, 2, lds, st, d, m->coop, n_cells, ks, ys, js, ctl + c0); break;
+      }
+      HIP_TRY(hipGetLastError());
+      return MICM_HIP_OK;
+    });
   }
 
   int enqueue_order(micm_hip_state* s, hipStream_t st)
@@ -2978,225 +2985,247 @@ extern "C"
 
   // ---- kernel entry points
 
+// (grouped arrays: cell c0, a multiple of 64, starts c0 times the values per cell after the first)
 #define KERNEL_PRELUDE()                                                   \
   if (int rc = check_device_mech(m))                                       \
     return rc;                                                             \
-  if (n_cells < 0)                                                         \
+  if (all_cells < 0)                                                       \
     return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "negative cell count");     \
-  if (n_cells == 0)                                                        \
+  if (all_cells == 0)                                                      \
     return MICM_HIP_OK;                                                    \
   hipStream_t st = static_cast<hipStream_t>(stream)
 
-  int micm_hip_calculate_rate_constants(const micm_hip_mechanism* m, int64_t n_cells, const double* cond,
+  int micm_hip_calculate_rate_constants(const micm_hip_mechanism* m, int64_t all_cells, const double* cond,
                                         const double* custom, double* k, void* stream)
   {
     KERNEL_PRELUDE();
-    if (!cond || !k || (m->dev.n_custom > 0 && !custom))
+    const DevMech& d = m->dev;
+    if (!cond || !k || (d.n_custom > 0 && !custom))
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
-    hipLaunchKernelGGL(k_rate_constants, rate_grid(n_cells, m->dev.n_reactions), dim3(kBlock), 0, st, m->dev, n_cells,
-                       cond, custom, k);
-    HIP_TRY(hipGetLastError());
-    return MICM_HIP_OK;
+    return for_slices(all_cells, 1, [&](int64_t c0, int64_t n_cells) -> int {
+      hipLaunchKernelGGL(k_rate_constants, rate_grid(n_cells, d.n_reactions), dim3(kBlock), 0, st, d, n_cells,
+                         cond + c0 * 3, custom ? custom + c0 * d.n_custom : nullptr, k + c0 * d.n_reactions);
+      HIP_TRY(hipGetLastError());
+      return MICM_HIP_OK;
+    });
   }
 
   // (C++ linkage: templates; the entry points below are the C-ABI)
   extern "C++" template<bool FROM_ZERO>
-  int add_forcing_entry(const micm_hip_mechanism* m, int64_t n_cells, const double* k, const double* y, double* f,
+  int add_forcing_entry(const micm_hip_mechanism* m, int64_t all_cells, const double* k, const double* y, double* f,
                         void* stream)
   {
     KERNEL_PRELUDE();
     if (!k || !y || !f)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
+    const DevMech& d = m->dev;
     const int tc = gather_tile_cells(m);
-    if (tc > 0)
-    {
-      const size_t lds = gather_tile_bytes(m, tc);
-      switch (tc)
+    return for_slices(all_cells, tc > 0 ? kGatherThreads / tc : 1, [&](int64_t c0, int64_t n_cells) -> int {
+      const double *ks = k + c0 * d.n_reactions, *ys = y + c0 * d.n_species;
+      double* fs = f + c0 * d.n_species;
+      if (tc > 0)
       {
-        case 16: LAUNCH_GATHER_Z(k_add_forcing_tiled, 16, FROM_ZERO, lds, st, m->dev, m->coop, n_cells, k, y, f); break;
-        case 8: LAUNCH_GATHER_Z(k_add_forcing_tiled, 8, FROM_ZERO, lds, st, m->dev, m->coop, n_cells, k, y, f); break;
-        case 4: LAUNCH_GATHER_Z(k_add_forcing_tiled, 4, FROM_ZERO, lds, st, m->dev, m->coop, n_cells, k, y, f); break;
-        default: LAUNCH_GATHER_Z(k_add_forcing_tiled, 2, FROM_ZERO, lds, st, m->dev, m->coop, n_cells, k, y, f); break;
+        const size_t lds = gather_tile_bytes(m, tc);
+        switch (tc)
+        {
+          case 16: LAUNCH_GATHER_Z(k_add_forcing_tiled, 16, FROM_ZERO, lds, st, d, m->coop, n_cells, ks, ys, fs); break;
+          case 8: LAUNCH_GATHER_Z(k_add_forcing_tiled, 8, FROM_ZERO, lds, st, d, m->coop, n_cells, ks, ys, fs); break;
+          case 4: LAUNCH_GATHER_Z(k_add_forcing_tiled, 4, FROM_ZERO, lds, st, d, m->coop, n_cells, ks, ys, fs); break;
+          default: LAUNCH_GATHER_Z(k_add_forcing_tiled, 2, FROM_ZERO, lds, st, d, m->coop, n_cells, ks, ys, fs); break;
+        }
       }
-    }
-    else
-    {
-      hipLaunchKernelGGL(k_add_forcing<FROM_ZERO>, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, m->dev, n_cells, k, y,
-                         f);
-    }
-    HIP_TRY(hipGetLastError());
-    return MICM_HIP_OK;
+      else
+      {
+        hipLaunchKernelGGL(k_add_forcing<FROM_ZERO>, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, d, n_cells, ks, ys, fs);
+      }
+      HIP_TRY(hipGetLastError());
+      return MICM_HIP_OK;
+    });
   }
 
   extern "C++" template<bool FROM_ZERO>
-  int subtract_jacobian_entry(const micm_hip_mechanism* m, int64_t n_cells, const double* k, const double* y,
+  int subtract_jacobian_entry(const micm_hip_mechanism* m, int64_t all_cells, const double* k, const double* y,
                               double* jac, void* stream)
   {
     KERNEL_PRELUDE();
     if (!k || !y || !jac)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
+    const DevMech& d = m->dev;
     const int tc = gather_tile_cells(m);
-    if (tc > 0)
-    {
-      const size_t lds = gather_tile_bytes(m, tc);
-      switch (tc)
+    return for_slices(all_cells, tc > 0 ? kGatherThreads / tc : 1, [&](int64_t c0, int64_t n_cells) -> int {
+      const double *ks = k + c0 * d.n_reactions, *ys = y + c0 * d.n_species;
+      double* js = jac + c0 * d.nnz_jac;
+      if (tc > 0)
       {
-        case 16:
-          LAUNCH_GATHER_Z(k_subtract_jacobian_tiled, 16, FROM_ZERO, lds, st, m->dev, m->coop, n_cells, k, y, jac);
-          break;
-        case 8:
-          LAUNCH_GATHER_Z(k_subtract_jacobian_tiled, 8, FROM_ZERO, lds, st, m->dev, m->coop, n_cells, k, y, jac);
-          break;
-        case 4:
-          LAUNCH_GATHER_Z(k_subtract_jacobian_tiled, 4, FROM_ZERO, lds, st, m->dev, m->coop, n_cells, k, y, jac);
-          break;
-        default:
-          LAUNCH_GATHER_Z(k_subtract_jacobian_tiled, 2, FROM_ZERO, lds, st, m->dev, m->coop, n_cells, k, y, jac);
-          break;
+        const size_t lds = gather_tile_bytes(m, tc);
+        switch (tc)
+        {
+          case 16:
+            LAUNCH_GATHER_Z(k_subtract_jacobian_tiled, 16, FROM_ZERO, lds, st, d, m->coop, n_cells, ks, ys, js);
+            break;
+          case 8:
+            LAUNCH_GATHER_Z(k_subtract_jacobian_tiled, 8, FROM_ZERO, lds, st, d, m->coop, n_cells, ks, ys, js);
+            break;
+          case 4:
+            LAUNCH_GATHER_Z(k_subtract_jacobian_tiled, 4, FROM_ZERO, lds, st, d, m->coop, n_cells, ks, ys, js);
+            break;
+          default:
+            LAUNCH_GATHER_Z(k_subtract_jacobian_tiled, 2, FROM_ZERO, lds, st, d, m->coop, n_cells, ks, ys, js);
+            break;
+        }
       }
-    }
-    else
-    {
-      hipLaunchKernelGGL(k_subtract_jacobian<FROM_ZERO>, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, m->dev, n_cells, k,
-                         y, jac);
-    }
-    HIP_TRY(hipGetLastError());
-    return MICM_HIP_OK;
+      else
+      {
+        hipLaunchKernelGGL(k_subtract_jacobian<FROM_ZERO>, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, d, n_cells, ks,
+                           ys, js);
+      }
+      HIP_TRY(hipGetLastError());
+      return MICM_HIP_OK;
+    });
   }
 
-  int micm_hip_add_forcing_terms(const micm_hip_mechanism* m, int64_t n_cells, const double* k, const double* y,
+  int micm_hip_add_forcing_terms(const micm_hip_mechanism* m, int64_t all_cells, const double* k, const double* y,
                                  double* f, void* stream)
   {
-    return add_forcing_entry<false>(m, n_cells, k, y, f, stream);
+    return add_forcing_entry<false>(m, all_cells, k, y, f, stream);
   }
 
-  int micm_hip_fill_and_add_forcing_terms(const micm_hip_mechanism* m, int64_t n_cells, const double* k,
+  int micm_hip_fill_and_add_forcing_terms(const micm_hip_mechanism* m, int64_t all_cells, const double* k,
                                           const double* y, double* f, void* stream)
   {
-    return add_forcing_entry<true>(m, n_cells, k, y, f, stream);
+    return add_forcing_entry<true>(m, all_cells, k, y, f, stream);
   }
 
-  int micm_hip_subtract_jacobian_terms(const micm_hip_mechanism* m, int64_t n_cells, const double* k, const double* y,
+  int micm_hip_subtract_jacobian_terms(const micm_hip_mechanism* m, int64_t all_cells, const double* k, const double* y,
                                        double* jac, void* stream)
   {
-    return subtract_jacobian_entry<false>(m, n_cells, k, y, jac, stream);
+    return subtract_jacobian_entry<false>(m, all_cells, k, y, jac, stream);
   }
 
-  int micm_hip_fill_and_subtract_jacobian_terms(const micm_hip_mechanism* m, int64_t n_cells, const double* k,
+  int micm_hip_fill_and_subtract_jacobian_terms(const micm_hip_mechanism* m, int64_t all_cells, const double* k,
                                                 const double* y, double* jac, void* stream)
   {
-    return subtract_jacobian_entry<true>(m, n_cells, k, y, jac, stream);
+    return subtract_jacobian_entry<true>(m, all_cells, k, y, jac, stream);
   }
 
-  int micm_hip_alpha_minus_jacobian(const micm_hip_mechanism* m, int64_t n_cells, double* jac, double alpha, void* stream)
+  int micm_hip_alpha_minus_jacobian(const micm_hip_mechanism* m, int64_t all_cells, double* jac, double alpha,
+                                    void* stream)
   {
     KERNEL_PRELUDE();
     if (!jac)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
-    if (m->dev.n_species == 0)
+    const DevMech& d = m->dev;
+    return for_slices(all_cells, d.n_species, [&](int64_t c0, int64_t n_cells) -> int {
+      hipLaunchKernelGGL(k_alpha_minus_jacobian,
+                         dim3(static_cast<unsigned>(
+                             (n_groups_of(n_cells) * static_cast<int64_t>(d.n_species) * kGroup + kBlock - 1) / kBlock)),
+                         dim3(kBlock), 0, st, d, n_cells, jac + c0 * d.nnz_jac, alpha);
+      HIP_TRY(hipGetLastError());
       return MICM_HIP_OK;
-    hipLaunchKernelGGL(k_alpha_minus_jacobian,
-                       dim3(static_cast<unsigned>((n_groups_of(n_cells) * static_cast<int64_t>(m->dev.n_species) * kGroup +
-                                                   kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0, st, m->dev, n_cells, jac, alpha);
-    HIP_TRY(hipGetLastError());
-    return MICM_HIP_OK;
+    });
   }
 
-  int micm_hip_lu_decompose(const micm_hip_mechanism* m, int64_t n_cells, const double* jac, double* lower, double* upper,
-                            void* stream)
+  int micm_hip_lu_decompose(const micm_hip_mechanism* m, int64_t all_cells, const double* jac, double* lower,
+                            double* upper, void* stream)
   {
     KERNEL_PRELUDE();
     if (!jac || !lower || !upper)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
+    const DevMech& d = m->dev;
     const int tc = lu_tile_cells(m);
-    if (phases_with_tail(m, n_cells, tail_factor_lds(m->tail)))
-    {
-      HIP_TRY(lu_decompose_tail(m->dev, m->tail, n_cells, tiled_blocks(1, n_cells), jac, lower, upper, st));
-    }
-    else if (tc > 0)
-    {
-      const size_t lds = static_cast<size_t>(m->coop.nnz_alu) * tc * sizeof(double);
-      const unsigned blocks = tiled_blocks(tc, n_cells);
-      switch (tc)
+    const bool tail = phases_with_tail(m, all_cells, tail_factor_lds(m->tail));
+    const int64_t threads = tail ? kTailThreads : tc > 0 ? kTileThreads / tc : 1;
+    return for_slices(all_cells, threads, [&](int64_t c0, int64_t n_cells) -> int {
+      const double* js = jac + c0 * d.nnz_jac;
+      double *lo = lower + c0 * d.nnz_lower, *up = upper + c0 * d.nnz_upper;
+      if (tail)
       {
-        case 16: LAUNCH_TILED(k_lu_decompose_tiled<16>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
-        case 8: LAUNCH_TILED(k_lu_decompose_tiled<8>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
-        default: LAUNCH_TILED(k_lu_decompose_tiled<1>, blocks, lds, st, m->dev, m->coop, n_cells, jac, lower, upper); break;
+        HIP_TRY(lu_decompose_tail(d, m->tail, n_cells, tiled_blocks(1, n_cells), js, lo, up, st));
       }
-    }
-    else
-    {
-      hipLaunchKernelGGL(k_lu_decompose, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, m->dev, n_cells, jac, lower, upper);
-    }
-    HIP_TRY(hipGetLastError());
-    return MICM_HIP_OK;
+      else if (tc > 0)
+      {
+        const size_t lds = static_cast<size_t>(m->coop.nnz_alu) * tc * sizeof(double);
+        const unsigned blocks = tiled_blocks(tc, n_cells);
+        switch (tc)
+        {
+          case 16: LAUNCH_TILED(k_lu_decompose_tiled<16>, blocks, lds, st, d, m->coop, n_cells, js, lo, up); break;
+          case 8: LAUNCH_TILED(k_lu_decompose_tiled<8>, blocks, lds, st, d, m->coop, n_cells, js, lo, up); break;
+          default: LAUNCH_TILED(k_lu_decompose_tiled<1>, blocks, lds, st, d, m->coop, n_cells, js, lo, up); break;
+        }
+      }
+      else
+      {
+        hipLaunchKernelGGL(k_lu_decompose, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, d, n_cells, js, lo, up);
+      }
+      HIP_TRY(hipGetLastError());
+      return MICM_HIP_OK;
+    });
   }
 
-  int micm_hip_lu_solve(const micm_hip_mechanism* m, int64_t n_cells, const double* lower, const double* upper, double* x,
-                        void* stream)
+  int micm_hip_lu_solve(const micm_hip_mechanism* m, int64_t all_cells, const double* lower, const double* upper,
+                        double* x, void* stream)
   {
     KERNEL_PRELUDE();
     if (!lower || !upper || !x)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
-    const int tc = tile_cells(m, static_cast<size_t>(m->coop.nnz_alu) + 2 * static_cast<size_t>(m->dev.n_species));
-    if (phases_with_tail(m, n_cells, tail_solve_lds(m->dev, m->tail)))
+    const DevMech& d = m->dev;
+    const int tc = tile_cells(m, static_cast<size_t>(m->coop.nnz_alu) + 2 * static_cast<size_t>(d.n_species));
+    const bool tail = phases_with_tail(m, all_cells, tail_solve_lds(d, m->tail));
+    const int64_t threads = tail ? kTailThreads : tc > 0 ? kTileThreads / tc : 1;
+    size_t lds = (static_cast<size_t>(m->coop.nnz_alu) + 2 * static_cast<size_t>(d.n_species)) * tc * sizeof(double);
+    // one cell per workgroup: a product buffer for the two-phase back substitution
+    // from what two workgroups per CU leave (levels with more terms run task by task)
+    int p_capacity = 0;
+    if (tc == 1)
     {
-      HIP_TRY(lu_solve_tail(m->dev, m->tail, n_cells, tiled_blocks(1, n_cells), lower, upper, x, st));
+      const size_t spare = lds_limit() / 2 > lds ? (lds_limit() / 2 - lds) / sizeof(double) : 0;
+      p_capacity = static_cast<int>(std::min<size_t>(static_cast<size_t>(m->coop.bwd.max_level_terms), spare));
+      lds += static_cast<size_t>(p_capacity) * sizeof(double);
     }
-    else if (tc > 0)
-    {
-      size_t lds = (static_cast<size_t>(m->coop.nnz_alu) + 2 * static_cast<size_t>(m->dev.n_species)) * tc *
-                   sizeof(double);
-      // one cell per workgroup: a product buffer for the two-phase back substitution
-      // from what two workgroups per CU leave (levels with more terms run task by task)
-      int p_capacity = 0;
-      if (tc == 1)
+    return for_slices(all_cells, threads, [&](int64_t c0, int64_t n_cells) -> int {
+      const double *lo = lower + c0 * d.nnz_lower, *up = upper + c0 * d.nnz_upper;
+      double* xs = x + c0 * d.n_species;
+      if (tail)
       {
-        const size_t spare = lds_limit() / 2 > lds ? (lds_limit() / 2 - lds) / sizeof(double) : 0;
-        p_capacity = static_cast<int>(std::min<size_t>(static_cast<size_t>(m->coop.bwd.max_level_terms), spare));
-        lds += static_cast<size_t>(p_capacity) * sizeof(double);
+        HIP_TRY(lu_solve_tail(d, m->tail, n_cells, tiled_blocks(1, n_cells), lo, up, xs, st));
       }
-      const unsigned blocks = tiled_blocks(tc, n_cells);
-      switch (tc)
+      else if (tc > 0)
       {
-        case 16:
-          LAUNCH_TILED(k_lu_solve_tiled<16>, blocks, lds, st, m->dev, m->coop, n_cells, lower, upper, x, p_capacity);
-          break;
-        case 8:
-          LAUNCH_TILED(k_lu_solve_tiled<8>, blocks, lds, st, m->dev, m->coop, n_cells, lower, upper, x, p_capacity);
-          break;
-        case 4:
-          LAUNCH_TILED(k_lu_solve_tiled<4>, blocks, lds, st, m->dev, m->coop, n_cells, lower, upper, x, p_capacity);
-          break;
-        case 2:
-          LAUNCH_TILED(k_lu_solve_tiled<2>, blocks, lds, st, m->dev, m->coop, n_cells, lower, upper, x, p_capacity);
-          break;
-        default:
-          LAUNCH_TILED(k_lu_solve_tiled<1>, blocks, lds, st, m->dev, m->coop, n_cells, lower, upper, x, p_capacity);
-          break;
+        const unsigned blocks = tiled_blocks(tc, n_cells);
+        switch (tc)
+        {
+          case 16: LAUNCH_TILED(k_lu_solve_tiled<16>, blocks, lds, st, d, m->coop, n_cells, lo, up, xs, p_capacity); break;
+          case 8: LAUNCH_TILED(k_lu_solve_tiled<8>, blocks, lds, st, d, m->coop, n_cells, lo, up, xs, p_capacity); break;
+          case 4: LAUNCH_TILED(k_lu_solve_tiled<4>, blocks, lds, st, d, m->coop, n_cells, lo, up, xs, p_capacity); break;
+          case 2: LAUNCH_TILED(k_lu_solve_tiled<2>, blocks, lds, st, d, m->coop, n_cells, lo, up, xs, p_capacity); break;
+          default: LAUNCH_TILED(k_lu_solve_tiled<1>, blocks, lds, st, d, m->coop, n_cells, lo, up, xs, p_capacity); break;
+        }
       }
-    }
-    else
-    {
-      hipLaunchKernelGGL(k_lu_solve, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, m->dev, n_cells, lower, upper, x);
-    }
-    HIP_TRY(hipGetLastError());
-    return MICM_HIP_OK;
+      else
+      {
+        hipLaunchKernelGGL(k_lu_solve, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, d, n_cells, lo, up, xs);
+      }
+      HIP_TRY(hipGetLastError());
+      return MICM_HIP_OK;
+    });
   }
 
-  int micm_hip_normalized_error(const micm_hip_mechanism* m, int64_t n_cells, const double* y, const double* ynew,
+  int micm_hip_normalized_error(const micm_hip_mechanism* m, int64_t all_cells, const double* y, const double* ynew,
                                 const double* yerr, const double* atol, double rtol, double* error, void* stream)
   {
     KERNEL_PRELUDE();
     if (!y || !ynew || !yerr || !atol || !error)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
-    hipLaunchKernelGGL(k_normalized_error, dim3(static_cast<unsigned>(n_groups_of(n_cells) * (kGroup / kErrorCells))),
-                       dim3(kBlock), 0, st, m->dev.n_species, n_cells, y,
-                       ynew, yerr, atol, rtol, error);
-    HIP_TRY(hipGetLastError());
-    return MICM_HIP_OK;
+    const int64_t n = m->dev.n_species;
+    return for_slices(all_cells, kBlock / kErrorCells, [&](int64_t c0, int64_t n_cells) -> int {
+      hipLaunchKernelGGL(k_normalized_error, dim3(static_cast<unsigned>(n_groups_of(n_cells) * (kGroup / kErrorCells))),
+                         dim3(kBlock), 0, st, m->dev.n_species, n_cells, y + c0 * n, ynew + c0 * n, yerr + c0 * n, atol,
+                         rtol, error + c0);
+      HIP_TRY(hipGetLastError());
+      return MICM_HIP_OK;
+    });
   }
+
   int micm_hip_normalized_error_state(const micm_hip_mechanism* m, int64_t n_cells, const double* y,
                                       const double* ynew, const double* errors, const double* atol, double rtol,
                                       int64_t vector_length, double* error, void* stream)

@@ -14,3 +14,18 @@ extern "C" int lu_tile_cells_host(int64_t doubles_per_cell, int64_t lds_limit)
 {
   return lu_tile_cells(static_cast<std::size_t>(doubles_per_cell), static_cast<std::size_t>(lds_limit));
 }
+
+// The slices of n_cells cells as (first, cells) pairs; their number, or -1 past `most` of them.
+extern "C" int64_t slices_host(int64_t n_cells, int64_t threads_per_cell, int64_t* out, int64_t most)
+{
+  int64_t n = 0;
+  const int rc = for_slices(n_cells, threads_per_cell, [&](int64_t first, int64_t cells) {
+    if (n == most)
+      return 1;
+    out[2 * n] = first;
+    out[2 * n + 1] = cells;
+    ++n;
+    return 0;
+  });
+  return rc ? -1 : n;
+}

@@ -18,6 +18,8 @@ def lib(tmp_path_factory):
     lib = ctypes.CDLL(out)
     for name in ("tile_cells_host", "tile_cells_host"):
         getattr(lib, name).argtypes = [ctypes.c_int64, ctypes.c_int64]
+    lib.slices_host.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.POINTER(ctypes.c_int64), ctypes.c_int64]
+    lib.slices_host.restype = ctypes.c_int64
     return lib
 
 
@@ -33,3 +35,25 @@ def test_a_tile_has_a_kernel_of_its_size(lib, kernel, rule, limit):
         assert tc == 0 or tc in built, (doubles, tc)
         assert (tc == 0) == (doubles * 8 > limit), (doubles, tc)
         assert tc <= 1 or 2 * doubles * tc * 8 <= limit, (doubles, tc)
+
+
+@pytest.mark.parametrize("threads", [1, 3, 16, 20, 210, 256, 511, 1 << 20])
+@pytest.mark.parametrize("cells", [0, 1, 64, 513, 1 << 22, (1 << 28) + 37, (1 << 32) + 1])
+def test_slices_cover_the_cells_and_fit_a_launch(lib, cells, threads):
+    """Each cell is in one slice, slices start at whole groups for every XCD, and a slice's threads,
+    rounded up to such groups, are fewer than the 2^32 that a launch takes."""
+    if cells * threads > 1 << 40:
+        pytest.skip("more slices than any memory holds cells for")
+    most = 4096
+    out = (ctypes.c_int64 * (2 * most))()
+    n = lib.slices_host(cells, threads, out, most)
+    assert n >= 0
+    at = 0
+    for q in range(n):
+        first, count = out[2 * q], out[2 * q + 1]
+        assert first == at and count > 0 and first % 512 == 0
+        assert (count + 511) // 512 * 512 * threads < 1 << 32
+        at += count
+    assert at == cells
+    if cells * threads <= 1 << 30:
+        assert n == min(cells, 1)  # ordinary calls stay one launch
