@@ -53,4 +53,26 @@ namespace micm_hip
         return rc;
     return 0;
   }
+
+  // Results of one cell on the host: seven counters, the final time and the status.
+  constexpr std::size_t kResultBytes = 7 * sizeof(int64_t) + sizeof(double) + sizeof(int32_t);
+  constexpr std::size_t kStagingMost = 256 * 1024;
+
+  // Pinned memory of a State for its copies to the host: the largest of the results, the
+  // variables and the rate constants (the latter two in whole groups of 64 cells) that is at most
+  // kStagingMost and no larger than the results or the variables; 0 where none is, so that a
+  // State of many cells has none.  Larger copies gain little by it: their time is the transfer's.
+  constexpr std::size_t staging_bytes(int64_t n_cells, int64_t n_species, int64_t n_reactions)
+  {
+    const std::size_t cells = static_cast<std::size_t>(n_cells), padded = (cells + 63) / 64 * 64;
+    const std::size_t results = cells * kResultBytes;
+    const std::size_t variables = padded * sizeof(double) * static_cast<std::size_t>(n_species);
+    const std::size_t rates = padded * sizeof(double) * static_cast<std::size_t>(n_reactions);
+    const std::size_t most = std::min(kStagingMost, std::max(results, variables));
+    std::size_t bytes = 0;
+    for (std::size_t copy : { results, variables, rates })
+      if (copy <= most)
+        bytes = std::max(bytes, copy);
+    return bytes;
+  }
 }  // namespace micm_hip

@@ -3296,12 +3296,14 @@ extern "C"
     HIP_TRY(hipMalloc(&s->coop_next, sizeof(int)));
     HIP_TRY(hipMalloc(&s->order_bins, sizeof(int) * (kOrderBins + 1)));
     HIP_TRY(hipHostMalloc(&s->host_active, sizeof(unsigned int)));
-    constexpr size_t kStagingMost = 256 * 1024;
-    const size_t per_cell = std::max<size_t>(sizeof(int64_t) * 7 + sizeof(double) + sizeof(int32_t),
-                                             sizeof(double) * std::max(d.n_species, 3));
-    s->staging_bytes = std::min(kStagingMost, static_cast<size_t>(s->n_groups) * kGroup * per_cell);
-    if (s->staging_bytes > 0)
-      HIP_TRY(hipHostMalloc(&s->staging, s->staging_bytes));
+    s->staging_bytes = staging_bytes(n_cells, d.n_species, d.n_reactions);
+    if (s->staging_bytes > 0 && hipHostMalloc(&s->staging, s->staging_bytes) != hipSuccess)
+    {
+      // without it the copies go to pageable memory
+      (void)hipGetLastError();
+      s->staging = nullptr;
+      s->staging_bytes = 0;
+    }
     HIP_TRY(hipMemcpy(s->atol, m->t.absolute_tolerances.data(), sizeof(double) * d.n_species, hipMemcpyHostToDevice));
     *out = s.release();
     return MICM_HIP_OK;

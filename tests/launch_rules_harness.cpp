@@ -29,3 +29,8 @@ extern "C" int64_t slices_host(int64_t n_cells, int64_t threads_per_cell, int64_
   });
   return rc ? -1 : n;
 }
+
+extern "C" int64_t staging_bytes_host(int64_t n_cells, int64_t n_species, int64_t n_reactions)
+{
+  return static_cast<int64_t>(staging_bytes(n_cells, n_species, n_reactions));
+}

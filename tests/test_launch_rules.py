@@ -19,6 +19,8 @@ def lib(tmp_path_factory):
     for name in ("tile_cells_host", "tile_cells_host"):
         getattr(lib, name).argtypes = [ctypes.c_int64, ctypes.c_int64]
     lib.slices_host.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.POINTER(ctypes.c_int64), ctypes.c_int64]
+    lib.staging_bytes_host.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
+    lib.staging_bytes_host.restype = ctypes.c_int64
     lib.slices_host.restype = ctypes.c_int64
     return lib
 
@@ -57,3 +59,15 @@ def test_slices_cover_the_cells_and_fit_a_launch(lib, cells, threads):
     assert at == cells
     if cells * threads <= 1 << 30:
         assert n == min(cells, 1)  # ordinary calls stay one launch
+
+
+@pytest.mark.parametrize("species,reactions", [(1, 0), (3, 2), (9, 70), (20, 50), (60, 200), (210, 560), (5000, 1)])
+def test_pinned_memory_of_a_state_is_what_a_copy_of_it_uses(lib, species, reactions):
+    """No pinned byte that no copy to the host reaches, at most 256 KiB, and pinned memory for the
+    results and the variables wherever they fit that."""
+    for cells in (1, 2, 63, 64, 65, 400, 1000, 3855, 3856, 4096, 10000, 100000, 1 << 28):
+        padded = (cells + 63) // 64 * 64
+        copies = [68 * cells, 8 * padded * species, 8 * padded * reactions]
+        got = lib.staging_bytes_host(cells, species, reactions)
+        assert got <= 256 * 1024 and (got == 0 or got in copies)
+        assert all(got >= c for c in copies[:2] if c <= 256 * 1024)
