@@ -314,21 +314,36 @@ int micm_hip_state_set_handoff(micm_hip_state* state, int64_t steps);
  * threads and 16 to 256 species the compact layout is the kernel that takes the factor's last
  * rows as a dense block, which the library's choice of staging (-1) also picks for 256 threads or
  * its own choice of threads; 5 / 6 / 7: that kernel built for three waves per SIMD (168
- * registers) / two (256) / two, 4 leaving the choice to the occupancy.  With the library's choice
- * of staging (-1), mechanisms of at most eight species run one cell per lane whatever the threads
- * (recorded Solves excepted).  A tuning knob in the role of the vector length L of the reference's GPU policies
- * (cuda_solver_builder.hpp:24-38); results do not depend on it. */
+ * registers) / two (256) / two, 4 leaving the choice to the occupancy; for other numbers of
+ * species and threads 5, 6 and 7 are the same as 4.  With the library's choice of staging (-1),
+ * mechanisms of at most eight species run one cell per lane whatever the threads (recorded
+ * Solves excepted).  A tuning knob in the role of the vector length L of the reference's GPU
+ * policies (cuda_solver_builder.hpp:24-38); results do not depend on it. */
 int micm_hip_state_set_cooperative_shape(micm_hip_state* state, int32_t threads, int32_t stage);
 /* Blocking of the cooperative form's LU level schedule: the shortest run of products an
  * element's ordered sum (lu_decomposition_doolittle.inl:325-403) is split into, except its
  * last -- 1, 2, 4 or 8; -1 keeps every sum whole; 0: the library's default (4).  Every
  * blocking subtracts the same products in the same order; it only moves where a sum is
- * split between the levels of the schedule.  A tuning knob (the autotuner's "LU schedule
+ * split between the levels of the schedule.  It has no effect where no such schedule runs: the
+ * kernels with the dense block and with one cell per lane (MICM_HIP_KERNEL_BLOCK, _LANE), so by
+ * default for 16 to 256 species and for the smallest mechanisms.  A tuning knob (the autotuner's "LU schedule
  * blocking"); results do not depend on it. */
 int micm_hip_state_set_lu_blocking(micm_hip_state* state, int32_t min_segment);
 /* Whether the cooperative form fits this mechanism on the current device (its
  * per-cell working set must fit one workgroup's LDS); *out = 1 or 0. */
 int micm_hip_mechanism_cooperative_supported(const micm_hip_mechanism* mechanism, int32_t stages, int32_t* out);
+/* What a Solve (not a recorded one) in the cooperative form launches on the current device for a
+ * shape as micm_hip_state_set_cooperative_shape takes it: out[0] the kernel (MICM_HIP_KERNEL_*),
+ * out[1] its threads per cell, out[2] the tables it stages, out[3] the waves per SIMD that it is
+ * built for where there are several builds, else 0.  Shapes with the same four are one launch,
+ * so a tuner need not time both. */
+#define MICM_HIP_KERNEL_NONE 0    /* the form does not fit the mechanism */
+#define MICM_HIP_KERNEL_LEVELS 1  /* level schedules */
+#define MICM_HIP_KERNEL_COMPACT 2 /* level schedules, compact per-cell layout */
+#define MICM_HIP_KERNEL_BLOCK 3   /* the factor's last rows as a dense block */
+#define MICM_HIP_KERNEL_LANE 4    /* one cell per lane */
+int micm_hip_mechanism_cooperative_kernel(const micm_hip_mechanism* mechanism, int32_t stages, int32_t threads,
+                                          int32_t stage, int32_t* out);
 
 /* Solver::UpdateStateParameters (solver.hpp:217-247) on the device. */
 int micm_hip_update_state_parameters(const micm_hip_mechanism* mechanism, micm_hip_state* state);

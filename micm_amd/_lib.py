@@ -18,6 +18,7 @@ OK = 0
 STATE_NAMES = {0: "NotYetCalled", 1: "Running", 2: "Converged", 3: "ConvergenceExceededMaxSteps",
                4: "StepSizeTooSmall", 5: "RepeatedlySingularMatrix", 6: "NaNDetected", 7: "InfDetected"}
 SOLVE_LOCKSTEP, SOLVE_PLAIN, SOLVE_PERSISTENT, SOLVE_COOPERATIVE = 0, 1, 2, 3
+KERNEL_NONE, KERNEL_LEVELS, KERNEL_COMPACT, KERNEL_BLOCK, KERNEL_LANE = 0, 1, 2, 3, 4
 SOLVE_UPDATE_RATES = 0x100  # OR-ed into a form: UpdateStateParameters fused into the Solve launch
 PRESETS = {2: 2, 3: 3, 4: 4, "4da": 41, "6da": 61, 41: 41, 61: 61}
 
@@ -97,6 +98,7 @@ _SIGNATURES = {
     "micm_hip_packed_set_stream": [_vp, _vp],
     "micm_hip_packed_destroy": [_vp],
     "micm_hip_mechanism_cooperative_supported": [_vp, ctypes.c_int32, _i32p],
+    "micm_hip_mechanism_cooperative_kernel": [_vp, _i32, _i32, _i32, _i32p],
     "micm_hip_update_state_parameters": [_vp, _vp],
     "micm_hip_solve": [_vp, _vp, ctypes.c_double, ctypes.POINTER(RosenbrockParameters), ctypes.c_int32],
     "micm_hip_normalized_error_state": [_vp, _i64, _vp, _vp, _vp, _vp, ctypes.c_double, _i64, _vp, _vp],
@@ -275,6 +277,13 @@ class Mechanism:
         out = ctypes.c_int32(0)
         check(lib().micm_hip_mechanism_cooperative_supported(self.h, int(stages), ctypes.byref(out)))
         return bool(out.value)
+
+    def cooperative_kernel(self, stages, threads=0, stage=-1):
+        """(KERNEL_*, threads per cell, staged tables, waves per SIMD) that a Solve in the cooperative
+        form launches for a shape (micm_hip_mechanism_cooperative_kernel)."""
+        out = (ctypes.c_int32 * 4)()
+        check(lib().micm_hip_mechanism_cooperative_kernel(self.h, int(stages), int(threads), int(stage), out))
+        return tuple(out)
 
     def normalized_error(self, n_cells, y, ynew, yerr, atol, rtol, error, stream=None):
         check(lib().micm_hip_normalized_error(self.h, n_cells, y, ynew, yerr, atol, float(rtol), error, stream))

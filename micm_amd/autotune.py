@@ -19,17 +19,17 @@ import numpy as np
 
 from . import _lib
 
-# (label, form, handoff steps, cooperative threads, staging); the shapes that are
-# usually fast come first, so that the pilot can give up on slow ones early
 # the same shape built with the larger register budget
 WIDER_BUILD = {"cooperative256-compact-w3": "cooperative256-compact-w2"}
 
+# (label, form, handoff steps, cooperative threads, staging); the shapes that are
+# usually fast come first, so that the pilot can give up on slow ones early
 CANDIDATES = (
     ("cooperative128", _lib.SOLVE_COOPERATIVE, -1, 128, -1),
     ("cooperative256", _lib.SOLVE_COOPERATIVE, -1, 256, -1),
     ("cooperative64", _lib.SOLVE_COOPERATIVE, -1, 64, -1),
     ("cooperative512", _lib.SOLVE_COOPERATIVE, -1, 512, -1),
-    # the compact layout's register budgets: three waves per SIMD (168 registers) or two (256)
+    # the dense-block kernel's register budgets: three waves per SIMD (168 registers) or two (256)
     ("cooperative256-compact-w3", _lib.SOLVE_COOPERATIVE, -1, 256, 5),
     ("cooperative256-compact-w2", _lib.SOLVE_COOPERATIVE, -1, 256, 6),
     ("cooperative64-global-tables", _lib.SOLVE_COOPERATIVE, -1, 64, 0),
@@ -60,6 +60,34 @@ def apply(state, choice):
     state.set_cooperative_shape(choice["threads"], choice["stage"])
     state.set_lu_blocking(choice.get("lu_blocking", 0))
     return choice["form"]
+
+
+def _kernel(mech, stages, candidate):
+    """What a candidate's cooperative launch runs (DeviceState.set_cooperative_shape's shapes often
+    share one kernel); the candidate itself for a mechanism that cannot say."""
+    query = getattr(mech, "cooperative_kernel", None)
+    return candidate if query is None else query(stages, candidate[3], candidate[4])
+
+
+def _distinct(mech, stages, candidates):
+    """The candidates that launch different things, the first of each, and label -> label kept for
+    the others."""
+    kept, first, same = [], {}, {}
+    for c in candidates:
+        if c[1] == _lib.SOLVE_COOPERATIVE:
+            k = _kernel(mech, stages, c)
+            if k in first:
+                same[c[0]] = first[k]
+                continue
+            first[k] = c[0]
+        kept.append(c)
+    return kept, same
+
+
+def _has_lu_schedule(mech, stages, candidate):
+    """Whether the LU blocking changes anything for a cooperative candidate."""
+    kernel = _kernel(mech, stages, candidate)
+    return kernel is candidate or kernel[0] in (_lib.KERNEL_LEVELS, _lib.KERNEL_COMPACT)
 
 
 def _time_candidates(mech, y, k, dt, params, candidates, repeats, verbose, give_up=None, lu_blocking=0):
@@ -105,14 +133,17 @@ def autotune(mech, state, dt, params, sample=65536, first_sample=2048, pilot=256
     candidate reached), handoff_to (the cooperative candidate a persistent choice hands its
     slow cells to), lu_blocking (micm_hip_state_set_lu_blocking, for the fastest
     cooperative shape of the last sample; 0 keeps the default) and lu_blocking_seconds
-    (first-sample times of that shape with each blocking)."""
+    (first-sample times of that shape with each blocking).  Of candidates that launch the same
+    kernel only the first is timed, and blockings only for a kernel that has the LU schedule."""
     n = state.n_cells
     m = min(sample, n)
     key = _key(mech, params.stages, dt, m)
     if key in _cache:
         return dict(_cache[key])
     supported = mech.cooperative_supported(params.stages)
-    cands = [c for c in candidates if c[1] != _lib.SOLVE_COOPERATIVE or supported]
+    cands, same = _distinct(mech, params.stages,
+                            [c for c in candidates if c[1] != _lib.SOLVE_COOPERATIVE or supported])
+    wider_build = {same.get(c, c): same.get(w, w) for c, w in WIDER_BUILD.items()}
     y_all = state.get_variables()
     k_all = state.get_rate_constants()
 
@@ -166,7 +197,7 @@ def autotune(mech, state, dt, params, sample=65536, first_sample=2048, pilot=256
         # finalist's build with the larger register budget stays in beside it (the last pick
         # prefers it on a near tie)
         top = ranked[:finalists]
-        wider = [c for c in ranked[finalists:] if c[0] in {WIDER_BUILD.get(f[0]) for f in top}]
+        wider = [c for c in ranked[finalists:] if c[0] in {wider_build.get(f[0]) for f in top}]
         cands = top + wider + [c for c in ranked[finalists:]
                                if c[1] == _lib.SOLVE_PLAIN and times[c[0]] <= 2.0 * best1 and c not in wider]
     first_times = dict(times)
@@ -176,7 +207,7 @@ def autotune(mech, state, dt, params, sample=65536, first_sample=2048, pilot=256
     # on the first sample; a blocking that is 2 % faster there is timed on the last sample too
     # and taken if it is faster there as well
     coop = sorted((c for c in cands if c[1] == _lib.SOLVE_COOPERATIVE and c[0] in times), key=lambda c: times[c[0]])
-    if coop and m1 > m0 and coop[0][0] in first_times:
+    if coop and m1 > m0 and coop[0][0] in first_times and _has_lu_schedule(mech, params.stages, coop[0]):
         top = coop[0]
         base = first_times[top[0]]
         best_t, best_b = base, 0
@@ -202,8 +233,10 @@ def autotune(mech, state, dt, params, sample=65536, first_sample=2048, pilot=256
     cands = [c for c in last if c[0] in times]
     win = min(cands, key=lambda c: times[c[0]])
     # a build bounded to fewer registers wins only by more than 1 %: its extra waves per
-    # SIMD help only where LDS holds that many cells per CU, and its spills cost HBM traffic
-    wider = {c[0]: c for c in cands}.get(WIDER_BUILD.get(win[0]))
+    # SIMD help only where LDS holds that many cells per CU (60/200, 65,536 cells: 129 ms
+    # against 180 with two waves); elsewhere it spills 45 vector registers for the same time
+    # (210/560: within 0.7 % of two waves from 256 to 65,536 cells)
+    wider = {c[0]: c for c in cands}.get(wider_build.get(win[0]))
     if wider is not None and times[wider[0]] <= 1.01 * times[win[0]]:
         win = wider
     label, form, handoff, threads, stage = win

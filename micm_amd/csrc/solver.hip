@@ -2611,16 +2611,29 @@ namespace
     return MICM_HIP_OK;
   }
 
+  int check_cooperative_shape(int32_t threads, int32_t stage)
+  {
+    if (threads != 0 && threads != 64 && threads != 128 && threads != 256 && threads != 512 && threads != 1024)
+      return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "threads per cell must be 0, 64, 128, 256, 512 or 1024");
+    if (stage < -1 || stage > 7)
+      return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "stage must be -1 .. 7");
+    return MICM_HIP_OK;
+  }
+
   // LDS of the one-lane-per-cell kernel where a Solve's cells take it, else 0: at most eight
   // species, the library's choice of layout (stage < 0; the threads per cell have nothing to do
   // in a mechanism of this size), no recording.
   // README system, whole Solves with their transfers, against a workgroup per cell: 1 cell 254 ->
   // 177 us, 1,000 cells 331 -> 213, 10,000 cells 1,147 -> 200, 100,000 cells 9.9 -> 0.62 ms; against
   // the persistent form 446 -> 176 us, 753 -> 200 us (10,000), 3.4 -> 0.62 ms (100,000).
+  size_t tiny_solve_lds(const micm_hip_mechanism* m, int stages, int stage_request)
+  {
+    return stage_request < 0 ? tiny_lds(m->dev, m->coop, m->tiny, stages) : 0;
+  }
+
   size_t tiny_solve_lds(const micm_hip_state* s, int stages)
   {
-    return s->coop_stage < 0 && !s->recording.records ? tiny_lds(s->mech->dev, s->mech->coop, s->mech->tiny, stages)
-                                                   : 0;
+    return s->recording.records ? 0 : tiny_solve_lds(s->mech, stages, s->coop_stage);
   }
 
   TinyArgs tiny_args(micm_hip_state* s, const DevParams& p)
@@ -3459,10 +3472,8 @@ extern "C"
   {
     if (!s)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null state");
-    if (threads != 0 && threads != 64 && threads != 128 && threads != 256 && threads != 512 && threads != 1024)
-      return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "threads per cell must be 0, 64, 128, 256, 512 or 1024");
-    if (stage < -1 || stage > 7)
-      return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "stage must be -1 .. 7");
+    if (int rc = check_cooperative_shape(threads, stage))
+      return rc;
     s->coop_threads = threads;
     s->coop_stage = stage;
     return MICM_HIP_OK;
@@ -3485,6 +3496,31 @@ extern "C"
     if (!out || stages < 1 || stages > 6)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "bad argument");
     *out = coop_lds_bytes(m, stages) > 0 ? 1 : 0;
+    return MICM_HIP_OK;
+  }
+
+  int micm_hip_mechanism_cooperative_kernel(const micm_hip_mechanism* m, int32_t stages, int32_t threads, int32_t stage,
+                                            int32_t* out)
+  {
+    if (int rc = check_device_mech(m))
+      return rc;
+    if (!out || stages < 1 || stages > 6)
+      return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "bad argument");
+    if (int rc = check_cooperative_shape(threads, stage))
+      return rc;
+    std::fill(out, out + 4, 0);
+    if (tiny_solve_lds(m, stages, stage) > 0)
+    {
+      out[0] = MICM_HIP_KERNEL_LANE;
+      return MICM_HIP_OK;
+    }
+    const CoopPlan plan = plan_coop(m, stages, stage, threads);
+    if (plan.lds == 0)
+      return MICM_HIP_OK;
+    out[0] = plan.tail ? MICM_HIP_KERNEL_BLOCK : plan.compact ? MICM_HIP_KERNEL_COMPACT : MICM_HIP_KERNEL_LEVELS;
+    out[1] = plan.threads;
+    out[2] = plan.stage;
+    out[3] = plan.min_waves;
     return MICM_HIP_OK;
   }
 
