@@ -313,7 +313,9 @@ int micm_hip_state_set_handoff(micm_hip_state* state, int64_t steps);
  * needs more than 64 threads and at least one thread per species, else ignored).  With 256
  * threads and 16 to 256 species the compact layout is the kernel that takes the factor's last
  * rows as a dense block, which the library's choice of staging (-1) also picks for 256 threads or
- * its own choice of threads; 5 / 6 / 7: that kernel built for three waves per SIMD (168
+ * its own choice of threads (one wavefront for factors of at most 700 entries over 90,112 cells
+ * or more; with cells that all take few attempts 64 threads are faster than the block from 2,000
+ * cells on for such factors); 5 / 6 / 7: that kernel built for three waves per SIMD (168
  * registers) / two (256) / two, 4 leaving the choice to the occupancy; for other numbers of
  * species and threads 5, 6 and 7 are the same as 4.  With the library's choice of staging (-1),
  * mechanisms of at most eight species run one cell per lane whatever the threads (recorded
@@ -332,8 +334,8 @@ int micm_hip_state_set_lu_blocking(micm_hip_state* state, int32_t min_segment);
 /* Whether the cooperative form fits this mechanism on the current device (its
  * per-cell working set must fit one workgroup's LDS); *out = 1 or 0. */
 int micm_hip_mechanism_cooperative_supported(const micm_hip_mechanism* mechanism, int32_t stages, int32_t* out);
-/* What a Solve (not a recorded one) in the cooperative form launches on the current device for a
- * shape as micm_hip_state_set_cooperative_shape takes it: out[0] the kernel (MICM_HIP_KERNEL_*),
+/* What a Solve (not a recorded one) in the cooperative form of n_cells cells launches on the
+ * current device for a shape as micm_hip_state_set_cooperative_shape takes it: out[0] the kernel (MICM_HIP_KERNEL_*),
  * out[1] its threads per cell, out[2] the tables it stages, out[3] the waves per SIMD that it is
  * built for where there are several builds, else 0.  Shapes with the same four are one launch,
  * so a tuner need not time both. */
@@ -342,8 +344,8 @@ int micm_hip_mechanism_cooperative_supported(const micm_hip_mechanism* mechanism
 #define MICM_HIP_KERNEL_COMPACT 2 /* level schedules, compact per-cell layout */
 #define MICM_HIP_KERNEL_BLOCK 3   /* the factor's last rows as a dense block */
 #define MICM_HIP_KERNEL_LANE 4    /* one cell per lane */
-int micm_hip_mechanism_cooperative_kernel(const micm_hip_mechanism* mechanism, int32_t stages, int32_t threads,
-                                          int32_t stage, int32_t* out);
+int micm_hip_mechanism_cooperative_kernel(const micm_hip_mechanism* mechanism, int64_t n_cells, int32_t stages,
+                                          int32_t threads, int32_t stage, int32_t* out);
 
 /* Solver::UpdateStateParameters (solver.hpp:217-247) on the device. */
 int micm_hip_update_state_parameters(const micm_hip_mechanism* mechanism, micm_hip_state* state);

@@ -98,7 +98,7 @@ _SIGNATURES = {
     "micm_hip_packed_set_stream": [_vp, _vp],
     "micm_hip_packed_destroy": [_vp],
     "micm_hip_mechanism_cooperative_supported": [_vp, ctypes.c_int32, _i32p],
-    "micm_hip_mechanism_cooperative_kernel": [_vp, _i32, _i32, _i32, _i32p],
+    "micm_hip_mechanism_cooperative_kernel": [_vp, _i64, _i32, _i32, _i32, _i32p],
     "micm_hip_update_state_parameters": [_vp, _vp],
     "micm_hip_solve": [_vp, _vp, ctypes.c_double, ctypes.POINTER(RosenbrockParameters), ctypes.c_int32],
     "micm_hip_normalized_error_state": [_vp, _i64, _vp, _vp, _vp, _vp, ctypes.c_double, _i64, _vp, _vp],
@@ -278,11 +278,12 @@ class Mechanism:
         check(lib().micm_hip_mechanism_cooperative_supported(self.h, int(stages), ctypes.byref(out)))
         return bool(out.value)
 
-    def cooperative_kernel(self, stages, threads=0, stage=-1):
-        """(KERNEL_*, threads per cell, staged tables, waves per SIMD) that a Solve in the cooperative
-        form launches for a shape (micm_hip_mechanism_cooperative_kernel)."""
+    def cooperative_kernel(self, stages, threads=0, stage=-1, n_cells=1):
+        """(KERNEL_*, threads per cell, staged tables, waves per SIMD) that a Solve of n_cells cells in
+        the cooperative form launches for a shape (micm_hip_mechanism_cooperative_kernel)."""
         out = (ctypes.c_int32 * 4)()
-        check(lib().micm_hip_mechanism_cooperative_kernel(self.h, int(stages), int(threads), int(stage), out))
+        check(lib().micm_hip_mechanism_cooperative_kernel(self.h, int(n_cells), int(stages), int(threads), int(stage),
+                                                          out))
         return tuple(out)
 
     def normalized_error(self, n_cells, y, ynew, yerr, atol, rtol, error, stream=None):

@@ -2451,13 +2451,26 @@ namespace
   // CU, or take the compact layout when that fits more cells per CU; 4: the compact layout.
   //
   // threads_request 0 (with stage_request < 0): the kernel with the dense block where it takes
-  // the mechanism (16 to 256 species), else one wavefront.  The dense block beats one wavefront
-  // from the smallest such mechanism on: 20,000 cells of 20/50 in 28 ms instead of 44, 10,000
-  // of 30/90 in 33 instead of 74, of 60/200 in 47 instead of 148 (bound by their slowest
-  // cells); below 16 species one wavefront is faster than 256 threads (README system, 1,000
-  // cells: 0.23 ms against 0.37).
+  // the mechanism (16 to 256 species), else one wavefront, which also takes the Solves of
+  // factors of at most kWaveFactor entries over kWaveCells cells or more (n_cells; 0: those
+  // that another form hands on).
+  //
+  // A cell's attempt is shorter with the block, so Solves bound by their slowest cells gain from
+  // the smallest such mechanism on: 20,000 cells of 20/50 in 28 ms instead of 44, 10,000 of 30/90
+  // in 33 instead of 74, of 60/200 in 47 instead of 148.  One wavefront holds more cells of a
+  // small factor per CU, and in large numbers those are what counts (block / wavefront, ms):
+  // 16 species (131 entries) 65,536 cells 20 / 42, 200,000 60 / 47; 20 (165) 27 / 44, 82 / 50;
+  // 30 (327) 46 / 66, 140 / 110, 100,000 70 / 66; 40 (634) 63 / 88, 188 / 163, 100,000 94 / 88; from
+  // 45 species (849) on the block wins everywhere (400,000 cells 428 / 439, 60/200 496 / 1,033).
+  // Cells that all take few attempts (at most 40) reach that point at 2,000 cells already
+  // (8,000 cells of 16 species 2.4 / 2.0 ms, of 20 3.2 / 2.0, of 40 4.2 / 3.8): a caller with such
+  // cells asks for 64 threads.  Below 16 species one wavefront is faster than 256 threads
+  // (12 species, 50,000 cells: 38 ms against 42).
+  constexpr int64_t kWaveFactor = 700;
+  constexpr int64_t kWaveCells = 90112;
+
   CoopPlan plan_coop(const micm_hip_mechanism* m, int stages, int stage_request = -1, int threads_request = 0,
-                     int lu_blocking = 0)
+                     int lu_blocking = 0, int64_t n_cells = 0)
   {
     // 4: the compact layout, its register budget chosen by occupancy; 5 / 6 / 7: the compact
     // layout built for three / two waves per SIMD / without a register bound (256 threads)
@@ -2467,7 +2480,8 @@ namespace
       return plan;
     if (threads_request == 0 && stage_request < 0 && plan.lds > 0)
     {
-      (void)plan_tail(m, stage_request, plan);
+      if (m->coop.nnz_alu > kWaveFactor || n_cells < kWaveCells)
+        (void)plan_tail(m, stage_request, plan);
       return plan;
     }
     // the compact layout keeps one species per thread in registers and publishes the
@@ -2623,6 +2637,12 @@ namespace
     return MICM_HIP_OK;
   }
 
+  // The plan of a State's Solve in the cooperative form, or of the cells handed on to that form.
+  CoopPlan plan_solve(const micm_hip_state* s, int stages, bool handed_on)
+  {
+    return plan_coop(s->mech, stages, s->coop_stage, s->coop_threads, s->lu_blocking, handed_on ? 0 : s->n_cells);
+  }
+
   int check_cooperative_shape(int32_t threads, int32_t stage)
   {
     if (threads != 0 && threads != 64 && threads != 128 && threads != 256 && threads != 512 && threads != 1024)
@@ -2699,7 +2719,7 @@ namespace
       HIP_TRY(tiny_solve(a, lds, st));
       return MICM_HIP_OK;
     }
-    const CoopPlan plan = plan_coop(s->mech, p.stages, s->coop_stage, s->coop_threads, s->lu_blocking);
+    const CoopPlan plan = plan_solve(s, p.stages, resume != nullptr);
     if (plan.lds == 0)
       return fail(MICM_HIP_ERR_UNSUPPORTED, "the cooperative form does not fit this mechanism in LDS");
     if (plan.tail)
@@ -2733,27 +2753,34 @@ namespace
   // Whether a persistent Solve with the library's hand-off runs every cell in the cooperative
   // form from its first attempt: with the dense block an attempt costs the cooperative form
   // less than the per-lane form, whose lanes wait for each other's memory, except for small
-  // factors in numbers that fill the chip's lanes (64 lanes x 4 SIMDs x 256 CUs).  60/200:
+  // factors in numbers that fill the chip's lanes (64 lanes x 4 SIMDs x 256 CUs) and for those
+  // that the cooperative form takes with one wavefront (plan_coop).  60/200:
   // 20,011 cells 55 ms against 195 (hand-off after 16 steps) and 351 (48), 120,000 cells 250
   // against 370 and 519; 210/560, 20,000 cells 394 against 1,424; 20/50: 10,000 cells 28
-  // against 41, 200,000 cells 97 against 67 ms.  With one cell per lane (tiny_solve_lds) always.
-  constexpr int64_t kPerLaneFactor = 300;
+  // against 41, 200,000 cells 97 against 67 ms.  Cells that all take few attempts, at once / after
+  // 16 steps: 30 species (327 entries) 32,768 cells 13.9 / 20.4, 65,536 27.7 / 24.9, 131,072 55 / 36;
+  // 40 (634) 65,536 cells 33 / 42, 90,112 46 / 53, 131,072 66 / 59.  With one cell per lane
+  // (tiny_solve_lds) always.
+  constexpr int64_t kPerLaneFactor = 350;
   constexpr int64_t kPerLaneCells = 65536;
   constexpr int64_t kHandoffBlock = 16, kHandoffLevels = 48;  // default hand-off steps
 
+  // plan: that of the cells handed on.
   bool hands_off_at_once(const micm_hip_state* s, const CoopPlan& plan, int stages)
   {
     if (s->handoff_steps >= 0)
       return false;
+    const int64_t factor = s->mech->coop.nnz_alu;
     return tiny_solve_lds(s, stages) > 0 ||
-           (plan.tail && (s->mech->coop.nnz_alu > kPerLaneFactor || s->n_cells < kPerLaneCells));
+           (plan.tail && (factor > kPerLaneFactor || s->n_cells < kPerLaneCells) &&
+            (factor > kWaveFactor || s->n_cells < kWaveCells));
   }
 
   int prepare_solve(micm_hip_state* s, int32_t form, int stages)
   {
     if (form == MICM_HIP_SOLVE_COOPERATIVE || form == MICM_HIP_SOLVE_PERSISTENT)
     {
-      const CoopPlan plan = plan_coop(s->mech, stages, s->coop_stage, s->coop_threads, s->lu_blocking);
+      const CoopPlan plan = plan_solve(s, stages, form == MICM_HIP_SOLVE_PERSISTENT);
       if (form == MICM_HIP_SOLVE_PERSISTENT && hands_off_at_once(s, plan, stages))
         form = MICM_HIP_SOLVE_COOPERATIVE;
       if (plan.compact)
@@ -2836,7 +2863,7 @@ namespace
   {
     const micm_hip_mechanism* m = s->mech;
     const DevMech& d = m->dev;
-    const CoopPlan plan = plan_coop(m, p.stages, s->coop_stage, s->coop_threads, s->lu_blocking);
+    const CoopPlan plan = plan_solve(s, p.stages, form == MICM_HIP_SOLVE_PERSISTENT);
     if (form == MICM_HIP_SOLVE_COOPERATIVE || hands_off_at_once(s, plan, p.stages))
       return s->has_order ? launch_coop(s, p, s->order, s->order_bins + kOrderBins, 0, nullptr, update_rates, st)
                           : launch_coop(s, p, nullptr, nullptr, s->n_cells, nullptr, update_rates, st);
@@ -3511,12 +3538,12 @@ extern "C"
     return MICM_HIP_OK;
   }
 
-  int micm_hip_mechanism_cooperative_kernel(const micm_hip_mechanism* m, int32_t stages, int32_t threads, int32_t stage,
-                                            int32_t* out)
+  int micm_hip_mechanism_cooperative_kernel(const micm_hip_mechanism* m, int64_t n_cells, int32_t stages, int32_t threads,
+                                            int32_t stage, int32_t* out)
   {
     if (int rc = check_device_mech(m))
       return rc;
-    if (!out || stages < 1 || stages > 6)
+    if (!out || n_cells < 1 || stages < 1 || stages > 6)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "bad argument");
     if (int rc = check_cooperative_shape(threads, stage))
       return rc;
@@ -3526,7 +3553,7 @@ extern "C"
       out[0] = MICM_HIP_KERNEL_LANE;
       return MICM_HIP_OK;
     }
-    const CoopPlan plan = plan_coop(m, stages, stage, threads);
+    const CoopPlan plan = plan_coop(m, stages, stage, threads, 0, n_cells);
     if (plan.lds == 0)
       return MICM_HIP_OK;
     out[0] = plan.tail ? MICM_HIP_KERNEL_BLOCK : plan.compact ? MICM_HIP_KERNEL_COMPACT : MICM_HIP_KERNEL_LEVELS;
@@ -3702,7 +3729,7 @@ extern "C"
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "flags: only MICM_HIP_SOLVE_UPDATE_RATES");
     if (params->stages < 1 || params->stages > 6)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "stages must be 1..6");
-    const CoopPlan plan = plan_coop(m, static_cast<int>(params->stages), s->coop_stage, s->coop_threads, s->lu_blocking);
+    const CoopPlan plan = plan_solve(s, static_cast<int>(params->stages), false);
     if (plan.lds == 0)
       return fail(MICM_HIP_ERR_UNSUPPORTED, "the cooperative form does not fit this mechanism in LDS");
     int64_t rows = 0;
@@ -3839,7 +3866,7 @@ extern "C"
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "flags: only MICM_HIP_SOLVE_UPDATE_RATES");
     if (params->stages < 1 || params->stages > 6)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "stages must be 1..6");
-    if (plan_coop(m, static_cast<int>(params->stages), s->coop_stage, s->coop_threads, s->lu_blocking).lds == 0)
+    if (plan_solve(s, static_cast<int>(params->stages), false).lds == 0)
       return fail(MICM_HIP_ERR_UNSUPPORTED, "recorded solves run the cooperative form, which does not fit this mechanism");
     const DevParams p = make_params(*params, time_step, s->rtol);
     if (int rc = prepare_solve(s, MICM_HIP_SOLVE_COOPERATIVE, p.stages))
