@@ -529,6 +529,40 @@ namespace
     }
   }
 
+  // Cells from which a thread per cell is the faster of the two kernels for alpha - J, and for the
+  // per-cell norm: from then on its loads alone keep memory busy, and it forms no addresses for
+  // one element each.  us, a thread per element (norm: sixteen a cell) / per cell:
+  //   alpha - J  20 species: 20,000 cells 4.1 / 5.6, 65,536 5.7 / 6.5, 131,072 8.5 / 8.1,
+  //              1,000,000 60 / 51; 60: 131,072 22 / 25, 200,000 31.5 / 30.1, 500,000 124 / 92; 210: 20,000 13 / 58,
+  //              131,072 111 / 127, 500,000 412 / 347
+  //   norm       20 species: 20,000 cells 5.1 / 6.3, 131,072 14.1 / 14.7, 200,000 19.3 / 16.5, 2,000,000
+  //              226 / 164; 60: 20,000 5.9 / 34, 200,000 49 / 65, 1,000,000 244 / 239; 210: 20,000 18 / 124,
+  //              500,000 434 / 432
+  // Below sixteen species a thread per cell is as fast or faster for any number (3 species, norm:
+  // 64 cells 4.9 / 4.0, 2,000,000 103 / 23).
+  constexpr int kFewSpecies = 16, kMoreSpecies = 30;
+
+  bool alpha_per_cell(int n_species, int64_t n_cells)
+  {
+    return n_species < kFewSpecies || n_cells >= (n_species < kMoreSpecies ? 98304 : 163840);
+  }
+
+  bool norm_per_cell(int n_species, int64_t n_cells)
+  {
+    return n_species < kFewSpecies || n_cells >= (n_species < kMoreSpecies ? 163840 : 327680);
+  }
+
+  __global__ void __launch_bounds__(kBlock) k_alpha_minus_jacobian_cells(DevMech m, int64_t n_cells,
+                                                                         double* __restrict__ jac, double alpha)
+  {
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (c >= n_cells)
+      return;
+    Lane J = lane_view(jac, c / kGroup, m.nnz_jac, c % kGroup);
+    for (int i = 0; i < m.n_species; ++i)
+      J[m.jac_diag[i]] += alpha * 1.0;
+  }
+
   // One thread per (diagonal element, cell): a thread per cell walking the diagonal leaves all
   // but n_cells lanes idle (210 species, 4,096 cells: 64 us).
   __global__ void __launch_bounds__(kBlock) k_alpha_minus_jacobian(DevMech m, int64_t n_cells, double* __restrict__ jac,
@@ -566,7 +600,26 @@ namespace
                     lane_view(const_cast<double*>(upper), g, m.nnz_upper, l), lane_view(x, g, m.n_species, l));
   }
 
-  // The per-cell norm (path.hpp, error_sum): a workgroup takes kErrorCells cells of a group, its
+  // The per-cell norm (path.hpp, error_sum), a thread per cell.
+  __global__ void __launch_bounds__(kBlock) k_normalized_error_cells(int n_species, int64_t n_cells,
+                                                                     const double* __restrict__ y,
+                                                                     const double* __restrict__ ynew,
+                                                                     const double* __restrict__ yerr,
+                                                                     const double* __restrict__ atol, double rtol,
+                                                                     double* __restrict__ err)
+  {
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (c >= n_cells)
+      return;
+    const size_t g = c / kGroup;
+    const int l = c % kGroup;
+    const double s = error_sum(n_species, lane_view(const_cast<double*>(y), g, n_species, l),
+                               lane_view(const_cast<double*>(ynew), g, n_species, l),
+                               lane_view(const_cast<double*>(yerr), g, n_species, l), atol, rtol);
+    err[c] = smax(sqrt(s / static_cast<double>(n_species > 0 ? n_species : 1)), 1.0e-10);
+  }
+
+  // The same with all lanes of few cells: a workgroup takes kErrorCells cells of a group, its
   // threads form the squares of kErrorSpecies species at a time into LDS, and one lane per cell
   // adds them in species order.  A thread per cell forming and adding its own terms leaves the
   // chip idle below 100,000 cells (210 species, 4,096 cells: 154 us).
@@ -3167,11 +3220,16 @@ extern "C"
     if (!jac)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
     const DevMech& d = m->dev;
-    return for_slices(all_cells, d.n_species, [&](int64_t c0, int64_t n_cells) -> int {
-      hipLaunchKernelGGL(k_alpha_minus_jacobian,
-                         dim3(static_cast<unsigned>(
-                             (n_groups_of(n_cells) * static_cast<int64_t>(d.n_species) * kGroup + kBlock - 1) / kBlock)),
-                         dim3(kBlock), 0, st, d, n_cells, jac + c0 * d.nnz_jac, alpha);
+    const bool per_cell = alpha_per_cell(d.n_species, all_cells);
+    return for_slices(all_cells, per_cell ? 1 : d.n_species, [&](int64_t c0, int64_t n_cells) -> int {
+      if (per_cell)
+        hipLaunchKernelGGL(k_alpha_minus_jacobian_cells, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, d, n_cells,
+                           jac + c0 * d.nnz_jac, alpha);
+      else
+        hipLaunchKernelGGL(k_alpha_minus_jacobian,
+                           dim3(static_cast<unsigned>(
+                               (n_groups_of(n_cells) * static_cast<int64_t>(d.n_species) * kGroup + kBlock - 1) / kBlock)),
+                           dim3(kBlock), 0, st, d, n_cells, jac + c0 * d.nnz_jac, alpha);
       HIP_TRY(hipGetLastError());
       return MICM_HIP_OK;
     });
@@ -3269,10 +3327,15 @@ extern "C"
     if (!y || !ynew || !yerr || !atol || !error)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
     const int64_t n = m->dev.n_species;
-    return for_slices(all_cells, kBlock / kErrorCells, [&](int64_t c0, int64_t n_cells) -> int {
-      hipLaunchKernelGGL(k_normalized_error, dim3(static_cast<unsigned>(n_groups_of(n_cells) * (kGroup / kErrorCells))),
-                         dim3(kBlock), 0, st, m->dev.n_species, n_cells, y + c0 * n, ynew + c0 * n, yerr + c0 * n, atol,
-                         rtol, error + c0);
+    const bool per_cell = norm_per_cell(m->dev.n_species, all_cells);
+    return for_slices(all_cells, per_cell ? 1 : kBlock / kErrorCells, [&](int64_t c0, int64_t n_cells) -> int {
+      const double *ys = y + c0 * n, *yn = ynew + c0 * n, *ye = yerr + c0 * n;
+      if (per_cell)
+        hipLaunchKernelGGL(k_normalized_error_cells, dim3(grid_for(n_cells)), dim3(kBlock), 0, st, m->dev.n_species,
+                           n_cells, ys, yn, ye, atol, rtol, error + c0);
+      else
+        hipLaunchKernelGGL(k_normalized_error, dim3(static_cast<unsigned>(n_groups_of(n_cells) * (kGroup / kErrorCells))),
+                           dim3(kBlock), 0, st, m->dev.n_species, n_cells, ys, yn, ye, atol, rtol, error + c0);
       HIP_TRY(hipGetLastError());
       return MICM_HIP_OK;
     });
