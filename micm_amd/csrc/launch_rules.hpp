@@ -58,20 +58,23 @@ namespace micm_hip
   constexpr std::size_t kResultBytes = 7 * sizeof(int64_t) + sizeof(double) + sizeof(int32_t);
   constexpr std::size_t kStagingMost = 256 * 1024;
 
-  // Pinned memory of a State for its copies to the host: the largest of the results, the
-  // variables and the rate constants (the latter two in whole groups of 64 cells) that is at most
-  // kStagingMost and no larger than the results or the variables; 0 where none is, so that a
-  // State of many cells has none.  Larger copies gain little by it: their time is the transfer's.
+  // Grouped arrays go through pinned memory below this size only: a copy to pageable memory takes
+  // 21 us up to 16 KiB and 11 from there on, and the host reads the pinned buffer more slowly
+  // (pageable / pinned, us: 10 KiB 21 / 13, 17 KiB 11.2 / 12.5, 80 KiB 15 / 22, 240 KiB 26 / 46).
+  constexpr std::size_t kStagingGrouped = 16 * 1024;
+
+  // Pinned memory of a State for its copies to the host: the largest of the results (three copies
+  // in one wait) up to kStagingMost and of the variables and the rate constants (in whole groups
+  // of 64 cells) below kStagingGrouped; 0 where none is, so that a State of many cells has none.
   constexpr std::size_t staging_bytes(int64_t n_cells, int64_t n_species, int64_t n_reactions)
   {
     const std::size_t cells = static_cast<std::size_t>(n_cells), padded = (cells + 63) / 64 * 64;
     const std::size_t results = cells * kResultBytes;
     const std::size_t variables = padded * sizeof(double) * static_cast<std::size_t>(n_species);
     const std::size_t rates = padded * sizeof(double) * static_cast<std::size_t>(n_reactions);
-    const std::size_t most = std::min(kStagingMost, std::max(results, variables));
-    std::size_t bytes = 0;
-    for (std::size_t copy : { results, variables, rates })
-      if (copy <= most)
+    std::size_t bytes = results <= kStagingMost ? results : 0;
+    for (std::size_t copy : { variables, rates })
+      if (copy < kStagingGrouped)
         bytes = std::max(bytes, copy);
     return bytes;
   }

@@ -1817,9 +1817,9 @@ struct micm_hip_state
   double* lockstep_error = nullptr;
   int* queue_next = nullptr;
   unsigned int* host_active = nullptr;  // pinned
-  // Pinned, for results that fit on their way to the host: a copy to pageable memory waits for
-  // itself, 15 to 25 us each (the results of 1,000 cells 80 -> 29 us, of one cell 46 -> 22, its
-  // concentrations 22 -> 14).  Copies to the device gain nothing by it.
+  // Pinned, for what fits on its way to the host (launch_rules.hpp, staging_bytes): a copy to
+  // pageable memory waits for itself (the results of 1,000 cells 54 -> 27 us, of one cell 45 -> 21,
+  // its concentrations 21 -> 13).  Copies to the device gain nothing by it.
   char* staging = nullptr;
   size_t staging_bytes = 0;
   mutable std::mutex staging_lock;
@@ -2037,11 +2037,16 @@ namespace
         out[(static_cast<size_t>(c / kGroup) * n_vals + v) * kGroup + c % kGroup] = host[c * n_vals + v];
   }
 
-  void grouped_to_host(const double* in, int64_t n_cells, int64_t n_vals, double* host)
+  // (out of line: inlined into its callers, the inner loop of a few values came out twice as slow)
+  __attribute__((noinline)) void grouped_to_host(const double* in, int64_t n_cells, int64_t n_vals, double* host)
   {
-    for (int64_t c = 0; c < n_cells; ++c)
-      for (int64_t v = 0; v < n_vals; ++v)
-        host[c * n_vals + v] = in[(static_cast<size_t>(c / kGroup) * n_vals + v) * kGroup + c % kGroup];
+    for (int64_t first = 0; first < n_cells; first += kGroup, in += kGroup * n_vals)
+    {
+      const int64_t cells = std::min<int64_t>(kGroup, n_cells - first);
+      for (int64_t l = 0; l < cells; ++l)
+        for (int64_t v = 0; v < n_vals; ++v)
+          *host++ = in[v * kGroup + l];
+    }
   }
 
   size_t grouped_doubles(const micm_hip_state* s, int64_t n_vals)
@@ -2069,7 +2074,7 @@ namespace
     if (n_vals == 0)
       return MICM_HIP_OK;
     const size_t count = static_cast<size_t>(s->n_groups) * n_vals * kGroup, bytes = count * sizeof(double);
-    if (bytes <= s->staging_bytes)
+    if (bytes < kStagingGrouped && bytes <= s->staging_bytes)
     {
       const std::lock_guard<std::mutex> lock(s->staging_lock);
       double* buf = reinterpret_cast<double*>(s->staging);
