@@ -20,17 +20,33 @@ namespace micm_hip
     return doubles_per_cell * sizeof(double) <= lds_limit ? 1 : 0;
   }
 
-  // The same for the LU kernel, which is built for tiles of 16 cells, 8 and 1 (kLuTiles): with
-  // 160 KB of LDS, factors whose tiles would have 4 or 2 cells (1,281 entries and more) take the
-  // kernel with the dense block, and those that cannot run one cell at a time.
-  constexpr int kLuTiles[] = { 16, 8, 1 };
-  constexpr int lu_tile_cells(std::size_t doubles_per_cell, std::size_t lds_limit)
+  // Whether the single-phase LU (substitution) takes the kernel with the factor's dense block, one
+  // cell per workgroup, rather than the tiled one.  Up to kTailCells cells, the workgroups that
+  // three to a CU hold at once, the block does: a tile of many cells leaves most CUs idle.  With
+  // more cells it does for factors of at least kTailFactor entries and kTailProducts products,
+  // whose work the block's rows hold; sparser ones gain by it only where a CU holds few of their
+  // tiles: the LU from 1,650 entries (tiles of four, two to a CU) and 2,048 cells on, the
+  // substitution from 1,280 entries and 3,600 products on.  LU / substitution, us, block against
+  // tiled:
+  //   16 species (131 entries), 768 cells 12.5 : 14.5 / 8.1 : 15.8, 1,500 cells 17.4 : 14.5 / 11.0 : 15.7;
+  //   20 (165), 768 cells 16.5 : 16.6 / 11.7 : 16.9; 50 (919), 1,500 41 : 51 / 34 : 52, 20,000 318 : 312 / 315 : 282
+  //   160 (1,252, 1,882 products), 1,500 48 : 47 / 42 : 37, 4,096 99 : 64 / 95 : 84
+  //   120 (1,417, 4,291), 1,500 54 : 47 / 41 : 49, 8,000 192 : 158 / 167 : 174
+  //   200 (1,697, 3,653), 1,500 56 : 46 / 48 : 60, 2,500 77 : 97 / 71 : 120
+  //   60/200 (1,304, 7,668), 1,500 45 : 54 / 36 : 69, 20,000 382 : 439 / 347 : 456
+  //   TS1 (2,381, 6,986), 4,096 122 : 163 / 105 : 222; 210/560 (8,548, 121,036), 4,096 545 : 1,665 / 341 : 1,303
+  constexpr int64_t kTailCells = 768, kTailFactor = 1200, kTailProducts = 6000;
+
+  constexpr bool lu_with_block(int64_t factor, int64_t products, int64_t n_cells)
   {
-    const int most = tile_cells(doubles_per_cell, lds_limit);
-    for (int tc : kLuTiles)
-      if (tc <= most)
-        return tc;
-    return 0;
+    return n_cells <= kTailCells || (factor >= kTailFactor && products >= kTailProducts) ||
+           (factor >= 1650 && n_cells > 2048);
+  }
+
+  constexpr bool substitution_with_block(int64_t factor, int64_t products, int64_t n_cells)
+  {
+    return n_cells <= kTailCells || (factor >= kTailFactor && products >= kTailProducts) ||
+           (factor >= 1280 && products >= 3600);
   }
 
   // A launch takes fewer than 2^32 threads; of more, HIP runs the number modulo 2^32 and reports

@@ -2355,31 +2355,10 @@ namespace
     return static_cast<size_t>(std::max(max_lds, optin)) - 64;  // static __shared__ of the kernel
   }
 
-  // tile_cells / lu_tile_cells (launch_rules.hpp) of a mechanism, 0 also where the level
-  // schedules are unavailable.
+  // tile_cells (launch_rules.hpp) of a mechanism, 0 also where the level schedules are unavailable.
   int tile_cells(const micm_hip_mechanism* m, size_t doubles_per_cell)
   {
     return m->t.coop_levels_ok ? micm_hip::tile_cells(doubles_per_cell, lds_limit()) : 0;
-  }
-
-  int lu_tile_cells(const micm_hip_mechanism* m)
-  {
-    return m->t.coop_levels_ok ? micm_hip::lu_tile_cells(static_cast<size_t>(m->coop.nnz_alu), lds_limit()) : 0;
-  }
-
-  // Whether the single-phase LU and substitution take the kernels with the factor's dense block
-  // (one cell per workgroup) rather than the tiled ones: for factors of at least kTailFactor
-  // entries, and for smaller ones below kTailCells cells, where a tile of many cells leaves most
-  // CUs idle.  LU, us, block / tiled: 210/560 (8,548 entries) 77 / 214 for 64 cells and 545 /
-  // 1,665 for 4,096; TS1 (2,381) 135 / 166, 60/200 (1,304) 98 / 118 for 4,096 and 433 / 440 for
-  // 20,000; 50 species (989) 32 / 55 for 1,000 and 374 / 359 for 20,000; 24 species (238) 19 / 23
-  // for 1,000 and 51 / 24 for 4,096.
-  constexpr int kTailFactor = 1200;
-  constexpr int64_t kTailCells = 768;
-
-  bool phases_with_tail(const micm_hip_mechanism* m, int64_t n_cells, size_t lds)
-  {
-    return m->tail.size > 0 && (m->coop.nnz_alu >= kTailFactor || n_cells <= kTailCells) && lds <= lds_limit();
   }
 
   // Cells per workgroup of the tiled forcing / Jacobian kernels: the largest power of two
@@ -3247,8 +3226,9 @@ extern "C"
     if (!jac || !lower || !upper)
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
     const DevMech& d = m->dev;
-    const int tc = lu_tile_cells(m);
-    const bool tail = phases_with_tail(m, all_cells, tail_factor_lds(m->tail));
+    const int tc = tile_cells(m, static_cast<size_t>(m->coop.nnz_alu));
+    const bool tail = m->tail.size > 0 && tail_factor_lds(m->tail) <= lds_limit() &&
+                      lu_with_block(m->coop.nnz_alu, m->t.lu_multiply_adds(), all_cells);
     const int64_t threads = tail ? kTailThreads : tc > 0 ? kTileThreads / tc : 1;
     return for_slices(all_cells, threads, [&](int64_t c0, int64_t n_cells) -> int {
       const double* js = jac + c0 * d.nnz_jac;
@@ -3265,6 +3245,8 @@ extern "C"
         {
           case 16: LAUNCH_TILED(k_lu_decompose_tiled<16>, blocks, lds, st, d, m->coop, n_cells, js, lo, up); break;
           case 8: LAUNCH_TILED(k_lu_decompose_tiled<8>, blocks, lds, st, d, m->coop, n_cells, js, lo, up); break;
+          case 4: LAUNCH_TILED(k_lu_decompose_tiled<4>, blocks, lds, st, d, m->coop, n_cells, js, lo, up); break;
+          case 2: LAUNCH_TILED(k_lu_decompose_tiled<2>, blocks, lds, st, d, m->coop, n_cells, js, lo, up); break;
           default: LAUNCH_TILED(k_lu_decompose_tiled<1>, blocks, lds, st, d, m->coop, n_cells, js, lo, up); break;
         }
       }
@@ -3285,7 +3267,8 @@ extern "C"
       return fail(MICM_HIP_ERR_INVALID_ARGUMENT, "null device pointer");
     const DevMech& d = m->dev;
     const int tc = tile_cells(m, static_cast<size_t>(m->coop.nnz_alu) + 2 * static_cast<size_t>(d.n_species));
-    const bool tail = phases_with_tail(m, all_cells, tail_solve_lds(d, m->tail));
+    const bool tail = m->tail.size > 0 && tail_solve_lds(d, m->tail) <= lds_limit() &&
+                      substitution_with_block(m->coop.nnz_alu, m->t.lu_multiply_adds(), all_cells);
     const int64_t threads = tail ? kTailThreads : tc > 0 ? kTileThreads / tc : 1;
     size_t lds = (static_cast<size_t>(m->coop.nnz_alu) + 2 * static_cast<size_t>(d.n_species)) * tc * sizeof(double);
     // one cell per workgroup: a product buffer for the two-phase back substitution

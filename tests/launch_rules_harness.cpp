@@ -10,9 +10,9 @@ extern "C" int tile_cells_host(int64_t doubles_per_cell, int64_t lds_limit)
   return tile_cells(static_cast<std::size_t>(doubles_per_cell), static_cast<std::size_t>(lds_limit));
 }
 
-extern "C" int lu_tile_cells_host(int64_t doubles_per_cell, int64_t lds_limit)
+extern "C" int with_block_host(int64_t factor, int64_t products, int64_t n_cells, int substitution)
 {
-  return lu_tile_cells(static_cast<std::size_t>(doubles_per_cell), static_cast<std::size_t>(lds_limit));
+  return substitution ? substitution_with_block(factor, products, n_cells) : lu_with_block(factor, products, n_cells);
 }
 
 // The slices of n_cells cells as (first, cells) pairs; their number, or -1 past `most` of them.

@@ -16,8 +16,8 @@ def lib(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", os.path.join(ROOT, "tests", "launch_rules_harness.cpp"),
                     "-o", out], check=True)
     lib = ctypes.CDLL(out)
-    for name in ("tile_cells_host", "tile_cells_host"):
-        getattr(lib, name).argtypes = [ctypes.c_int64, ctypes.c_int64]
+    lib.tile_cells_host.argtypes = [ctypes.c_int64, ctypes.c_int64]
+    lib.with_block_host.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
     lib.slices_host.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.POINTER(ctypes.c_int64), ctypes.c_int64]
     lib.staging_bytes_host.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
     lib.staging_bytes_host.restype = ctypes.c_int64
@@ -25,15 +25,14 @@ def lib(tmp_path_factory):
     return lib
 
 
-@pytest.mark.parametrize("kernel,rule", [("k_lu_decompose_tiled", "lu_tile_cells_host"),
-                                         ("k_lu_solve_tiled", "tile_cells_host")])
+@pytest.mark.parametrize("kernel", ["k_lu_decompose_tiled", "k_lu_solve_tiled"])
 @pytest.mark.parametrize("limit", [64 * 1024 - 64, 160 * 1024 - 64])
-def test_a_tile_has_a_kernel_of_its_size(lib, kernel, rule, limit):
+def test_a_tile_has_a_kernel_of_its_size(lib, kernel, limit):
     """The grid is sized for the tile that the rule gives, so the launch needs a kernel built for
     exactly that tile: with a smaller one, cells past its first would be left out."""
     built = {int(tc) for tc in re.findall(rf"LAUNCH_TILED\({kernel}<(\d+)>", open(SOLVER).read())}
     for doubles in range(1, 22000):
-        tc = getattr(lib, rule)(doubles, limit)
+        tc = lib.tile_cells_host(doubles, limit)
         assert tc == 0 or tc in built, (doubles, tc)
         assert (tc == 0) == (doubles * 8 > limit), (doubles, tc)
         assert tc <= 1 or 2 * doubles * tc * 8 <= limit, (doubles, tc)
@@ -70,3 +69,13 @@ def test_pinned_memory_of_a_state_is_what_a_copy_of_it_uses(lib, species, reacti
         got = lib.staging_bytes_host(cells, species, reactions)
         used = [c for c, most in zip(copies, (256 * 1024, 16 * 1024 - 1, 16 * 1024 - 1)) if c <= most]
         assert got == max(used, default=0)
+
+
+@pytest.mark.parametrize("factor,products,cells,lu,substitution", [
+    (131, 200, 768, True, True), (131, 200, 769, False, False), (1100, 9000, 5000, False, False),
+    (1304, 7668, 769, True, True), (2381, 6986, 20000, True, True), (8548, 121036, 4096, True, True),
+    (1252, 1882, 769, False, False), (1252, 1882, 100000, False, False), (1417, 4291, 8000, False, True),
+    (1697, 3653, 2048, False, True), (1697, 3653, 2049, True, True), (1700, 2000, 4000, True, False)])
+def test_dense_block_by_entries_products_and_cells(lib, factor, products, cells, lu, substitution):
+    assert bool(lib.with_block_host(factor, products, cells, 0)) == lu
+    assert bool(lib.with_block_host(factor, products, cells, 1)) == substitution
