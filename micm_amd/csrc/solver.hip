@@ -2028,16 +2028,20 @@ namespace
     return w;
   }
 
-  void host_to_grouped(const double* host, int64_t n_cells, int64_t n_vals, double* out)
+  // Between the host's order and the grouped one (out of line: inlined into their callers, the inner
+  // loop of a few values came out twice as slow).  host_to_grouped leaves the places past the last
+  // cell as they are.
+  __attribute__((noinline)) void host_to_grouped(const double* host, int64_t n_cells, int64_t n_vals, double* out)
   {
-    const int64_t ng = n_groups_of(n_cells);
-    std::fill(out, out + static_cast<size_t>(ng) * n_vals * kGroup, 0.0);
-    for (int64_t c = 0; c < n_cells; ++c)
-      for (int64_t v = 0; v < n_vals; ++v)
-        out[(static_cast<size_t>(c / kGroup) * n_vals + v) * kGroup + c % kGroup] = host[c * n_vals + v];
+    for (int64_t first = 0; first < n_cells; first += kGroup, out += kGroup * n_vals)
+    {
+      const int64_t cells = std::min<int64_t>(kGroup, n_cells - first);
+      for (int64_t l = 0; l < cells; ++l)
+        for (int64_t v = 0; v < n_vals; ++v)
+          out[v * kGroup + l] = *host++;
+    }
   }
 
-  // (out of line: inlined into its callers, the inner loop of a few values came out twice as slow)
   __attribute__((noinline)) void grouped_to_host(const double* in, int64_t n_cells, int64_t n_vals, double* host)
   {
     for (int64_t first = 0; first < n_cells; first += kGroup, in += kGroup * n_vals)
@@ -2061,12 +2065,13 @@ namespace
     if (n_vals == 0)
       return MICM_HIP_OK;
     const size_t count = static_cast<size_t>(s->n_groups) * n_vals * kGroup, bytes = count * sizeof(double);
-    std::vector<double> buf(count);
+    std::vector<double> buf(count);  // zeros
     host_to_grouped(host, s->n_cells, n_vals, buf.data());
     HIP_TRY(hipMemcpyAsync(dst, buf.data(), bytes, hipMemcpyHostToDevice, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     return MICM_HIP_OK;
   }
+
   int get_grouped(const micm_hip_state* s, const double* src, double* host, int64_t n_vals)
   {
     if (!s || (!host && n_vals))
