@@ -62,20 +62,20 @@ def apply(state, choice):
     return choice["form"]
 
 
-def _kernel(mech, stages, candidate):
-    """What a candidate's cooperative launch runs (DeviceState.set_cooperative_shape's shapes often
-    share one kernel); the candidate itself for a mechanism that cannot say."""
+def _kernel(mech, stages, candidate, n_cells):
+    """What a candidate's cooperative launch over n_cells cells runs (DeviceState.set_cooperative_shape's
+    shapes often share one kernel); the candidate itself for a mechanism that cannot say."""
     query = getattr(mech, "cooperative_kernel", None)
-    return candidate if query is None else query(stages, candidate[3], candidate[4])
+    return candidate if query is None else query(stages, candidate[3], candidate[4], n_cells)
 
 
-def _distinct(mech, stages, candidates):
+def _distinct(mech, stages, candidates, n_cells):
     """The candidates that launch different things, the first of each, and label -> label kept for
     the others."""
     kept, first, same = [], {}, {}
     for c in candidates:
         if c[1] == _lib.SOLVE_COOPERATIVE:
-            k = _kernel(mech, stages, c)
+            k = _kernel(mech, stages, c, n_cells)
             if k in first:
                 same[c[0]] = first[k]
                 continue
@@ -84,9 +84,9 @@ def _distinct(mech, stages, candidates):
     return kept, same
 
 
-def _has_lu_schedule(mech, stages, candidate):
+def _has_lu_schedule(mech, stages, candidate, n_cells):
     """Whether the LU blocking changes anything for a cooperative candidate."""
-    kernel = _kernel(mech, stages, candidate)
+    kernel = _kernel(mech, stages, candidate, n_cells)
     return kernel is candidate or kernel[0] in (_lib.KERNEL_LEVELS, _lib.KERNEL_COMPACT)
 
 
@@ -142,7 +142,7 @@ def autotune(mech, state, dt, params, sample=65536, first_sample=2048, pilot=256
         return dict(_cache[key])
     supported = mech.cooperative_supported(params.stages)
     cands, same = _distinct(mech, params.stages,
-                            [c for c in candidates if c[1] != _lib.SOLVE_COOPERATIVE or supported])
+                            [c for c in candidates if c[1] != _lib.SOLVE_COOPERATIVE or supported], n)
     wider_build = {same.get(c, c): same.get(w, w) for c, w in WIDER_BUILD.items()}
     y_all = state.get_variables()
     k_all = state.get_rate_constants()
@@ -207,7 +207,7 @@ def autotune(mech, state, dt, params, sample=65536, first_sample=2048, pilot=256
     # on the first sample; a blocking that is 2 % faster there is timed on the last sample too
     # and taken if it is faster there as well
     coop = sorted((c for c in cands if c[1] == _lib.SOLVE_COOPERATIVE and c[0] in times), key=lambda c: times[c[0]])
-    if coop and m1 > m0 and coop[0][0] in first_times and _has_lu_schedule(mech, params.stages, coop[0]):
+    if coop and m1 > m0 and coop[0][0] in first_times and _has_lu_schedule(mech, params.stages, coop[0], n):
         top = coop[0]
         base = first_times[top[0]]
         best_t, best_b = base, 0

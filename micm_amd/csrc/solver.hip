@@ -2694,20 +2694,33 @@ namespace
     return MICM_HIP_OK;
   }
 
-  // LDS of the one-lane-per-cell kernel where a Solve's cells take it, else 0: at most eight
-  // species, the library's choice of layout (stage < 0; the threads per cell have nothing to do
-  // in a mechanism of this size), no recording.
+  // LDS of the one-lane-per-cell kernel where a Solve's n_cells cells take it, else 0: mechanisms
+  // that fit it (tiny.hpp), the library's choice of layout (stage < 0; the threads per cell have
+  // nothing to do in a mechanism of this size), no recording.
   // README system, whole Solves with their transfers, against a workgroup per cell: 1 cell 254 ->
   // 177 us, 1,000 cells 331 -> 213, 10,000 cells 1,147 -> 200, 100,000 cells 9.9 -> 0.62 ms; against
   // the persistent form 446 -> 176 us, 753 -> 200 us (10,000), 3.4 -> 0.62 ms (100,000).
-  size_t tiny_solve_lds(const micm_hip_mechanism* m, int stages, int stage_request)
+  //
+  // One lane takes the reactions one after another, a wavefront per cell takes them side by side:
+  // below kTinyCells cells, which the chip holds at once (eight wavefronts a CU), the lane is the
+  // faster one only for few reactions.  ms, lane / wavefront: 3 species 6 reactions, 1 cell 0.21 / 0.28, 1,000 0.25 / 0.38;
+  // 20 reactions 0.51 / 0.36, 0.57 / 0.46, 3,000 0.57 / 0.81; 2 species 8 reactions, 1 cell
+  // 0.27 / 0.30, 24 reactions 0.45 / 0.29; 4 species 8 reactions 0.27 / 0.37, 18 reactions 0.46 / 0.41;
+  // 5 species (the wider build) 6 reactions 0.36 / 0.32, 12 reactions, 1,000 cells 0.52 / 0.55.
+  // Against the persistent form (`persistent`) it always is: 1 cell of these 0.8 to 2.2 ms there.
+  constexpr int64_t kTinyCells = 2304;
+  constexpr int kTinyReactions = 10, kTinyFewSpecies = 4;
+
+  size_t tiny_solve_lds(const micm_hip_mechanism* m, int64_t n_cells, int stages, int stage_request, bool persistent)
   {
-    return stage_request < 0 ? tiny_lds(m->dev, m->coop, m->tiny, stages) : 0;
+    const bool faster = persistent || n_cells >= kTinyCells ||
+                        (m->dev.n_species <= kTinyFewSpecies && m->dev.n_reactions <= kTinyReactions);
+    return stage_request < 0 && faster ? tiny_lds(m->dev, m->coop, m->tiny, stages) : 0;
   }
 
-  size_t tiny_solve_lds(const micm_hip_state* s, int stages)
+  size_t tiny_solve_lds(const micm_hip_state* s, int stages, bool persistent)
   {
-    return s->recording.records ? 0 : tiny_solve_lds(s->mech, stages, s->coop_stage);
+    return s->recording.records ? 0 : tiny_solve_lds(s->mech, s->n_cells, stages, s->coop_stage, persistent);
   }
 
   TinyArgs tiny_args(micm_hip_state* s, const DevParams& p)
@@ -2745,22 +2758,26 @@ namespace
     return MICM_HIP_OK;
   }
 
+  // (list null: every cell)
+  int launch_tiny(micm_hip_state* s, const DevParams& p, size_t lds, const int32_t* list, const int* count,
+                  const CellControl* resume, bool update_rates, hipStream_t st)
+  {
+    if (update_rates)
+      if (int rc = launch_rate_constants(s, st))
+        return rc;
+    TinyArgs a = tiny_args(s, p);
+    a.list = list;
+    a.list_count = count;
+    a.resume = resume;
+    HIP_TRY(tiny_solve(a, lds, st));
+    return MICM_HIP_OK;
+  }
+
   int launch_coop(micm_hip_state* s, const DevParams& p, const int32_t* list, const int* count, int64_t n_fixed,
                   const CellControl* resume, bool update_rates, hipStream_t st)
   {
-    if (const size_t lds = tiny_solve_lds(s, p.stages))
-    {
-      if (update_rates)
-        if (int rc = launch_rate_constants(s, st))
-          return rc;
-      TinyArgs a = tiny_args(s, p);
-      a.n_cells = list ? s->n_cells : n_fixed;
-      a.list = list;
-      a.list_count = count;
-      a.resume = resume;
-      HIP_TRY(tiny_solve(a, lds, st));
-      return MICM_HIP_OK;
-    }
+    if (const size_t lds = tiny_solve_lds(s, p.stages, false))
+      return launch_tiny(s, p, lds, list, count, resume, update_rates, st);
     const CoopPlan plan = plan_solve(s, p.stages, resume != nullptr);
     if (plan.lds == 0)
       return fail(MICM_HIP_ERR_UNSUPPORTED, "the cooperative form does not fit this mechanism in LDS");
@@ -2813,7 +2830,7 @@ namespace
     if (s->handoff_steps >= 0)
       return false;
     const int64_t factor = s->mech->coop.nnz_alu;
-    return tiny_solve_lds(s, stages) > 0 ||
+    return tiny_solve_lds(s, stages, true) > 0 ||
            (plan.tail && (factor > kPerLaneFactor || s->n_cells < kPerLaneCells) &&
             (factor > kWaveFactor || s->n_cells < kWaveCells));
   }
@@ -2894,8 +2911,9 @@ namespace
   int enqueue_solve(micm_hip_state* s, const DevParams& p, int32_t form, bool update_rates, hipStream_t st)
   {
     // one cell per lane: as the cells stand, no order
-    if (tiny_solve_lds(s, p.stages) > 0 && (form == MICM_HIP_SOLVE_COOPERATIVE || s->handoff_steps < 0))
-      return launch_coop(s, p, nullptr, nullptr, s->n_cells, nullptr, update_rates, st);
+    if (form == MICM_HIP_SOLVE_COOPERATIVE || s->handoff_steps < 0)
+      if (const size_t lds = tiny_solve_lds(s, p.stages, form == MICM_HIP_SOLVE_PERSISTENT))
+        return launch_tiny(s, p, lds, nullptr, nullptr, nullptr, update_rates, st);
     if (int rc = enqueue_solve_cells(s, p, form, update_rates, st))
       return rc;
     return enqueue_order(s, st);
@@ -3604,7 +3622,7 @@ extern "C"
     if (int rc = check_cooperative_shape(threads, stage))
       return rc;
     std::fill(out, out + 4, 0);
-    if (tiny_solve_lds(m, stages, stage) > 0)
+    if (tiny_solve_lds(m, n_cells, stages, stage, false) > 0)
     {
       out[0] = MICM_HIP_KERNEL_LANE;
       return MICM_HIP_OK;

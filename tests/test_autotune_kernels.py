@@ -14,14 +14,14 @@ LEVELS, COMPACT, BLOCK, LANE = _lib.KERNEL_LEVELS, _lib.KERNEL_COMPACT, _lib.KER
 
 def block_kernels(default_waves):
     """16 to 256 species."""
-    def kernel(stages, threads, stage):
+    def kernel(stages, threads, stage, n_cells=1):
         if stage < 0 and threads in (0, 256) or threads == 256 and stage >= 4:
             return BLOCK, 256, 0, {5: 3, 6: 2, 7: 2}.get(stage, default_waves)
         return (COMPACT if stage < 0 else LEVELS), threads, max(stage, 0) & 3, 0
     return kernel
 
 
-def lane_kernels(stages, threads, stage):
+def lane_kernels(stages, threads, stage, n_cells=1):
     """The smallest mechanisms."""
     if stage < 0:
         return LANE, 0, 0, 0

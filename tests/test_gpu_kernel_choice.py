@@ -16,7 +16,10 @@ def test_kernel_of_a_shape(n_species, default):
     print(f"kernel choice: {n_species} species", flush=True)
     if default == _lib.KERNEL_LEVELS and not mech.cooperative_supported(4):
         default = _lib.KERNEL_NONE
-    kernel, threads, _, waves = mech.cooperative_kernel(4)
+    # (the lane takes 5 species from 2,304 cells on)
+    if n_species == 5:
+        assert mech.cooperative_kernel(4, n_cells=2303)[0] == _lib.KERNEL_LEVELS
+    kernel, threads, _, waves = mech.cooperative_kernel(4, n_cells=2304)
     assert kernel == default
     assert (waves in (2, 3)) == (kernel == _lib.KERNEL_BLOCK)
     assert threads == {_lib.KERNEL_LANE: 0, _lib.KERNEL_NONE: 0, _lib.KERNEL_BLOCK: 256, _lib.KERNEL_LEVELS: 64}[kernel]
