@@ -262,16 +262,14 @@ def kernel_rooflines(mech, state, stream, n_cells, repeats=5):
     return out
 
 
-def solve_kernel(threads, stage, n_species):
+def solve_kernel(mech, n_cells, stages, threads, stage):
     """The cooperative form's kernel for a requested shape."""
-    if stage < 0 and n_species <= 8:
-        return "k_tiny"
-    if 16 <= n_species <= 256 and ((threads == 256 and (stage < 0 or stage >= 4)) or (threads == 0 and stage < 0)):
-        return "k_coop_tail"
-    return f"k_coop<{threads}>"
+    from micm_amd import _lib
+    kernel, launched = mech.cooperative_kernel(stages, threads, stage, n_cells)[:2]
+    return {_lib.KERNEL_LANE: "k_tiny", _lib.KERNEL_BLOCK: "k_coop_tail"}.get(kernel, f"k_coop<{launched}>")
 
 
-def measured_traffic(workload_name, n_cells, threads, stage, n_species):
+def measured_traffic(workload_name, n_cells, kernel, stage):
     """HBM bytes per Solve launch from a committed rocprofv3 PMC summary
     (profiles/*_hbm_traffic.md, FETCH_SIZE and WRITE_SIZE runs scaled by the same
     counters on a 1 GiB copy) when one covers this workload, cell count and
@@ -283,7 +281,7 @@ def measured_traffic(workload_name, n_cells, threads, stage, n_species):
         for block in text.split("```json")[1:]:
             rec = json.loads(block.split("```")[0])
             if (rec.get("workload"), rec.get("cells"), rec.get("kernel"), rec.get("stage")) == \
-                    (workload_name, n_cells, solve_kernel(threads, stage, n_species), stage):
+                    (workload_name, n_cells, kernel, stage):
                 return rec["traffic_bytes"], os.path.relpath(path, ROOT)
     return None, None
 
@@ -489,9 +487,10 @@ def main():
     achieved = bytes_per_step / (kernel_ms * 1e-3) / 1e9
     flops_per_step = algorithmic_flops(flops_per_invocation(desc, mech), stats)
     tflops = flops_per_step / (kernel_ms * 1e-3) / 1e12
-    traffic, traffic_source = (measured_traffic(args.workload, n_cells, coop_threads, coop_stage,
-                                                       mech.n_species) if coop_threads
-                               else (None, None))
+    traffic, traffic_source = (None, None)
+    if coop_threads:
+        kernel = solve_kernel(mech, n_cells, params.stages, coop_threads, coop_stage)
+        traffic, traffic_source = measured_traffic(args.workload, n_cells, kernel, coop_stage)
     conv = status == 2
     result = {
         "metric": {"210_560": "cell-solves/s, 210-species x 100k cells, batched Rosenbrock (FP64)",

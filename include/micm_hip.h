@@ -105,7 +105,7 @@ extern "C" {
 #define MICM_HIP_SOLVE_PERSISTENT 2 /* per-cell step size, persistent work-queue kernel; cells that
                                        reach the hand-off step count continue in the cooperative form */
 #define MICM_HIP_SOLVE_COOPERATIVE 3 /* per-cell step size, one workgroup per cell, working set in LDS
-                                        (one lane per cell for mechanisms of at most eight species) */
+                                        (one lane per cell for the smallest mechanisms) */
 /* OR-ed into the form: UpdateStateParameters with the Solve -- each cell's rate
  * constants are computed from its conditions and custom parameters (and stored in
  * the state), instead of by a separate micm_hip_update_state_parameters call.  Same
@@ -318,8 +318,9 @@ int micm_hip_state_set_handoff(micm_hip_state* state, int64_t steps);
  * cells on for such factors); 5 / 6 / 7: that kernel built for three waves per SIMD (168
  * registers) / two (256) / two, 4 leaving the choice to the occupancy; for other numbers of
  * species and threads 5, 6 and 7 are the same as 4.  With the library's choice of staging (-1),
- * mechanisms of at most eight species run one cell per lane whatever the threads (recorded
- * Solves excepted).  A tuning knob in the role of the vector length L of the reference's GPU
+ * the smallest mechanisms (up to 4 species and 10 reactions, and what fits 48 KB of LDS, some six
+ * species, from 2,304 cells on) run one cell per lane whatever the threads (recorded Solves
+ * excepted).  A tuning knob in the role of the vector length L of the reference's GPU
  * policies (cuda_solver_builder.hpp:24-38); results do not depend on it. */
 int micm_hip_state_set_cooperative_shape(micm_hip_state* state, int32_t threads, int32_t stage);
 /* Blocking of the cooperative form's LU level schedule: the shortest run of products an

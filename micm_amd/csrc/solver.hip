@@ -1460,11 +1460,11 @@ namespace
   // thread per species): the compact layout of coop_layout_compact, with k_wg holding
   // gridDim.x rate-constant rows of n_reactions doubles.
   //
-  // With 256 threads per cell the kernel is compiled for three waves per SIMD (at most
-  // 168 VGPRs, a few of them spilled), which lets a third cell onto a CU where LDS
-  // allows (TS1: 1.26x); the compact layout also has builds for two waves per SIMD (256
-  // registers) and without a bound (MINW 2, 1): where LDS allows two cells per CU anyway
-  // (210/560) the one that keeps two cells per CU with the fewest spills is taken.
+  // With 256 threads per cell the kernel is compiled for three waves per SIMD (at most 168
+  // VGPRs, a few of them spilled), which lets a third cell onto a CU.  Those threads are for
+  // fewer than 16 species, more than 256 and the staged layouts: between, they are
+  // coop_tail.hip's kernel (9 to 15 species, 2,000 and 50,000 cells: builds for three waves, two
+  // and without a bound within 2.5 % of each other).
   template<int NT>
   constexpr int coop_min_waves_per_eu()
   {
@@ -1473,15 +1473,13 @@ namespace
 
   // RECORD: a recorded Solve, appending each cell's checkpoints to `tape` (a separate
   // build, so that the ordinary Solve's register allocation does not carry it)
-  template<int NT, int STAGE, bool COMPACT = false, int MINW = coop_min_waves_per_eu<NT>(), bool RECORD = false>
-  __global__ void __launch_bounds__(NT, MINW) k_coop(DevMech m, DevCoop c, DevParams p, int p_capacity, int64_t n_fixed,
-                                               const int32_t* __restrict__ list, const int* list_count, int* next,
-                                               const CellControl* resume, double* __restrict__ y_state,
-                                               double* __restrict__ k_state, const double* __restrict__ atol,
-                                               int32_t* status_out, int64_t* stats_out, double* final_time_out,
-                                               const double* __restrict__ cond_state,
-                                               const double* __restrict__ custom_state, double* __restrict__ k_wg,
-                                               Tape tape)
+  template<int NT, int STAGE, bool COMPACT = false, bool RECORD = false>
+  __global__ void __launch_bounds__(NT, coop_min_waves_per_eu<NT>())
+      k_coop(DevMech m, DevCoop c, DevParams p, int p_capacity, int64_t n_fixed, const int32_t* __restrict__ list,
+             const int* list_count, int* next, const CellControl* resume, double* __restrict__ y_state,
+             double* __restrict__ k_state, const double* __restrict__ atol, int32_t* status_out, int64_t* stats_out,
+             double* final_time_out, const double* __restrict__ cond_state, const double* __restrict__ custom_state,
+             double* __restrict__ k_wg, Tape tape)
   {
     static_assert(!COMPACT || STAGE == 0, "the compact layout reads the tables from global memory");
     extern __shared__ double lds[];
@@ -2479,7 +2477,10 @@ namespace
     plan.p_capacity = 0;
     plan.compact = true;
     plan.tail = true;
-    // the register budget that fits the most cells per CU, the larger one among equals
+    // the register budget that fits the most cells per CU (60/200: three waves per SIMD, 65,536
+    // cells 129 ms, with two 180), the larger one among equals, which spills no vector registers
+    // (210/560, three / two: 256 cells 127.3 / 127.8 ms, 20,000 376.5 / 377.8, 65,536 1,250 / 1,253;
+    // between, both are 128 or 154, as two of the slowest cells share a CU or not)
     plan.min_waves = occ3 > occ2 ? 3 : 2;
     if (stage_request == 5 && occ3 > 0)
       plan.min_waves = 3;
@@ -2614,12 +2615,12 @@ namespace
     return MICM_HIP_OK;
   }
 
-  template<int NT, int STAGE, bool COMPACT, int MINW, bool RECORD>
+  template<int NT, int STAGE, bool COMPACT, bool RECORD>
   int launch_coop_build(micm_hip_state* s, const DevParams& p, const CoopPlan& plan, const int32_t* list,
                         const int* count, int64_t n_fixed, const CellControl* resume, bool update_rates, hipStream_t st)
   {
     const micm_hip_mechanism* m = s->mech;
-    const void* fn = reinterpret_cast<const void*>(k_coop<NT, STAGE, COMPACT, MINW, RECORD>);
+    const void* fn = reinterpret_cast<const void*>(k_coop<NT, STAGE, COMPACT, RECORD>);
     HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(plan.lds)));
     int64_t blocks = 0;
     if (int rc = coop_blocks(plan, blocks))
@@ -2634,7 +2635,7 @@ namespace
     if (!list)
       blocks = std::max<int64_t>(1, std::min(blocks, n_fixed));
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, next);
-    hipLaunchKernelGGL((k_coop<NT, STAGE, COMPACT, MINW, RECORD>), dim3(static_cast<unsigned>(blocks)), dim3(NT),
+    hipLaunchKernelGGL((k_coop<NT, STAGE, COMPACT, RECORD>), dim3(static_cast<unsigned>(blocks)), dim3(NT),
                        plan.lds, st, m->dev, coop_with_blocking(m, s->lu_blocking, NT), p, plan.p_capacity, n_fixed, list,
                        count,
                        next, resume, s->y, s->k, s->atol,
@@ -2644,15 +2645,13 @@ namespace
     return MICM_HIP_OK;
   }
 
-  template<int NT, int STAGE, bool COMPACT = false, int MINW = coop_min_waves_per_eu<NT>()>
+  template<int NT, int STAGE, bool COMPACT = false>
   int launch_coop_shape(micm_hip_state* s, const DevParams& p, const CoopPlan& plan, const int32_t* list,
                         const int* count, int64_t n_fixed, const CellControl* resume, bool update_rates, hipStream_t st)
   {
     if (s->recording.records)
-      return launch_coop_build<NT, STAGE, COMPACT, MINW, true>(s, p, plan, list, count, n_fixed, resume, update_rates,
-                                                             st);
-    return launch_coop_build<NT, STAGE, COMPACT, MINW, false>(s, p, plan, list, count, n_fixed, resume, update_rates,
-                                                            st);
+      return launch_coop_build<NT, STAGE, COMPACT, true>(s, p, plan, list, count, n_fixed, resume, update_rates, st);
+    return launch_coop_build<NT, STAGE, COMPACT, false>(s, p, plan, list, count, n_fixed, resume, update_rates, st);
   }
 
   template<int NT>
@@ -3674,7 +3673,7 @@ extern "C"
       }
       const bool lockstep = form == MICM_HIP_SOLVE_LOCKSTEP;
       p.error_group = s->lockstep_group;
-      // a wavefront of cells of a mechanism of at most eight species: one lane per cell
+      // a wavefront of cells of a mechanism that fits: one lane per cell
       // (README system through the facade: 1 cell 495 -> 242 us, 64 cells 493 -> 292; the loop in
       // one workgroup takes its values and tables from global memory)
       if (lockstep && s->n_cells <= kGroup)

@@ -1,4 +1,4 @@
-// tiny.hip -- Solves of mechanisms of at most eight species, one cell per lane.
+// tiny.hip -- Solves of the smallest mechanisms (tiny.hpp), one cell per lane.
 #include "tiny.hpp"
 
 #include "path.hpp"

@@ -1,4 +1,7 @@
-// tiny.hpp -- Solves of mechanisms of at most eight species, one cell per lane (tiny.hip).
+// tiny.hpp -- Solves of the smallest mechanisms, one cell per lane (tiny.hip): those whose columns
+// of 64 cells fit kTinyLds.  With four stages that is 4 species and 54 columns for the rate
+// constants and for the rates or Jacobian terms (less the lists), 5 species and 39, 6 and 22; none
+// of 7 species with more than a reaction or two, none of 8.
 #pragma once
 
 #include "device.hpp"
@@ -33,8 +36,8 @@ namespace micm_hip
     double* final_time;
   };
 
-  // Dynamic LDS of one wavefront of 64 cells; 0 where the mechanism has no tables or needs more
-  // than kTinyLds.
+  // Dynamic LDS of one wavefront of 64 cells; 0 where the mechanism has no tables (more than
+  // kTinySpecies species) or needs more than kTinyLds.
   constexpr size_t kTinyLds = 48 * 1024;
   size_t tiny_lds(const DevMech& m, const DevCoop& c, const DevTiny& t, int stages);
 
