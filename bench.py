@@ -263,13 +263,15 @@ def kernel_rooflines(mech, state, stream, n_cells, repeats=5):
 
 
 def solve_kernel(mech, n_cells, stages, threads, stage):
-    """The cooperative form's kernel for a requested shape."""
+    """The cooperative form's kernel for a requested shape, and its build where it has several."""
     from micm_amd import _lib
-    kernel, launched = mech.cooperative_kernel(stages, threads, stage, n_cells)[:2]
-    return {_lib.KERNEL_LANE: "k_tiny", _lib.KERNEL_BLOCK: "k_coop_tail"}.get(kernel, f"k_coop<{launched}>")
+    kernel, launched, _, waves = mech.cooperative_kernel(stages, threads, stage, n_cells)
+    if kernel == _lib.KERNEL_BLOCK:
+        return "k_coop_tail", f"k_coop_tail<{waves}, false>"
+    return ("k_tiny" if kernel == _lib.KERNEL_LANE else f"k_coop<{launched}>"), None
 
 
-def measured_traffic(workload_name, n_cells, kernel, stage):
+def measured_traffic(workload_name, n_cells, kernel, build, stage):
     """HBM bytes per Solve launch from a committed rocprofv3 PMC summary
     (profiles/*_hbm_traffic.md, FETCH_SIZE and WRITE_SIZE runs scaled by the same
     counters on a 1 GiB copy) when one covers this workload, cell count and
@@ -280,8 +282,8 @@ def measured_traffic(workload_name, n_cells, kernel, stage):
         text = open(path).read()
         for block in text.split("```json")[1:]:
             rec = json.loads(block.split("```")[0])
-            if (rec.get("workload"), rec.get("cells"), rec.get("kernel"), rec.get("stage")) == \
-                    (workload_name, n_cells, kernel, stage):
+            same = rec.get("launch") == build if build else rec.get("stage") == stage
+            if same and (rec.get("workload"), rec.get("cells"), rec.get("kernel")) == (workload_name, n_cells, kernel):
                 return rec["traffic_bytes"], os.path.relpath(path, ROOT)
     return None, None
 
@@ -489,8 +491,8 @@ def main():
     tflops = flops_per_step / (kernel_ms * 1e-3) / 1e12
     traffic, traffic_source = (None, None)
     if coop_threads:
-        kernel = solve_kernel(mech, n_cells, params.stages, coop_threads, coop_stage)
-        traffic, traffic_source = measured_traffic(args.workload, n_cells, kernel, coop_stage)
+        kernel, build = solve_kernel(mech, n_cells, params.stages, coop_threads, coop_stage)
+        traffic, traffic_source = measured_traffic(args.workload, n_cells, kernel, build, coop_stage)
     conv = status == 2
     result = {
         "metric": {"210_560": "cell-solves/s, 210-species x 100k cells, batched Rosenbrock (FP64)",

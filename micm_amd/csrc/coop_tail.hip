@@ -288,7 +288,7 @@ namespace
 
   // LuDecompositionDoolittle::Decompose for one cell (lu_decomposition_doolittle.inl:325-403).
   // Bound as the Solve's factorisation is by its chain, not by the 87 KB a 210/560 cell reads
-  // and writes: 4,096 cells in 545 us, 1,665 with the level schedule alone.
+  // and writes: 4,096 cells in 525 us, 1,654 with the level schedule alone.
   __global__ void __launch_bounds__(kTailThreads, 2)
       k_lu_decompose_tail(DevMech m, DevTail t, int64_t n_cells, const double* __restrict__ jac,
                           double* __restrict__ lower, double* __restrict__ upper)
@@ -322,7 +322,7 @@ namespace
   }
 
   // LinearSolver::Solve for one cell (linear_solver.inl:235-294), dividing by L[i][i] as the
-  // reference does where it is not 1.  210/560, 4,096 cells: 341 us, 1,303 with the level
+  // reference does where it is not 1.  210/560, 4,096 cells: 344 us, 1,307 with the level
   // schedules alone.
   __global__ void __launch_bounds__(kTailThreads, 2)
       k_lu_solve_tail(DevMech m, DevTail t, int64_t n_cells, const double* __restrict__ lower,

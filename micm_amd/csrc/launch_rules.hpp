@@ -34,7 +34,7 @@ namespace micm_hip
   //   120 (1,417, 4,291), 1,500 54 : 47 / 41 : 49, 8,000 192 : 158 / 167 : 174
   //   200 (1,697, 3,653), 1,500 56 : 46 / 48 : 60, 2,500 77 : 97 / 71 : 120
   //   60/200 (1,304, 7,668), 1,500 45 : 54 / 36 : 69, 20,000 382 : 439 / 347 : 456
-  //   TS1 (2,381, 6,986), 4,096 122 : 163 / 105 : 222; 210/560 (8,548, 121,036), 4,096 545 : 1,665 / 341 : 1,303
+  //   TS1 (2,381, 6,986), 4,096 122 : 163 / 105 : 222; 210/560 (8,548, 121,036), 4,096 525 : 1,654 / 344 : 1,307
   constexpr int64_t kTailCells = 768, kTailFactor = 1200, kTailProducts = 6000;
 
   constexpr bool lu_with_block(int64_t factor, int64_t products, int64_t n_cells)
