@@ -1,6 +1,7 @@
-"""Single phases on numbers of cells whose threads no longer fit one launch (2^32 threads; the
-per-cell norm takes sixteen threads a cell, alpha - J one per species).  Outputs against the same
-operations in PyTorch, bit for bit, over every cell."""
+"""Single phases on more cells than one launch has threads for when a cell takes as many as the
+kernels for few cells give it (the per-cell norm sixteen, alpha - J one per species; a launch of
+2^32 threads and more runs their number modulo 2^32).  Outputs against the same operations in
+PyTorch, bit for bit, over every cell."""
 import numpy as np
 import pytest
 
